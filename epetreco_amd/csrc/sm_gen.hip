@@ -167,6 +167,9 @@ __device__ __forceinline__ bool slab_rect(const Geo& g, const RowRays& R, int r,
   return iy0 <= iy1 && iz0 <= iz1;
 }
 
+// row_cnt of a row that k_sm_walk left to a launch with more cells, or to k_sm_rows
+constexpr int WALK_LEFT = INT_MIN, WALK_GENERAL = INT_MIN + 1;
+
 struct RowShared {
   RowRays rays;
   int wy0[MAX_SLABS], wy1[MAX_SLABS], wz0[MAX_SLABS], wz1[MAX_SLABS];
@@ -190,17 +193,19 @@ struct RowShared {
 // Candidate mode (keep_zeros = 1): full scan, every candidate kept.
 __global__ __launch_bounds__(GEN_BLOCK) void k_sm_rows(Geo g, const int* __restrict__ list,
                                                       int row0, int rowcap, int keep_zeros,
+                                                      const int* __restrict__ left,
                                                       int* __restrict__ scol,
                                                       float* __restrict__ sval,
                                                       int* __restrict__ row_cnt) {
   __shared__ RowShared S;
   const int tid = threadIdx.x;
-  const int row = row0 + blockIdx.x;
+  const int at = left ? left[blockIdx.x] : blockIdx.x;   // row of this launch's rows
+  const int row = row0 + at;
   const int cnl = list ? list[row] : row;
   const int nrays = g.nrays;
   const ChannelIds ci = channel_ids(g, cnl);
-  int* ocol = scol + (size_t)blockIdx.x * rowcap;
-  float* oval = sval + (size_t)blockIdx.x * rowcap;
+  int* ocol = scol + (size_t)at * rowcap;
+  float* oval = sval + (size_t)at * rowcap;
 
   if (tid == 0) S.flag = 0;
   __syncthreads();
@@ -300,7 +305,7 @@ __global__ __launch_bounds__(GEN_BLOCK) void k_sm_rows(Geo g, const int* __restr
       }
       nmarked = pos;
       if (nmarked > rowcap) {
-        if (tid == 0) row_cnt[blockIdx.x] = -nmarked;
+        if (tid == 0) row_cnt[at] = -nmarked;
         return;   // uniform
       }
       __syncthreads();   // marked list visible to the whole workgroup
@@ -343,11 +348,332 @@ __global__ __launch_bounds__(GEN_BLOCK) void k_sm_rows(Geo g, const int* __restr
     }
     overflow = kept > rowcap;
     if (overflow) {
-      if (tid == 0) row_cnt[blockIdx.x] = -kept;
+      if (tid == 0) row_cnt[at] = -kept;
       return;
     }
   }
-  if (tid == 0) row_cnt[blockIdx.x] = kept;
+  if (tid == 0) row_cnt[at] = kept;
+}
+
+// ------------------------------------------------------------------ walked rows
+// The same rows as k_sm_rows, ray by ray instead of voxel by voxel.  A voxel's
+// value is the sum of its rays' lengths in ray order, and a ray meets about one
+// voxel in 30 of the row's, so a workgroup of NW wavefronts keeps the row's
+// sums in LDS (cells: the y/z bounding windows of all rays, x-plane by x-plane,
+// so that cell order is voxel order) and walks the rays one after the other,
+// one lane per plane of the axis the rays run along (x or z): the lane adds the
+// ray's exact length to the few voxels of its plane that the ray's rectangle
+// (MARK_EPS wider) holds.  Planes are disjoint, so no two lanes add to one
+// voxel, and a wavefront's LDS operations keep their order, so every sum is the
+// reference's.  A plane parameter (box face - start) / direction depends only
+// on (ray, axis, plane): one table per ray in LDS replaces six correctly
+// rounded divisions per (voxel, ray).  Adding a ray that does not cross a voxel
+// adds exactly 0, so leaving it out keeps the sum.
+//
+// Bound by the chain of LDS reads and VALU work of one ray after the other.
+// Channels of 916 entries (52^3, 64 rays): 40,000 took 7.86 ms in k_sm_rows and
+// take 2.12 ms here, 100,000 18.6 and 5.2 ms; 11,250 of 57 entries (16^3, 8 rays)
+// 275 and 59 us.
+//
+// A ray parallel to an axis meets every voxel of that axis (the reference
+// ignores the axis then), so its windows span it.  Rows it does not take are
+// marked in row_cnt: windows of more than `ncells` cells WALK_LEFT, for a launch
+// with more, and a ray with no component along the walk's axis WALK_GENERAL, for
+// k_sm_rows.
+struct WalkWin {      // window of an x-plane
+  int base;           // cell of (iy, iz) = base + iy * wz + iz
+  int wz;             // cells per y line (0: no cells)
+  int y, z;           // low | high << 16, inclusive
+};
+
+template <int NW>
+__global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restrict__ list,
+                                                      int row0, int rowcap, int keep_zeros,
+                                                      int ncells, const int* __restrict__ left,
+                                                      int* __restrict__ scol,
+                                                      float* __restrict__ sval,
+                                                      int* __restrict__ row_cnt) {
+  constexpr int BLOCK = NW * WAVE;
+  extern __shared__ float4 walk_lds[];
+  __shared__ int s_wave[NW];
+  __shared__ int s_flag;
+  const int nx = g.gn[0], ny = g.gn[1], nz = g.gn[2], nrays = g.nrays;
+  const int no = max(nx, nz) + 1;
+  float4* rp = walk_lds;                                  // nrays: start, length
+  float4* rd = rp + nrays;                                // nrays: direction
+  WalkWin* win = reinterpret_cast<WalkWin*>(rd + nrays);  // nx
+  int* off = reinterpret_cast<int*>(win + nx);            // nx + 1: first cell of a plane
+  float* tab = reinterpret_cast<float*>(off + nx + 1);    // per wavefront: y faces, then x or z faces
+  float* cell = tab + NW * (ny + 1 + no);                 // ncells
+  const int tid = threadIdx.x, lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int at = left ? left[blockIdx.x] : blockIdx.x;   // row of this launch's rows
+  const int row = row0 + at;
+  const int cnl = list ? list[row] : row;
+  const ChannelIds ci = channel_ids(g, cnl);
+  int* ocol = scol + (size_t)at * rowcap;
+  float* oval = sval + (size_t)at * rowcap;
+
+  if (tid == 0) s_flag = 0;
+  __syncthreads();
+  for (int r = tid; r < nrays; r += BLOCK) {
+    float ray[6];
+    make_ray(g, ci, cnl, r, ray);
+    const float d0 = ray[3] - ray[0], d1 = ray[4] - ray[1], d2 = ray[5] - ray[2];
+    rp[r] = make_float4(ray[0], ray[1], ray[2], absolute3(d0, d1, d2));
+    rd[r] = make_float4(d0, d1, d2, d0 == 0.0f ? 0.0f : 1.0f / d0);
+  }
+  __syncthreads();
+  // the axis the rays run along, by the first ray (any choice gives the same sums)
+  const bool along_x = fabsf(rd[0].x) >= fabsf(rd[0].z);
+  for (int r = tid; r < nrays; r += BLOCK)
+    if ((along_x ? rd[r].x : rd[r].z) == 0.0f) atomicOr(&s_flag, 1);
+  __syncthreads();
+  if (s_flag) {   // uniform
+    if (tid == 0) row_cnt[at] = WALK_GENERAL;
+    return;
+  }
+
+  // windows: bounding boxes of the rays' rectangles in every x-plane
+  int ncell = 0;
+  const float iy_d = 1.0f / g.gd[1], iz_d = 1.0f / g.gd[2];
+  for (int base = 0; base < nx; base += BLOCK) {
+    const int i = base + tid;
+    float y0 = 1e30f, y1 = -1e30f, z0 = 1e30f, z1 = -1e30f;
+    const float xlo = g.go[0] + (float)i * g.gd[0], xhi = g.go[0] + (float)(i + 1) * g.gd[0];
+    for (int r = 0; r < nrays; r++) {
+      const float4 p = rp[r], d = rd[r];
+      float ta = (xlo - p.x) * d.w, tb = (xhi - p.x) * d.w;
+      if (d.x == 0.0f) {   // every x-plane: the ray's way through the grid's z range
+        ta = (g.go[2] - p.z) / d.z;
+        tb = (g.go[2] + (float)nz * g.gd[2] - p.z) / d.z;
+      }
+      const float ya = (p.y + ta * d.y - g.go[1]) * iy_d, yb = (p.y + tb * d.y - g.go[1]) * iy_d;
+      const float za = (p.z + ta * d.z - g.go[2]) * iz_d, zb = (p.z + tb * d.z - g.go[2]) * iz_d;
+      float fy0 = fminf(ya, yb) - MARK_EPS, fy1 = fmaxf(ya, yb) + MARK_EPS;
+      float fz0 = fminf(za, zb) - MARK_EPS, fz1 = fmaxf(za, zb) + MARK_EPS;
+      if (d.y == 0.0f) { fy0 = 0.0f; fy1 = (float)ny; }
+      if (d.z == 0.0f) { fz0 = 0.0f; fz1 = (float)nz; }
+      if (fy1 >= 0.0f && fz1 >= 0.0f && fy0 < (float)ny && fz0 < (float)nz) {
+        y0 = fminf(y0, fy0); y1 = fmaxf(y1, fy1);
+        z0 = fminf(z0, fz0); z1 = fmaxf(z1, fz1);
+      }
+    }
+    const bool hit = i < nx && y0 <= y1;
+    const int wy0 = (int)floorf(fmaxf(y0, 0.0f)), wy1 = (int)floorf(fminf(y1, (float)(ny - 1)));
+    const int wz0 = (int)floorf(fmaxf(z0, 0.0f)), wz1 = (int)floorf(fminf(z1, (float)(nz - 1)));
+    const int area = hit ? (wy1 - wy0 + 1) * (wz1 - wz0 + 1) : 0;
+    int tot;
+    const int ex = ncell + block_excl_sum<BLOCK>(area, s_wave, &tot);
+    if (i < nx) {
+      const int wz = hit ? wz1 - wz0 + 1 : 0;
+      win[i] = hit ? WalkWin{ex - wy0 * wz - wz0, wz, wy0 | wy1 << 16, wz0 | wz1 << 16}
+                   : WalkWin{0, 0, 1, 1};   // low 1 > high 0: holds nothing
+      off[i] = ex;
+    }
+    ncell += tot;
+  }
+  if (tid == 0) off[nx] = ncell;
+  if (ncell > ncells) {   // uniform
+    if (tid == 0) row_cnt[at] = WALK_LEFT;
+    return;
+  }
+  for (int k = tid; k < ncell; k += BLOCK) cell[k] = 0.0f;
+  __syncthreads();
+
+  const int nd = along_x ? nx : nz, nother = along_x ? nz : nx;
+  const float god = along_x ? g.go[0] : g.go[2], gdd = along_x ? g.gd[0] : g.gd[2];
+  const float goo = along_x ? g.go[2] : g.go[0], gdo = along_x ? g.gd[2] : g.gd[0];
+  const float io_d = 1.0f / gdo;
+  float* taby = tab + w * (ny + 1 + no);
+  float* tabo = taby + ny + 1;
+  const int i = w * WAVE + lane;      // this lane's plane
+  const bool own = i < nd;
+  const WalkWin wx = win[along_x && own ? i : 0];
+  if (w * WAVE < nd) {
+    for (int r = 0; r < nrays; r++) {
+      const float4 p = rp[r], d = rd[r];
+      const float pd = along_x ? p.x : p.z, dd = along_x ? d.x : d.z;
+      const float po = along_x ? p.z : p.x, d_o = along_x ? d.z : d.x;
+      for (int k = lane; k <= ny; k += WAVE) taby[k] = ((g.go[1] + (float)k * g.gd[1]) - p.y) / d.y;
+      for (int k = lane; k <= nother; k += WAVE) tabo[k] = ((goo + (float)k * gdo) - po) / d_o;
+      __builtin_amdgcn_wave_barrier();
+      const float a = ((god + (float)i * gdd) - pd) / dd;
+      const float b = ((god + (float)(i + 1) * gdd) - pd) / dd;
+      const float lo = fminf(a, b), hi = fmaxf(a, b);
+      const float ya = (p.y + lo * d.y - g.go[1]) * iy_d, yb = (p.y + hi * d.y - g.go[1]) * iy_d;
+      const float oa = (po + lo * d_o - goo) * io_d, ob = (po + hi * d_o - goo) * io_d;
+      float fy0 = fminf(ya, yb) - MARK_EPS, fy1 = fmaxf(ya, yb) + MARK_EPS;
+      float fo0 = fminf(oa, ob) - MARK_EPS, fo1 = fmaxf(oa, ob) + MARK_EPS;
+      const bool all_y = d.y == 0.0f, all_o = d_o == 0.0f;   // uniform
+      if (all_y) { fy0 = 0.0f; fy1 = (float)ny; }
+      if (all_o) { fo0 = 0.0f; fo1 = (float)nother; }
+      if (own && fy1 >= 0.0f && fo1 >= 0.0f && fy0 < (float)ny && fo0 < (float)nother) {
+        const int y0 = (int)floorf(fmaxf(fy0, 0.0f)), y1 = min(ny - 1, (int)floorf(fy1));
+        const int o0 = (int)floorf(fmaxf(fo0, 0.0f)), o1 = min(nother - 1, (int)floorf(fo1));
+        for (int iy = y0; iy <= y1; iy++) {
+          const float t0 = taby[iy], t1 = taby[iy + 1];
+          const float lo1 = all_y ? lo : fmaxf(lo, fminf(t0, t1));
+          const float hi1 = all_y ? hi : fminf(hi, fmaxf(t0, t1));
+          if (!(lo1 < hi1)) continue;
+          for (int io = o0; io <= o1; io++) {
+            const float u0 = tabo[io], u1 = tabo[io + 1];
+            const float lo2 = all_o ? lo1 : fmaxf(lo1, fminf(u0, u1));
+            const float hi2 = all_o ? hi1 : fminf(hi1, fmaxf(u0, u1));
+            if (!(lo2 < hi2)) continue;
+            const WalkWin v = along_x ? wx : win[io];
+            const int iz = along_x ? io : i;
+            // inside the window (outside it the length is 0)
+            if (iy < (v.y & 0xFFFF) || iy > v.y >> 16 || iz < (v.z & 0xFFFF) || iz > v.z >> 16)
+              continue;
+            cell[v.base + iy * v.wz + iz] += (hi2 - lo2) * p.w;
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  __syncthreads();
+
+  float p0[3], p1[3];
+  pixel_centres(g, ci, p0, p1);
+  int kept = 0;
+  if (!keep_zeros) {
+    // the cells with a value, then their voxels, the candidate test and the mean
+    for (int base = 0; base < ncell; base += BLOCK) {
+      const int k = base + tid;
+      const float a = k < ncell ? cell[k] : 0.0f;
+      int tot;
+      const int r = block_rank<BLOCK>(a != 0.0f, s_wave, &tot);
+      if (a != 0.0f && kept + r < rowcap) { ocol[kept + r] = k; oval[kept + r] = a; }
+      kept += tot;
+    }
+    if (kept > rowcap) {
+      if (tid == 0) row_cnt[at] = -kept;
+      return;   // uniform
+    }
+    const int nval = kept;
+    kept = 0;
+    __syncthreads();   // the list is visible to the whole workgroup
+    for (int base = 0; base < nval; base += BLOCK) {
+      const int k = base + tid;
+      int v = -1;
+      float a = 0.0f;
+      if (k < nval) {
+        const int c = ocol[k];
+        a = oval[k] / (float)nrays;
+        int lo = 0, hi = nx - 1;   // plane of cell c: last x with off[x] <= c
+        while (lo < hi) {
+          const int mid = (lo + hi + 1) >> 1;
+          if (off[mid] <= c) lo = mid; else hi = mid - 1;
+        }
+        const WalkWin q = win[lo];
+        const int rel = c - off[lo];
+        v = (lo * ny + (q.y & 0xFFFF) + rel / q.wz) * nz + (q.z & 0xFFFF) + rel % q.wz;
+      }
+      __syncthreads();   // every read of this part of the list precedes the writes
+      const bool keep = v >= 0 && a != 0.0f && is_candidate(g, p0, p1, v);
+      int tot;
+      const int r = block_rank<BLOCK>(keep, s_wave, &tot);
+      if (keep) { ocol[kept + r] = v; oval[kept + r] = a; }
+      kept += tot;
+    }
+  } else {
+    // every candidate: plane by plane over the box that holds the voxel centres
+    // within the candidate radius of the centre line (its section with the
+    // plane is an ellipse of half-axes R sqrt(1 + (u_y / u_x)^2) and z alike)
+    const float ab0 = p1[0] - p0[0], ab1 = p1[1] - p0[1], ab2 = p1[2] - p0[2];
+    const float inv = 1.0f / ab0, R = g.sumRadii * 1.001f;
+    const bool steep = !(fabsf(ab0) * 64.0f > absolute3(ab0, ab1, ab2));
+    const float hy = R * sqrtf(1.0f + ab1 * inv * ab1 * inv), hz = R * sqrtf(1.0f + ab2 * inv * ab2 * inv);
+    for (int ix = 0; ix < nx; ix++) {
+      int y0 = 0, y1 = ny - 1, z0 = 0, z1 = nz - 1;
+      if (!steep) {
+        const float t = (g.go[0] + ((float)ix + 0.5f) * g.gd[0] - p0[0]) * inv;
+        const float yc = p0[1] + t * ab1 - g.go[1], zc = p0[2] + t * ab2 - g.go[2];
+        y0 = (int)fmaxf(0.0f, floorf((yc - hy) * iy_d - 0.52f));
+        y1 = (int)fminf((float)(ny - 1), ceilf((yc + hy) * iy_d - 0.48f));
+        z0 = (int)fmaxf(0.0f, floorf((zc - hz) * iz_d - 0.52f));
+        z1 = (int)fminf((float)(nz - 1), ceilf((zc + hz) * iz_d - 0.48f));
+      }
+      const int bz = z1 - z0 + 1;
+      const int box = y1 >= y0 && bz > 0 ? (y1 - y0 + 1) * bz : 0;
+      const WalkWin q = win[ix];
+      for (int base = 0; base < box; base += BLOCK) {
+        const int k = base + tid;
+        const int iy = y0 + k / bz, iz = z0 + k % bz;
+        const int v = (ix * ny + iy) * nz + iz;
+        const bool keep = k < box && is_candidate(g, p0, p1, v);
+        int tot;
+        const int r = block_rank<BLOCK>(keep, s_wave, &tot);
+        if (keep && kept + r < rowcap) {
+          const bool in = iy >= (q.y & 0xFFFF) && iy <= q.y >> 16 && iz >= (q.z & 0xFFFF) &&
+                          iz <= q.z >> 16;
+          ocol[kept + r] = v;
+          oval[kept + r] = (in ? cell[q.base + iy * q.wz + iz] : 0.0f) / (float)nrays;
+        }
+        kept += tot;
+      }
+    }
+    if (kept > rowcap) {
+      if (tid == 0) row_cnt[at] = -kept;
+      return;
+    }
+  }
+  if (tid == 0) row_cnt[at] = kept;
+}
+
+// LDS of k_sm_walk for `cells` cells
+static size_t walk_lds_bytes(const Geo& g, int nw, int cells) {
+  const size_t no = (size_t)std::max(g.gn[0], g.gn[2]) + 1;
+  return 32 * (size_t)g.nrays + sizeof(WalkWin) * g.gn[0] + sizeof(int) * (g.gn[0] + 1) +
+         sizeof(float) * (nw * ((size_t)g.gn[1] + 1 + no) + cells);
+}
+
+// Wavefronts per channel, one lane per plane of the longer of x and z; 0 where
+// the grid is beyond the walk.
+static int walk_waves(const Geo& g) {
+  const int nd = std::max(g.gn[0], g.gn[2]);
+  if (nd > 256 || g.gn[1] > 32767) return 0;
+  return nd <= 64 ? 1 : nd <= 128 ? 2 : 4;
+}
+
+// Cells of the window sets.  A launch's LDS is what limits the wavefronts in
+// flight (at 52^3, 64 rays: 1,212 cells on average, 2,174 at the 99th
+// percentile; at 104^3, 32 rays: 6,461 and 10,976), so rows go through the
+// smallest set that usually holds them, and the few beyond it through the next.
+constexpr int WALK_SETS = 4;
+constexpr size_t WALK_LDS = 158 * 1024;   // dynamic LDS, of 160 KB
+static const int walk_cells[WALK_SETS] = {512, 2304, 8704, 32768};
+
+static int walk_first_set(const Geo& g) {
+  // mean window: 0.7 of a segment wide plus the voxels its edges cut
+  const double wy = 0.7 * g.segy / g.gd[1] + 1.5, wz = 0.7 * g.segz / g.gd[2] + 2.0;
+  const double cells = 1.3 * std::max(g.gn[0], g.gn[2]) * wy * wz;
+  for (int i = 0; i < WALK_SETS; i++)
+    if (cells <= walk_cells[i]) return i;
+  return WALK_SETS;
+}
+
+static int launch_walk(hipStream_t st, const Geo& g, int nw, int cells, int rows, const int* list,
+                       int row0, int rowcap, int keep_zeros, const int* left, int* scol, float* sval,
+                       int* cnt) {
+  const size_t lds = walk_lds_bytes(g, nw, cells);
+#define EPET_WALK(N)                                                                             \
+  do {                                                                                           \
+    if (lds > 64 * 1024)                                                                         \
+      (void)hipFuncSetAttribute((const void*)k_sm_walk<N>,                                       \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);           \
+    k_sm_walk<N><<<(unsigned)rows, N * WAVE, lds, st>>>(g, list, row0, rowcap, keep_zeros, cells, \
+                                                        left, scol, sval, cnt);                  \
+  } while (0)
+  if (nw == 1) EPET_WALK(1);
+  else if (nw == 2) EPET_WALK(2);
+  else EPET_WALK(4);
+#undef EPET_WALK
+  return hipGetLastError() == hipSuccess
+             ? EPET_OK
+             : fail(EPET_ERR_HIP, __FILE__, __LINE__, "k_sm_walk launch");
 }
 
 // Copy each row's entries from the per-row scratch into the packed arrays.
@@ -417,6 +743,8 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
   const size_t budget = (size_t)4 << 30;   // per-row scratch budget
   int* cnt = nullptr;
   int64_t* off = nullptr;
+  int* left_d = nullptr;
+  const int nw = walk_waves(g);
   int r0 = 0;
   int maxrows = 0;
   int rc = EPET_OK;
@@ -427,9 +755,12 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
     if (rows > maxrows) {
       if (cnt) (void)hipFreeAsync(cnt, ctx->stream);
       if (off) (void)hipFreeAsync(off, ctx->stream);
+      if (left_d) (void)hipFreeAsync(left_d, ctx->stream);
       cnt = nullptr;
       off = nullptr;
+      left_d = nullptr;
       if (hipMallocAsync((void**)&cnt, sizeof(int) * rows, ctx->stream) != hipSuccess ||
+          hipMallocAsync((void**)&left_d, sizeof(int) * rows, ctx->stream) != hipSuccess ||
           hipMallocAsync((void**)&off, sizeof(int64_t) * (rows + 1), ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
         rc = fail(EPET_ERR_ALLOC, __FILE__, __LINE__, "row counts");
@@ -442,16 +773,53 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
     if (rc != EPET_OK) break;
     int* scol = (int*)scr;
     float* sval = (float*)((int*)scr + (size_t)rows * rowcap);
-    k_sm_rows<<<(unsigned)rows, GEN_BLOCK, 0, ctx->stream>>>(g, list, r0, (int)rowcap,
-                                                             keep_zeros, scol, sval, cnt);
-    if (hipGetLastError() != hipSuccess) { rc = fail(EPET_ERR_HIP, __FILE__, __LINE__, "k_sm_rows launch"); break; }
-    // overflow check: minimum of the counts
-    std::vector<int> hc(rows);
-    if (hipMemcpyAsync(hc.data(), cnt, sizeof(int) * rows, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess) {
-      rc = fail(EPET_ERR_HIP, __FILE__, __LINE__, "row count readback");
-      break;
+    // walked rows, window set by window set, then k_sm_rows: each launch on the
+    // rows that the one before left
+    std::vector<int> hc(rows), left, general;
+    auto counts = [&]() -> int {   // the rows' counts, and which rows have none yet
+      if (hipMemcpyAsync(hc.data(), cnt, sizeof(int) * rows, hipMemcpyDeviceToHost, ctx->stream) !=
+              hipSuccess ||
+          hipStreamSynchronize(ctx->stream) != hipSuccess)
+        return fail(EPET_ERR_HIP, __FILE__, __LINE__, "row count readback");
+      left.clear();
+      general.clear();
+      for (int i = 0; i < (int)rows; i++) {
+        if (hc[i] == WALK_LEFT) left.push_back(i);
+        if (hc[i] == WALK_GENERAL) general.push_back(i);
+      }
+      return EPET_OK;
+    };
+    auto upload = [&](const std::vector<int>& v) -> int {
+      if (!v.empty() && hipMemcpyAsync(left_d, v.data(), sizeof(int) * v.size(),
+                                       hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+        return fail(EPET_ERR_HIP, __FILE__, __LINE__, "row list upload");
+      return EPET_OK;
+    };
+    bool walked = false;
+    for (int set = nw ? walk_first_set(g) : WALK_SETS; set < WALK_SETS && rc == EPET_OK; set++) {
+      if (walk_lds_bytes(g, nw, walk_cells[set]) > WALK_LDS || (walked && left.empty())) break;
+      if (walked) rc = upload(left);
+      if (rc == EPET_OK)
+        rc = launch_walk(ctx->stream, g, nw, walk_cells[set], walked ? (int)left.size() : (int)rows,
+                         list, r0, (int)rowcap, keep_zeros, walked ? left_d : nullptr, scol, sval,
+                         cnt);
+      if (rc == EPET_OK) rc = counts();
+      walked = true;
     }
+    if (rc == EPET_OK && walked) {
+      left.insert(left.end(), general.begin(), general.end());
+      rc = upload(left);
+    }
+    if (rc == EPET_OK && !(walked && left.empty())) {
+      k_sm_rows<<<walked ? (unsigned)left.size() : (unsigned)rows, GEN_BLOCK, 0, ctx->stream>>>(
+          g, list, r0, (int)rowcap, keep_zeros, walked ? left_d : nullptr, scol, sval, cnt);
+      if (hipGetLastError() != hipSuccess)
+        rc = fail(EPET_ERR_HIP, __FILE__, __LINE__, "k_sm_rows launch");
+      else
+        rc = counts();
+    }
+    if (rc != EPET_OK) break;
+    // overflow check: minimum of the counts
     int need = 0;
     for (int v : hc) need = std::max(need, -v);
     if (need > 0) {
@@ -467,6 +835,7 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
   }
   if (cnt) (void)hipFreeAsync(cnt, ctx->stream);
   if (off) (void)hipFreeAsync(off, ctx->stream);
+  if (left_d) (void)hipFreeAsync(left_d, ctx->stream);
   return rc;
 }
 
