@@ -96,16 +96,16 @@ struct BlkCopy {
   float ms = 0.0f;
   BlkCopy* next = nullptr;     // copies for other padded frame counts
   ~BlkCopy() {
-    if (rowperm) (void)hipFree(rowperm);
-    if (colinv) (void)hipFree(colinv);
-    if (seg_base) (void)hipFree(seg_base);
-    if (nz_base) (void)hipFree(nz_base);
-    if (cnt) (void)hipFree(cnt);
-    if (ent) (void)hipFree(ent);
-    if (eval) (void)hipFree(eval);
-    if (partial) (void)hipFree(partial);
-    if (gp) (void)hipFree(gp);
-    if (work) (void)hipFree(work);
+    if (rowperm) (void)dev_free(rowperm);
+    if (colinv) (void)dev_free(colinv);
+    if (seg_base) (void)dev_free(seg_base);
+    if (nz_base) (void)dev_free(nz_base);
+    if (cnt) (void)dev_free(cnt);
+    if (ent) (void)dev_free(ent);
+    if (eval) (void)dev_free(eval);
+    if (partial) (void)dev_free(partial);
+    if (gp) (void)dev_free(gp);
+    if (work) (void)dev_free(work);
     delete next;
   }
 };
@@ -880,22 +880,22 @@ static int blk_build(epet_ctx* ctx, const epet_matrix* M, int Fp, const std::vec
   int* cnt32 = nullptr;
   int64_t* off = nullptr;
   const long long ngp = ((long long)B->T * B->C) << B->lgFp;
-  bool ok = hipMalloc((void**)&B->gp, sizeof(float) * (size_t)ngp) == hipSuccess &&
-            hipMalloc((void**)&B->rowperm, sizeof(int) * (size_t)B->m_pad) == hipSuccess &&
-            hipMalloc((void**)&B->work, sizeof(int) * 2) == hipSuccess &&
-            hipMalloc((void**)&B->colinv, sizeof(int) * ci.size()) == hipSuccess &&
-            hipMalloc((void**)&cpos_d, sizeof(int) * cpos.size()) == hipSuccess &&
-            hipMalloc((void**)&B->seg_base, sizeof(int64_t) * (size_t)B->T * (B->nG + 1)) ==
+  bool ok = dev_malloc((void**)&B->gp, sizeof(float) * (size_t)ngp) == hipSuccess &&
+            dev_malloc((void**)&B->rowperm, sizeof(int) * (size_t)B->m_pad) == hipSuccess &&
+            dev_malloc((void**)&B->work, sizeof(int) * 2) == hipSuccess &&
+            dev_malloc((void**)&B->colinv, sizeof(int) * ci.size()) == hipSuccess &&
+            dev_malloc((void**)&cpos_d, sizeof(int) * cpos.size()) == hipSuccess &&
+            dev_malloc((void**)&B->seg_base, sizeof(int64_t) * (size_t)B->T * (B->nG + 1)) ==
                 hipSuccess &&
-            hipMalloc((void**)&B->nz_base, sizeof(int64_t) * (size_t)B->T * (B->nG + 1)) ==
+            dev_malloc((void**)&B->nz_base, sizeof(int64_t) * (size_t)B->T * (B->nG + 1)) ==
                 hipSuccess &&
-            hipMalloc((void**)&B->cnt, sizeof(uint16_t) * (size_t)nseg) == hipSuccess &&
-            hipMalloc((void**)&cnt32, sizeof(int) * (size_t)nseg) == hipSuccess &&
-            hipMalloc((void**)&off, sizeof(int64_t) * (size_t)(nseg + 1)) == hipSuccess;
+            dev_malloc((void**)&B->cnt, sizeof(uint16_t) * (size_t)nseg) == hipSuccess &&
+            dev_malloc((void**)&cnt32, sizeof(int) * (size_t)nseg) == hipSuccess &&
+            dev_malloc((void**)&off, sizeof(int64_t) * (size_t)(nseg + 1)) == hipSuccess;
   auto cleanup = [&]() {
-    if (cpos_d) (void)hipFree(cpos_d);
-    if (cnt32) (void)hipFree(cnt32);
-    if (off) (void)hipFree(off);
+    if (cpos_d) (void)dev_free(cpos_d);
+    if (cnt32) (void)dev_free(cnt32);
+    if (off) (void)dev_free(off);
   };
   if (!ok) {
     (void)hipGetLastError();
@@ -949,10 +949,10 @@ static int blk_build(epet_ctx* ctx, const epet_matrix* M, int Fp, const std::vec
     const long long ngran = (long long)B->T * B->nG;
     int* gcount = nullptr;
     int64_t* nzoff = nullptr;
-    if (hipMalloc((void**)&gcount, sizeof(int) * (size_t)std::max(1ll, ngran)) != hipSuccess ||
-        hipMalloc((void**)&nzoff, sizeof(int64_t) * (size_t)(ngran + 1)) != hipSuccess) {
+    if (dev_malloc((void**)&gcount, sizeof(int) * (size_t)std::max(1ll, ngran)) != hipSuccess ||
+        dev_malloc((void**)&nzoff, sizeof(int64_t) * (size_t)(ngran + 1)) != hipSuccess) {
       (void)hipGetLastError();
-      if (gcount) (void)hipFree(gcount);
+      if (gcount) (void)dev_free(gcount);
       cleanup();
       delete B;
       return EPET_OK;
@@ -967,9 +967,9 @@ static int blk_build(epet_ctx* ctx, const epet_matrix* M, int Fp, const std::vec
       if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
         rc = fail(EPET_ERR_HIP, __FILE__, __LINE__, "blocked copy row bases");
     }
-    (void)hipFree(gcount);
-    (void)hipFree(nzoff);
-    (void)hipFree(cnt32);
+    (void)dev_free(gcount);
+    (void)dev_free(nzoff);
+    (void)dev_free(cnt32);
     cnt32 = nullptr;
     if (rc != EPET_OK) {
       cleanup();
@@ -978,9 +978,9 @@ static int blk_build(epet_ctx* ctx, const epet_matrix* M, int Fp, const std::vec
     }
     // entries, then BLK_ENT_PAD zero entries that batches reading past a run reach
     const size_t eb = M->value_type == EPET_VAL_F32 ? 2 : 4;
-    if (hipMalloc(&B->ent, eb * (size_t)(tot + BLK_ENT_PAD)) != hipSuccess ||
+    if (dev_malloc((void**)&B->ent, eb * (size_t)(tot + BLK_ENT_PAD)) != hipSuccess ||
         (M->value_type == EPET_VAL_F32 &&
-         hipMalloc((void**)&B->eval, sizeof(float) * (size_t)(tot + BLK_ENT_PAD)) != hipSuccess)) {
+         dev_malloc((void**)&B->eval, sizeof(float) * (size_t)(tot + BLK_ENT_PAD)) != hipSuccess)) {
       (void)hipGetLastError();
       cleanup();
       delete B;
@@ -1044,10 +1044,10 @@ static int blk_partial_ensure(BlkCopy* B, int splits) {
   if (splits <= 1) return EPET_OK;
   const long long need = (long long)splits * B->m_pad * B->Fp;
   if (need <= B->partial_len) return EPET_OK;
-  if (B->partial) (void)hipFree(B->partial);
+  if (B->partial) (void)dev_free(B->partial);
   B->partial = nullptr;
   B->partial_len = 0;
-  if (hipMalloc((void**)&B->partial, sizeof(float) * (size_t)need) != hipSuccess) {
+  if (dev_malloc((void**)&B->partial, sizeof(float) * (size_t)need) != hipSuccess) {
     (void)hipGetLastError();
     EPET_FAIL(EPET_ERR_ALLOC, "blocked products: partial sums");
   }

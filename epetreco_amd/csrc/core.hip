@@ -1,9 +1,12 @@
 // core.hip -- errors, contexts, geometry upload, device memory, prefix sums,
 // chunk helpers of libepet.so.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <mutex>
+#include <unordered_map>
 
 #include "epet_block.hpp"
 
@@ -30,12 +33,12 @@ int ctx_scratch(epet_ctx* ctx, size_t bytes, void** out) {
   if (bytes > ctx->scratch_bytes) {
     if (ctx->scratch) {
       EPET_HIP(hipStreamSynchronize(ctx->stream));
-      EPET_HIP(hipFree(ctx->scratch));
+      EPET_HIP(dev_free(ctx->scratch));
       ctx->scratch = nullptr;
       ctx->scratch_bytes = 0;
     }
     size_t want = bytes < (1u << 20) ? (1u << 20) : bytes;
-    if (hipMalloc(&ctx->scratch, want) != hipSuccess) {
+    if (dev_malloc(&ctx->scratch, want) != hipSuccess) {
       (void)hipGetLastError();
       EPET_FAIL(EPET_ERR_ALLOC, "scratch allocation of " + std::to_string(want) + " bytes failed");
     }
@@ -43,6 +46,179 @@ int ctx_scratch(epet_ctx* ctx, size_t bytes, void** out) {
   }
   *out = ctx->scratch;
   return EPET_OK;
+}
+
+// ------------------------------------------------------------------ blocks
+// Device blocks of matrices and plans, kept when they are freed and handed out
+// again: a reconstruction allocates and frees tens of blocks of up to hundreds
+// of MB, and at a few GB per 25 ms the driver's clearing of freed memory falls
+// behind (passes of 22 ms stalled for 50 to 130 ms now and then); a small build
+// spent 250 of 370 us in allocations.  At most DEV_KEEP bytes per device are
+// kept, for as long as a context on the device is open; they are given back
+// when the last one closes and when an allocation fails.  A block is kept only
+// once the device has finished all work (which hipFree waits for as well), so
+// any thread or stream may take it.
+constexpr size_t DEV_KEEP = (size_t)4 << 30;
+constexpr size_t TMP_KEEP = (size_t)1 << 30;   // stream-ordered temporaries
+constexpr int DEV_MAX = 64;
+
+struct DevBlocks {
+  std::mutex mu;
+  std::multimap<size_t, void*> kept;   // by size
+  size_t kept_bytes = 0;
+  int contexts = 0;
+  hipMemPool_t pool = nullptr;         // of stream-ordered temporaries
+};
+struct DevLive {
+  std::mutex mu;
+  std::unordered_map<void*, std::pair<int, size_t>> block;   // device, size
+};
+// never destroyed: matrices may be freed while the process ends
+static DevBlocks* dev_blocks() {
+  static DevBlocks* b = new DevBlocks[DEV_MAX];
+  return b;
+}
+static DevLive& dev_live() {
+  static DevLive* l = new DevLive();
+  return *l;
+}
+
+static void dev_trim(DevBlocks& d) {   // with the device current
+  std::multimap<size_t, void*> out;
+  {
+    std::lock_guard<std::mutex> lock(d.mu);
+    out.swap(d.kept);
+    d.kept_bytes = 0;
+  }
+  for (auto& b : out) (void)hipFree(b.second);
+}
+
+hipError_t dev_malloc(void** p, size_t bytes) {
+  *p = nullptr;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  bytes = (std::max<size_t>(bytes, 1) + 511) & ~(size_t)511;
+  if (dev < 0 || dev >= DEV_MAX) return hipErrorInvalidDevice;
+  DevBlocks& d = dev_blocks()[dev];
+  size_t got = bytes;
+  {
+    std::lock_guard<std::mutex> lock(d.mu);
+    // the smallest kept block that holds it and is at most an eighth larger
+    auto it = d.kept.lower_bound(bytes);
+    if (it != d.kept.end() && it->first <= bytes + bytes / 8 + 4096) {
+      *p = it->second;
+      got = it->first;
+      d.kept_bytes -= got;
+      d.kept.erase(it);
+    }
+  }
+  if (*p == nullptr) {
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      dev_trim(d);
+      e = hipMalloc(p, bytes);
+      if (e != hipSuccess) {
+        *p = nullptr;
+        return e;
+      }
+    }
+  }
+  DevLive& l = dev_live();
+  std::lock_guard<std::mutex> lock(l.mu);
+  l.block[*p] = {dev, got};
+  return hipSuccess;
+}
+
+hipError_t dev_free(void* p) {
+  if (!p) return hipSuccess;
+  int dev = -1, cur = -1;
+  size_t bytes = 0;
+  {
+    DevLive& l = dev_live();
+    std::lock_guard<std::mutex> lock(l.mu);
+    auto it = l.block.find(p);
+    if (it != l.block.end()) {
+      dev = it->second.first;
+      bytes = it->second.second;
+      l.block.erase(it);
+    }
+  }
+  if (dev < 0) return hipFree(p);
+  DevBlocks& d = dev_blocks()[dev];
+  (void)hipGetDevice(&cur);
+  if (cur != dev) (void)hipSetDevice(dev);
+  // unfinished work (or an error) leaves the block to hipFree
+  bool kept = false;
+  if (bytes <= DEV_KEEP / 4 && hipDeviceSynchronize() == hipSuccess) {
+    std::lock_guard<std::mutex> lock(d.mu);
+    if (d.contexts > 0 && d.kept_bytes + bytes <= DEV_KEEP) {
+      d.kept.emplace(bytes, p);
+      d.kept_bytes += bytes;
+      kept = true;
+    }
+  }
+  const hipError_t e = kept ? hipSuccess : hipFree(p);
+  if (cur != dev && cur >= 0) (void)hipSetDevice(cur);
+  return e;
+}
+
+// stream-ordered temporaries, from a pool that keeps up to TMP_KEEP bytes
+// between calls (the device's default pool gives them back at every
+// synchronisation)
+hipError_t tmp_malloc(void** p, size_t bytes, hipStream_t st) {
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < DEV_MAX) {
+    DevBlocks& d = dev_blocks()[dev];
+    hipMemPool_t pool;
+    {
+      std::lock_guard<std::mutex> lock(d.mu);
+      pool = d.pool;
+    }
+    if (pool) {
+      if (hipMallocFromPoolAsync(p, bytes, pool, st) == hipSuccess) return hipSuccess;
+      (void)hipGetLastError();
+      dev_trim(d);
+      return hipMallocFromPoolAsync(p, bytes, pool, st);
+    }
+  }
+  return hipMallocAsync(p, bytes, st);
+}
+
+// a context on `dev` (current) opens or closes
+static void dev_open(int dev) {
+  if (dev >= DEV_MAX) return;
+  DevBlocks& d = dev_blocks()[dev];
+  std::lock_guard<std::mutex> lock(d.mu);
+  if (d.contexts++ > 0) return;
+  hipMemPoolProps props{};
+  props.allocType = hipMemAllocationTypePinned;
+  props.handleTypes = hipMemHandleTypeNone;
+  props.location.type = hipMemLocationTypeDevice;
+  props.location.id = dev;
+  uint64_t keep = TMP_KEEP;
+  if (hipMemPoolCreate(&d.pool, &props) != hipSuccess ||
+      hipMemPoolSetAttribute(d.pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+    (void)hipGetLastError();   // temporaries then come from the default pool
+    if (d.pool) (void)hipMemPoolDestroy(d.pool);
+    d.pool = nullptr;
+  }
+}
+
+static void dev_close(int dev) {
+  if (dev >= DEV_MAX) return;
+  DevBlocks& d = dev_blocks()[dev];
+  hipMemPool_t pool = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(d.mu);
+    if (--d.contexts > 0) return;
+    pool = d.pool;
+    d.pool = nullptr;
+  }
+  (void)hipDeviceSynchronize();
+  if (pool) (void)hipMemPoolDestroy(pool);
+  dev_trim(d);
 }
 
 int ctx_geo(epet_ctx* ctx, Geo* g) {
@@ -172,7 +348,7 @@ template <typename Tin, typename Tout>
 static int scan_total(epet_ctx* ctx, const Tin* in, Tout* out, long long n, long long* total) {
   if (!total) return scan_impl<Tin, Tout>(ctx, in, out, n, nullptr);
   Tout* tdev = nullptr;
-  EPET_HIP(hipMallocAsync((void**)&tdev, sizeof(Tout), ctx->stream));
+  EPET_HIP(tmp_malloc((void**)&tdev, sizeof(Tout), ctx->stream));
   int r = scan_impl<Tin, Tout>(ctx, in, out, n, tdev);
   Tout th = 0;
   if (r == EPET_OK) r = read_pinned(ctx, &th, tdev, sizeof(Tout));
@@ -233,6 +409,7 @@ int epet_ctx_create(epet_ctx** out, int device, void* stream) {
     delete c;
     EPET_FAIL(EPET_ERR_ALLOC, "pinned host allocation failed");
   }
+  dev_open(device);
   *out = c;
   return EPET_OK;
 }
@@ -240,8 +417,13 @@ int epet_ctx_create(epet_ctx** out, int device, void* stream) {
 int epet_ctx_destroy(epet_ctx* ctx) {
   if (!ctx) return EPET_OK;
   (void)hipStreamSynchronize(ctx->stream);
-  if (ctx->scratch) (void)hipFree(ctx->scratch);
+  if (ctx->scratch) (void)dev_free(ctx->scratch);
   if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+  int cur = -1;
+  (void)hipGetDevice(&cur);
+  if (cur != ctx->device) (void)hipSetDevice(ctx->device);
+  dev_close(ctx->device);
+  if (cur != ctx->device && cur >= 0) (void)hipSetDevice(cur);
   delete ctx;
   return EPET_OK;
 }
@@ -320,7 +502,7 @@ int epet_set_seed(epet_ctx* ctx, uint64_t seed) {
 
 int epet_malloc(epet_ctx* ctx, void** ptr, size_t bytes) {
   EPET_CHECK(ctx && ptr, EPET_ERR_ARG, "null argument");
-  if (hipMalloc(ptr, bytes ? bytes : 1) != hipSuccess) {
+  if (dev_malloc(ptr, bytes) != hipSuccess) {
     (void)hipGetLastError();
     EPET_FAIL(EPET_ERR_ALLOC, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
   }
@@ -331,7 +513,7 @@ int epet_free(epet_ctx* ctx, void* ptr) {
   EPET_CHECK(ctx, EPET_ERR_ARG, "null context");
   if (ptr) {
     EPET_HIP(hipStreamSynchronize(ctx->stream));
-    EPET_HIP(hipFree(ptr));
+    EPET_HIP(dev_free(ptr));
   }
   return EPET_OK;
 }

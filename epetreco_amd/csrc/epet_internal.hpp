@@ -29,6 +29,14 @@ int fail(int code, const char* file, int line, const std::string& msg);
 #define EPET_TRY(call) \
   do { int _r = (call); if (_r != EPET_OK) return _r; } while (0)
 
+// ---------------------------------------------------------------- device blocks
+// hipMalloc / hipFree of matrix and plan arrays, with freed blocks kept for
+// the next ones (core.hip)
+hipError_t dev_malloc(void** p, size_t bytes);
+hipError_t dev_free(void* p);
+// hipMallocAsync from the library's pool (freed with hipFreeAsync)
+hipError_t tmp_malloc(void** p, size_t bytes, hipStream_t st);
+
 // ---------------------------------------------------------------- temporaries
 // Stream-ordered temporary device buffers, freed on the stream when the guard
 // leaves scope, so that every return path (error paths included) releases
@@ -45,7 +53,7 @@ class StreamTemps {
   hipError_t alloc(T** out, size_t bytes) {
     *out = nullptr;
     if (n_ == kMax) return hipErrorOutOfMemory;
-    const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(out), bytes, st_);
+    const hipError_t e = tmp_malloc(reinterpret_cast<void**>(out), bytes, st_);
     if (e == hipSuccess) p_[n_++] = *out;
     return e;
   }

@@ -361,10 +361,10 @@ static bool lds_wanted(const epet_ctx* ctx, const epet_matrix* A) {
 }
 
 static void lds_release(epet_matrix* A) {
-  if (A->lds_off) (void)hipFree(A->lds_off);
-  if (A->lds_val) (void)hipFree(A->lds_val);
-  if (A->lds_col16) (void)hipFree(A->lds_col16);
-  if (A->lds_partial) (void)hipFree(A->lds_partial);
+  if (A->lds_off) (void)dev_free(A->lds_off);
+  if (A->lds_val) (void)dev_free(A->lds_val);
+  if (A->lds_col16) (void)dev_free(A->lds_col16);
+  if (A->lds_partial) (void)dev_free(A->lds_partial);
   A->lds_off = nullptr;
   A->lds_val = nullptr;
   A->lds_col16 = nullptr;
@@ -389,10 +389,10 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
   if (mp.nx > 0) {
     // renumbered columns: rows re-sorted into y-major column order first
     const size_t vb0 = A->value_type == EPET_VAL_F32 ? 4 : 2;
-    if (hipMalloc((void**)&colp, sizeof(int) * (size_t)std::max(1ll, A->nnz)) != hipSuccess ||
-        hipMalloc(&valp, vb0 * (size_t)std::max(1ll, A->nnz)) != hipSuccess) {
+    if (dev_malloc((void**)&colp, sizeof(int) * (size_t)std::max(1ll, A->nnz)) != hipSuccess ||
+        dev_malloc((void**)&valp, vb0 * (size_t)std::max(1ll, A->nnz)) != hipSuccess) {
       (void)hipGetLastError();
-      if (colp) (void)hipFree(colp);
+      if (colp) (void)dev_free(colp);
       return EPET_OK;
     }
     const unsigned g = (unsigned)std::max<long long>(
@@ -407,8 +407,8 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
                                                   (uint16_t*)valp);
     const hipError_t le = hipGetLastError();
     if (le != hipSuccess) {
-      (void)hipFree(colp);
-      (void)hipFree(valp);
+      (void)dev_free(colp);
+      (void)dev_free(valp);
       EPET_FAIL(EPET_ERR_HIP, std::string("k_ysort_rows: ") + hipGetErrorString(le));
     }
     scol = colp;
@@ -423,9 +423,9 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
   void* val = nullptr;
   uint16_t* col16 = nullptr;
   bool ok = T >= 1 &&
-            hipMalloc((void**)&toff, sizeof(uint32_t) * (size_t)A->m * (T + 1)) == hipSuccess &&
-            hipMalloc((void**)&cnt, sizeof(int) * (size_t)std::max(1ll, nseg)) == hipSuccess &&
-            hipMalloc((void**)&off, sizeof(int64_t) * (size_t)(nseg + 1)) == hipSuccess;
+            dev_malloc((void**)&toff, sizeof(uint32_t) * (size_t)A->m * (T + 1)) == hipSuccess &&
+            dev_malloc((void**)&cnt, sizeof(int) * (size_t)std::max(1ll, nseg)) == hipSuccess &&
+            dev_malloc((void**)&off, sizeof(int64_t) * (size_t)(nseg + 1)) == hipSuccess;
   int rc = EPET_OK;
   if (ok) {
     launch_row_plan(st, A->m, T, TV, A->rowptr, scol, toff);
@@ -435,8 +435,8 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
     if (rc == EPET_OK && (tot < A->nnz || tot > A->nnz + (long long)(LDS_CHUNK - 1) * nseg))
       rc = fail(EPET_ERR_STATE, __FILE__, __LINE__, "tile-major copy: entry count mismatch");
     ok = rc == EPET_OK &&
-         hipMalloc(&val, vb * (size_t)std::max(1ll, tot)) == hipSuccess &&
-         hipMalloc((void**)&col16, sizeof(uint16_t) * (size_t)std::max(1ll, tot)) == hipSuccess;
+         dev_malloc((void**)&val, vb * (size_t)std::max(1ll, tot)) == hipSuccess &&
+         dev_malloc((void**)&col16, sizeof(uint16_t) * (size_t)std::max(1ll, tot)) == hipSuccess;
     if (rc == EPET_OK && !ok) (void)hipGetLastError();
     if (ok) {
       k_lds_set_last<<<1, 64, 0, st>>>(off, nseg, tot);
@@ -455,14 +455,14 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
   } else {
     (void)hipGetLastError();
   }
-  if (toff) (void)hipFree(toff);
-  if (cnt) (void)hipFree(cnt);
-  if (colp) (void)hipFree(colp);
-  if (valp) (void)hipFree(valp);
+  if (toff) (void)dev_free(toff);
+  if (cnt) (void)dev_free(cnt);
+  if (colp) (void)dev_free(colp);
+  if (valp) (void)dev_free(valp);
   if (!ok || rc != EPET_OK) {
-    if (off) (void)hipFree(off);
-    if (val) (void)hipFree(val);
-    if (col16) (void)hipFree(col16);
+    if (off) (void)dev_free(off);
+    if (val) (void)dev_free(val);
+    if (col16) (void)dev_free(col16);
     return rc;
   }
   *T_out = T;
@@ -498,7 +498,7 @@ int lds_prepare_map(epet_ctx* ctx, epet_matrix* A, bool voxel_columns) {
   const ColMap mp = voxel_columns ? voxel_map(ctx, A) : ColMap{};
   EPET_TRY(build_tile_major(ctx, A, LDS_TILE, mp, &T, &A->lds_off, &A->lds_val, &A->lds_col16));
   A->lds_map = mp;
-  if (A->lds_off && hipMalloc((void**)&A->lds_partial, sizeof(float) * (size_t)A->m * T) ==
+  if (A->lds_off && dev_malloc((void**)&A->lds_partial, sizeof(float) * (size_t)A->m * T) ==
                         hipSuccess) {
     A->lds_T = T;
     return EPET_OK;

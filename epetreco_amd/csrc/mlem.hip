@@ -512,11 +512,11 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
       return rc;                                                                         \
     }                                                                                    \
   } while (0)
-  EPET_MLEM_HIP(hipMallocAsync((void**)&e, sizeof(float) * std::max<long long>(1, (long long)A->m * F), st));
-  EPET_MLEM_HIP(hipMallocAsync((void**)&c, sizeof(float) * std::max<long long>(1, nv), st));
-  EPET_MLEM_HIP(hipMallocAsync((void**)&s, sizeof(float) * std::max(1, A->n), st));
-  EPET_MLEM_HIP(hipMallocAsync((void**)&ibuf, sizeof(int) * (1 + F), st));
-  EPET_MLEM_HIP(hipMallocAsync((void**)&dbuf, sizeof(double) * nd, st));
+  EPET_MLEM_HIP(tmp_malloc((void**)&e, sizeof(float) * std::max<long long>(1, (long long)A->m * F), st));
+  EPET_MLEM_HIP(tmp_malloc((void**)&c, sizeof(float) * std::max<long long>(1, nv), st));
+  EPET_MLEM_HIP(tmp_malloc((void**)&s, sizeof(float) * std::max(1, A->n), st));
+  EPET_MLEM_HIP(tmp_malloc((void**)&ibuf, sizeof(int) * (1 + F), st));
+  EPET_MLEM_HIP(tmp_malloc((void**)&dbuf, sizeof(double) * nd, st));
   int* itp = ibuf;
   int* active = ibuf + 1;
   double* ssum = dbuf;
@@ -678,11 +678,11 @@ int epet_mlem_tune(epet_ctx* ctx, epet_matrix* A, int F, int* cfg, float* ms) {
     if (c) (void)hipFreeAsync(c, st);
     if (itp) (void)hipFreeAsync(itp, st);
   };
-  if (hipMallocAsync((void**)&x, sizeof(float) * std::max(1ll, nx), st) != hipSuccess ||
-      hipMallocAsync((void**)&c, sizeof(float) * std::max(1ll, nx), st) != hipSuccess ||
-      hipMallocAsync((void**)&y, sizeof(float) * std::max(1ll, ny), st) != hipSuccess ||
-      hipMallocAsync((void**)&e, sizeof(float) * std::max(1ll, ny), st) != hipSuccess ||
-      hipMallocAsync((void**)&itp, sizeof(int), st) != hipSuccess) {
+  if (tmp_malloc((void**)&x, sizeof(float) * std::max(1ll, nx), st) != hipSuccess ||
+      tmp_malloc((void**)&c, sizeof(float) * std::max(1ll, nx), st) != hipSuccess ||
+      tmp_malloc((void**)&y, sizeof(float) * std::max(1ll, ny), st) != hipSuccess ||
+      tmp_malloc((void**)&e, sizeof(float) * std::max(1ll, ny), st) != hipSuccess ||
+      tmp_malloc((void**)&itp, sizeof(int), st) != hipSuccess) {
     (void)hipGetLastError();
     release();
     (void)hipStreamSynchronize(st);

@@ -739,12 +739,14 @@ template <typename Sink>
 static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
                          int keep_zeros, Sink&& sink) {
   const int V = g.V;
-  long long rowcap = keep_zeros ? V : std::min<long long>(V, 4096);
+  const int nw = walk_waves(g);
+  // entries per row of the scratch: a walked row has no more than its window's cells
+  const int set0 = nw ? walk_first_set(g) : WALK_SETS;
+  long long rowcap = keep_zeros ? V : std::min<long long>(V, set0 < WALK_SETS ? walk_cells[set0] : 4096);
   const size_t budget = (size_t)4 << 30;   // per-row scratch budget
   int* cnt = nullptr;
   int64_t* off = nullptr;
   int* left_d = nullptr;
-  const int nw = walk_waves(g);
   int r0 = 0;
   int maxrows = 0;
   int rc = EPET_OK;
@@ -759,9 +761,9 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
       cnt = nullptr;
       off = nullptr;
       left_d = nullptr;
-      if (hipMallocAsync((void**)&cnt, sizeof(int) * rows, ctx->stream) != hipSuccess ||
-          hipMallocAsync((void**)&left_d, sizeof(int) * rows, ctx->stream) != hipSuccess ||
-          hipMallocAsync((void**)&off, sizeof(int64_t) * (rows + 1), ctx->stream) != hipSuccess) {
+      if (tmp_malloc((void**)&cnt, sizeof(int) * rows, ctx->stream) != hipSuccess ||
+          tmp_malloc((void**)&left_d, sizeof(int) * rows, ctx->stream) != hipSuccess ||
+          tmp_malloc((void**)&off, sizeof(int64_t) * (rows + 1), ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
         rc = fail(EPET_ERR_ALLOC, __FILE__, __LINE__, "row counts");
         break;
@@ -796,7 +798,7 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
       return EPET_OK;
     };
     bool walked = false;
-    for (int set = nw ? walk_first_set(g) : WALK_SETS; set < WALK_SETS && rc == EPET_OK; set++) {
+    for (int set = set0; set < WALK_SETS && rc == EPET_OK; set++) {
       if (walk_lds_bytes(g, nw, walk_cells[set]) > WALK_LDS || (walked && left.empty())) break;
       if (walked) rc = upload(left);
       if (rc == EPET_OK)
@@ -1071,7 +1073,7 @@ int epet_getSystemMatrix(epet_ctx* ctx, float* sme_dev, int* vxlId_dev, int* cnl
   EPET_TRY(read_pinned(ctx, &start, truckDest_dev, sizeof(start)));
   long long written = (long long)start;
   int64_t* tot_dev = nullptr;
-  EPET_HIP(hipMallocAsync((void**)&tot_dev, sizeof(int64_t), ctx->stream));
+  EPET_HIP(tmp_malloc((void**)&tot_dev, sizeof(int64_t), ctx->stream));
   auto sink = [&](int r0, int rows, int* cnt, int64_t* off, long long chunk_nnz, int* scol,
                   float* sval, int rowcap) -> int {
     if (written + chunk_nnz > capacity)
@@ -1123,16 +1125,16 @@ int epet_sm_build(epet_ctx* ctx, const int* list_dev, int m, epet_matrix** out) 
   int* col = nullptr;
   float* val = nullptr;
   int64_t* rowptr = nullptr;
-  EPET_HIP(hipMalloc((void**)&rowptr, sizeof(int64_t) * ((size_t)m + 1)));
+  EPET_HIP(dev_malloc((void**)&rowptr, sizeof(int64_t) * ((size_t)m + 1)));
   auto grow = [&](long long need) -> int {
     if (need <= capacity) return EPET_OK;
     long long cap2 = std::max<long long>(need, capacity + capacity / 4);
     int* c2 = nullptr;
     float* v2 = nullptr;
-    if (hipMalloc((void**)&c2, sizeof(int) * (size_t)std::max(1ll, cap2)) != hipSuccess ||
-        hipMalloc((void**)&v2, sizeof(float) * (size_t)std::max(1ll, cap2)) != hipSuccess) {
+    if (dev_malloc((void**)&c2, sizeof(int) * (size_t)std::max(1ll, cap2)) != hipSuccess ||
+        dev_malloc((void**)&v2, sizeof(float) * (size_t)std::max(1ll, cap2)) != hipSuccess) {
       (void)hipGetLastError();
-      if (c2) (void)hipFree(c2);
+      if (c2) (void)dev_free(c2);
       EPET_FAIL(EPET_ERR_ALLOC, "system matrix allocation of " + std::to_string(cap2) +
                                     " entries failed");
     }
@@ -1142,12 +1144,12 @@ int epet_sm_build(epet_ctx* ctx, const int* list_dev, int m, epet_matrix** out) 
           hipMemcpyAsync(v2, val, sizeof(float) * used, hipMemcpyDeviceToDevice, ctx->stream) !=
               hipSuccess)) ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
-      (void)hipFree(c2);
-      (void)hipFree(v2);
+      (void)dev_free(c2);
+      (void)dev_free(v2);
       EPET_FAIL(EPET_ERR_HIP, "system matrix: growing the arrays");
     }
-    if (col) (void)hipFree(col);
-    if (val) (void)hipFree(val);
+    if (col) (void)dev_free(col);
+    if (val) (void)dev_free(val);
     col = c2; val = v2; capacity = cap2;
     return EPET_OK;
   };
@@ -1175,18 +1177,18 @@ int epet_sm_build(epet_ctx* ctx, const int* list_dev, int m, epet_matrix** out) 
   }
   if (rc != EPET_OK) {
     (void)hipStreamSynchronize(ctx->stream);
-    if (col) (void)hipFree(col);
-    if (val) (void)hipFree(val);
-    (void)hipFree(rowptr);
+    if (col) (void)dev_free(col);
+    if (val) (void)dev_free(val);
+    (void)dev_free(rowptr);
     return rc;
   }
   // channel ids of the rows (the list, or 0..m-1) and the geometry they refer to
   int* ids = nullptr;
-  if (hipMalloc((void**)&ids, sizeof(int) * (size_t)std::max(1, m)) != hipSuccess) {
+  if (dev_malloc((void**)&ids, sizeof(int) * (size_t)std::max(1, m)) != hipSuccess) {
     (void)hipGetLastError();
-    (void)hipFree(col);
-    (void)hipFree(val);
-    (void)hipFree(rowptr);
+    (void)dev_free(col);
+    (void)dev_free(val);
+    (void)dev_free(rowptr);
     EPET_FAIL(EPET_ERR_ALLOC, "row id allocation failed");
   }
   epet_matrix* A = new epet_matrix();

@@ -535,14 +535,14 @@ static void launch_tr_fill(hipStream_t st, int grid, int m, int n, int T, int ti
 }  // namespace epet
 
 epet_matrix::~epet_matrix() {
-  if (bp_toff) (void)hipFree(bp_toff);
-  if (bp_partial) (void)hipFree(bp_partial);
-  if (xb_toff) (void)hipFree(xb_toff);
-  if (xb_partial) (void)hipFree(xb_partial);
-  if (lds_off) (void)hipFree(lds_off);
-  if (lds_val) (void)hipFree(lds_val);
-  if (lds_col16) (void)hipFree(lds_col16);
-  if (lds_partial) (void)hipFree(lds_partial);
+  if (bp_toff) (void)dev_free(bp_toff);
+  if (bp_partial) (void)dev_free(bp_partial);
+  if (xb_toff) (void)dev_free(xb_toff);
+  if (xb_partial) (void)dev_free(xb_partial);
+  if (lds_off) (void)dev_free(lds_off);
+  if (lds_val) (void)dev_free(lds_val);
+  if (lds_col16) (void)dev_free(lds_col16);
+  if (lds_partial) (void)dev_free(lds_partial);
   epet::blk_release(this);
   if (tr) epet_matrix_destroy(tr);
 }
@@ -556,16 +556,16 @@ int matrix_alloc(epet_matrix** out, int m, int n, long long nnz, int value_type)
   A->nnz = nnz;
   A->value_type = value_type;
   const size_t vb = value_type == EPET_VAL_F32 ? 4 : 2;
-  bool ok = hipMalloc((void**)&A->rowptr, sizeof(int64_t) * ((size_t)m + 1)) == hipSuccess &&
-            hipMalloc((void**)&A->col, sizeof(int) * (size_t)std::max(1ll, nnz)) == hipSuccess &&
-            hipMalloc(&A->val, vb * (size_t)std::max(1ll, nnz)) == hipSuccess;
+  bool ok = dev_malloc((void**)&A->rowptr, sizeof(int64_t) * ((size_t)m + 1)) == hipSuccess &&
+            dev_malloc((void**)&A->col, sizeof(int) * (size_t)std::max(1ll, nnz)) == hipSuccess &&
+            dev_malloc((void**)&A->val, vb * (size_t)std::max(1ll, nnz)) == hipSuccess;
   if (ok && value_type != EPET_VAL_F32)
-    ok = hipMalloc((void**)&A->rowscale, sizeof(float) * (size_t)std::max(1, m)) == hipSuccess;
+    ok = dev_malloc((void**)&A->rowscale, sizeof(float) * (size_t)std::max(1, m)) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
-    if (A->rowptr) (void)hipFree(A->rowptr);
-    if (A->col) (void)hipFree(A->col);
-    if (A->val) (void)hipFree(A->val);
+    if (A->rowptr) (void)dev_free(A->rowptr);
+    if (A->col) (void)dev_free(A->col);
+    if (A->val) (void)dev_free(A->val);
     delete A;
     EPET_FAIL(EPET_ERR_ALLOC, "matrix allocation (" + std::to_string(nnz) + " entries) failed");
   }
@@ -683,11 +683,11 @@ int epet_matrix_destroy(epet_matrix* A) {
   if (!A) return EPET_OK;
   (void)hipDeviceSynchronize();
   if (A->owns) {
-    if (A->rowptr) (void)hipFree(A->rowptr);
-    if (A->col) (void)hipFree(A->col);
-    if (A->val) (void)hipFree(A->val);
-    if (A->rowscale) (void)hipFree(A->rowscale);
-    if (A->row_ids) (void)hipFree(A->row_ids);
+    if (A->rowptr) (void)dev_free(A->rowptr);
+    if (A->col) (void)dev_free(A->col);
+    if (A->val) (void)dev_free(A->val);
+    if (A->rowscale) (void)dev_free(A->rowscale);
+    if (A->row_ids) (void)dev_free(A->row_ids);
   }
   delete A;
   return EPET_OK;
@@ -763,7 +763,7 @@ int epet_matrix_select_rows(epet_ctx* ctx, const epet_matrix* A, const int* rows
     EPET_HIP(hipGetLastError());
   }
   if (A->row_ids) {
-    if (hipMalloc((void**)&B->row_ids, sizeof(int) * (size_t)std::max(1, nrows)) != hipSuccess) {
+    if (dev_malloc((void**)&B->row_ids, sizeof(int) * (size_t)std::max(1, nrows)) != hipSuccess) {
       (void)hipGetLastError();
       B->row_ids = nullptr;
     } else if (nrows) {
@@ -803,7 +803,7 @@ int epet_matrix_convert(epet_ctx* ctx, const epet_matrix* A, int vt, epet_matrix
                                          (uint16_t*)B->val, B->rowscale);
     EPET_HIP(hipGetLastError());
   }
-  if (A->row_ids && hipMalloc((void**)&B->row_ids, sizeof(int) * (size_t)std::max(1, A->m)) ==
+  if (A->row_ids && dev_malloc((void**)&B->row_ids, sizeof(int) * (size_t)std::max(1, A->m)) ==
                         hipSuccess) {
     if (A->m)
       EPET_HIP(hipMemcpyAsync(B->row_ids, A->row_ids, sizeof(int) * A->m, hipMemcpyDeviceToDevice,
@@ -860,7 +860,7 @@ int epet_matrix_transpose(epet_ctx* ctx, epet_matrix* A) {
   epet_matrix* T = nullptr;
   EPET_TRY(matrix_alloc(&T, A->n, A->m, A->nnz, A->value_type));
   MatrixGuard keep(T);
-  if (T->rowscale) { (void)hipFree(T->rowscale); T->rowscale = nullptr; }
+  if (T->rowscale) { (void)dev_free(T->rowscale); T->rowscale = nullptr; }
   long long tot = 0;
   EPET_TRY(exclusive_scan_i32_to_i64(ctx, total, T->rowptr, A->n, &tot));
   EPET_CHECK(tot == A->nnz, EPET_ERR_STATE, "transpose count mismatch");

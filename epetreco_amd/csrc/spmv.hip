@@ -266,10 +266,10 @@ int bp_prepare(epet_ctx* ctx, epet_matrix* A) {
   int nblk = std::max(1, std::min(A->m, (target_wgs + T - 1) / T));
   const size_t toff_bytes = sizeof(uint32_t) * (size_t)A->m * (T + 1);
   const size_t part_bytes = sizeof(float) * (size_t)nblk * A->n;
-  if (hipMalloc((void**)&A->bp_toff, toff_bytes) != hipSuccess ||
-      hipMalloc((void**)&A->bp_partial, part_bytes) != hipSuccess) {
+  if (dev_malloc((void**)&A->bp_toff, toff_bytes) != hipSuccess ||
+      dev_malloc((void**)&A->bp_partial, part_bytes) != hipSuccess) {
     (void)hipGetLastError();
-    if (A->bp_toff) (void)hipFree(A->bp_toff);
+    if (A->bp_toff) (void)dev_free(A->bp_toff);
     A->bp_toff = nullptr;
     A->bp_partial = nullptr;
     A->bp_failed = true;   // fall back to the atomic kernel
@@ -424,14 +424,14 @@ void launch_row_plan(hipStream_t st, int m, int T, int TS, const int64_t* rowptr
 void xb_prepare(epet_ctx* ctx, epet_matrix* At) {
   if (At->xb_toff || At->m == 0) return;
   const long long nt = (long long)At->m * (XB_BLOCKS + 1);
-  if (hipMalloc((void**)&At->xb_toff, sizeof(uint32_t) * nt) != hipSuccess) {
+  if (dev_malloc((void**)&At->xb_toff, sizeof(uint32_t) * nt) != hipSuccess) {
     (void)hipGetLastError();
     At->xb_toff = nullptr;
     return;
   }
-  if (hipMalloc((void**)&At->xb_partial, sizeof(float) * (size_t)At->m * XB_BLOCKS) != hipSuccess) {
+  if (dev_malloc((void**)&At->xb_partial, sizeof(float) * (size_t)At->m * XB_BLOCKS) != hipSuccess) {
     (void)hipGetLastError();
-    (void)hipFree(At->xb_toff);
+    (void)dev_free(At->xb_toff);
     At->xb_toff = nullptr;
     At->xb_partial = nullptr;
     return;
