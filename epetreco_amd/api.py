@@ -252,7 +252,8 @@ class Context:
     def mlem_tune(self, A: "Matrix", frames: int):
         """Autotune the multi-frame products for `frames`; returns
         ((rb_fwd, P_fwd, rb_bwd, P_bwd), (ms_fwd, ms_bwd)) for the blocked
-        products, ((R_fwd, P_fwd, R_bwd, P_bwd), ...) for the gather kernels."""
+        products, ((R_fwd, P_fwd, R_bwd, P_bwd), ...) for the gather kernels,
+        ((64, splits_fwd, 64, splits_bwd), ...) for bricks."""
         cfg = np.zeros(4, dtype=np.int32)
         ms = np.zeros(2, dtype=np.float32)
         check(lib().epet_mlem_tune(self._h, A.handle, int(frames),
@@ -268,7 +269,14 @@ class Context:
         check(lib().epet_mlem_kernels(self._h, A.handle, int(frames),
                                       info.ctypes.data_as(_lib.c_int_p),
                                       ms.ctypes.data_as(_lib.c_float_p)))
-        path = {2: "blocked", 1: "gather", 0: "untuned"}[int(info[0])]
+        path = {3: "bricks", 2: "blocked", 1: "gather", 0: "untuned"}[int(info[0])]
+        if path == "bricks":
+            def product(rows, splits, entries, t):
+                return {"rows_per_group": int(info[rows]), "splits": int(info[splits]),
+                        "entries_per_step": int(info[entries]), "tuned_ms": float(ms[t])}
+            return {"path": "bricks (32 x 16 matrix-core steps, k_brk)",
+                    "padded_frames": int(info[1]), "value_parts": int(info[2]),
+                    "forward": product(3, 4, 5, 0), "back_projection": product(7, 8, 6, 1)}
         if path == "blocked":
             def shape(o, t):
                 return {"frames_per_lane": int(info[o]), "lanes_per_row_slot": int(info[o + 1]),

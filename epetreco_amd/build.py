@@ -34,6 +34,7 @@ SOURCES = {
     "mframe.hip": [],
     "lds.hip": [],
     "blk.hip": [],
+    "brk.hip": [],
 }
 
 

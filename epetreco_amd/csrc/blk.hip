@@ -825,7 +825,7 @@ static std::vector<int> voxel_order(const MatGeo& g, int n) {
 // Channel order: by angle, then by the line's midpoint on the detector plane
 // (id0y + id1y, id0z + id1z) in Morton order, then by its slope: lines that
 // cross the same voxels come together.  Identity without channel ids.
-static std::vector<int> channel_order(const MatGeo& g, const std::vector<int>& ids) {
+std::vector<int> channel_order(const MatGeo& g, const std::vector<int>& ids) {
   const int m = (int)ids.size();
   std::vector<int> ord(m);
   std::iota(ord.begin(), ord.end(), 0);

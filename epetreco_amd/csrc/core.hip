@@ -401,6 +401,7 @@ int epet_ctx_create(epet_ctx** out, int device, void* stream) {
                                                                                 : BP_DEFAULT;
     e = getenv("EPET_BATCHED");
     c->opt.batched_gather = e && std::string(e) == "gather";
+    c->opt.batched_blocked = e && std::string(e) == "blocked";
   }
   c->stream = (hipStream_t)stream;
   hipDeviceProp_t prop;

@@ -118,13 +118,15 @@ struct Geo {
 //   EPET_LDS=0         single-frame products without LDS-tiled copies
 //   EPET_LDS_MAP=1     LDS-tiled copies of grid matrices in y-major voxel order
 //   EPET_BP=atomic|tiled|rows   single-frame back-projection variant
-//   EPET_BATCHED=gather         multi-frame MLEM with the gather kernels
+//   EPET_BATCHED=gather|blocked   multi-frame MLEM with the gather kernels, or
+//                               with the blocked products and no bricks
 enum { BP_DEFAULT = 0, BP_ATOMIC = 1, BP_TILED = 2, BP_ROWS = 3 };
 struct EpetOpts {
   bool lds = true;
   bool lds_map = false;
   int bp = BP_DEFAULT;
   bool batched_gather = false;
+  bool batched_blocked = false;
 };
 
 struct epet_ctx {
@@ -172,7 +174,10 @@ struct MatGeo {
   int nx = 0, ny = 0, nz = 0;
 };
 
-namespace epet { struct BlkCopy; }
+namespace epet {
+struct BlkCopy;
+struct BrkCopy;
+}
 
 struct epet_matrix {
   int m = 0, n = 0;
@@ -220,6 +225,9 @@ struct epet_matrix {
   // blocked multi-frame copy (register-accumulated products, one per padded
   // frame count in use) and its autotuned launch shape
   epet::BlkCopy* blk = nullptr;
+  // bricks of the multi-frame products on the matrix cores
+  epet::BrkCopy* brk = nullptr;
+  bool brk_failed = false;
   // multi-frame kernel configuration picked by the autotuner for mf_F frames
   // (rows per wavefront R, frames per lane tile P) and the times it measured
   int mf_F = 0, mf_fwd_R = 1, mf_fwd_P = 32, mf_bwd_R = 1, mf_bwd_P = 32;
@@ -239,6 +247,7 @@ constexpr int LDS_CHUNK = 8;        // tile-major segments are whole chunks of 8
 namespace epet {
 
 void blk_release(epet_matrix* A);   // frees the blocked copies of A
+void brk_release(epet_matrix* A);   // frees its bricks
 
 // device scratch owned by the context, grown on demand (stream-ordered use)
 int ctx_scratch(epet_ctx* ctx, size_t bytes, void** out);

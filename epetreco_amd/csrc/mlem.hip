@@ -49,8 +49,21 @@ int blk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& a, int reps);
 int blk_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& a);
 int blk_info(const epet_matrix* A, int F, int info[9], float ms[2]);
 
-// whether multi-frame MLEM on A runs the blocked products (copies built and
-// tuned for F frames, not turned off by the context)
+int brk_prepare(epet_ctx* ctx, epet_matrix* A, int F);
+bool brk_ready(const epet_matrix* A, int F);
+bool brk_built(const epet_matrix* A, int F);
+int brk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& a, int reps);
+int brk_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& a);
+int brk_info(const epet_matrix* A, int F, int info[9], float ms[2]);
+
+// whether multi-frame MLEM on A runs on bricks (built and tuned for F frames,
+// not turned off by the context), else whether it runs the blocked products
+static bool want_brk(const epet_ctx* ctx) {
+  return !ctx->opt.batched_gather && !ctx->opt.batched_blocked;
+}
+static bool use_brk(const epet_ctx* ctx, const epet_matrix* A, int F) {
+  return want_brk(ctx) && brk_ready(A, F);
+}
 static bool use_blk(const epet_ctx* ctx, const epet_matrix* A, int F) {
   return !ctx->opt.batched_gather && blk_ready(A, F);
 }
@@ -353,7 +366,9 @@ static int mlem_iteration(epet_ctx* ctx, const epet_matrix* A, int F, const floa
   int rc;
   if (F > 1 && A->tr) {
     const MfArgs a{F, x, y, e, c, itp, loglik};
-    rc = use_blk(ctx, A, F) ? blk_iteration(ctx, A, a) : mf_iteration(ctx, A, a);
+    rc = use_brk(ctx, A, F)   ? brk_iteration(ctx, A, a)
+         : use_blk(ctx, A, F) ? blk_iteration(ctx, A, a)
+                              : mf_iteration(ctx, A, a);
   } else {
     // single frame through the transposed copy: the ratio carries the row scale
     // and the back projection is a row-streaming product over the transpose
@@ -540,16 +555,25 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
     if (rc == EPET_OK && !bp_use_transpose(ctx, A)) rc = bp_prepare(ctx, const_cast<epet_matrix*>(A));
     if (rc != EPET_OK) { cleanup(); return rc; }
   } else if (F > 1 && A->tr && !ctx->opt.batched_gather) {
-    // blocked copies (built once per padded frame count) and their launch shape
-    rc = blk_prepare(ctx, const_cast<epet_matrix*>(A), F);
+    // bricks where they pay, and their launch shape
+    if (want_brk(ctx)) {
+      rc = brk_prepare(ctx, const_cast<epet_matrix*>(A), F);
+      if (rc == EPET_OK && brk_built(A, F) && !brk_ready(A, F)) {
+        const MfArgs a{F, x, y, e, c, itp, nullptr};
+        rc = brk_tune(ctx, const_cast<epet_matrix*>(A), a, 2);
+      }
+      if (rc != EPET_OK) { cleanup(); return rc; }
+    }
+    // else blocked copies (built once per padded frame count) and theirs
+    if (!use_brk(ctx, A, F)) rc = blk_prepare(ctx, const_cast<epet_matrix*>(A), F);
     // copies that could not be built leave the gather kernels in place
-    if (rc == EPET_OK && blk_built(A, F) && !blk_ready(A, F)) {
+    if (rc == EPET_OK && !use_brk(ctx, A, F) && blk_built(A, F) && !blk_ready(A, F)) {
       const MfArgs a{F, x, y, e, c, itp, nullptr};
       rc = blk_tune(ctx, const_cast<epet_matrix*>(A), a, 2);
     }
     if (rc != EPET_OK) { cleanup(); return rc; }
   }
-  if (F > 1 && A->tr && !use_blk(ctx, A, F) && A->mf_F != F) {
+  if (F > 1 && A->tr && !use_brk(ctx, A, F) && !use_blk(ctx, A, F) && A->mf_F != F) {
     const MfArgs a{F, x, y, e, c, itp, nullptr};
     rc = mf_tune(ctx, const_cast<epet_matrix*>(A), a, 2);
     if (rc != EPET_OK) { cleanup(); return rc; }
@@ -693,22 +717,35 @@ int epet_mlem_tune(epet_ctx* ctx, epet_matrix* A, int F, int* cfg, float* ms) {
   k_fill_i32_one<<<1, 64, 0, st>>>(itp, 0);
   const MfArgs a{F, x, y, e, c, itp, nullptr};
   int rc = EPET_OK;
-  bool blocked = false;
-  if (!ctx->opt.batched_gather) {
+  bool blocked = false, bricks = false;
+  if (want_brk(ctx)) {
+    rc = brk_prepare(ctx, A, F);
+    if (rc == EPET_OK && brk_built(A, F)) {
+      rc = brk_tune(ctx, A, a, 3);
+      bricks = true;
+    }
+  }
+  if (rc == EPET_OK && !bricks && !ctx->opt.batched_gather) {
     rc = blk_prepare(ctx, A, F);
     if (rc == EPET_OK && blk_built(A, F)) {
       rc = blk_tune(ctx, A, a, 3);
       blocked = true;
     }
   }
-  if (rc == EPET_OK && !blocked) {
+  if (rc == EPET_OK && !blocked && !bricks) {
     A->mf_F = 0;
     rc = mf_tune(ctx, A, a, 3);
   }
   release();
   EPET_HIP(hipStreamSynchronize(st));
   if (rc != EPET_OK) return rc;
-  if (blocked) {
+  if (bricks) {
+    int info[9];
+    float t[2];
+    EPET_TRY(brk_info(A, F, info, t));
+    if (cfg) { cfg[0] = info[3]; cfg[1] = info[4]; cfg[2] = info[7]; cfg[3] = info[8]; }
+    if (ms) { ms[0] = t[0]; ms[1] = t[1]; }
+  } else if (blocked) {
     int info[9];
     float t[2];
     EPET_TRY(blk_info(A, F, info, t));
@@ -725,7 +762,12 @@ int epet_mlem_kernels(epet_ctx* ctx, const epet_matrix* A, int F, int* info, flo
   EPET_CHECK(ctx && A && info, EPET_ERR_ARG, "null argument");
   for (int i = 0; i < 10; i++) info[i] = 0;
   float t[2] = {0.0f, 0.0f};
-  if (F >= 2 && A->tr && use_blk(ctx, A, F)) {
+  if (F >= 2 && A->tr && use_brk(ctx, A, F)) {
+    int bi[9];
+    EPET_TRY(brk_info(A, F, bi, t));
+    info[0] = 3;
+    for (int i = 1; i < 9; i++) info[i] = bi[i];
+  } else if (F >= 2 && A->tr && use_blk(ctx, A, F)) {
     int bi[9];
     EPET_TRY(blk_info(A, F, bi, t));
     info[0] = 2;

@@ -544,6 +544,7 @@ epet_matrix::~epet_matrix() {
   if (lds_col16) (void)dev_free(lds_col16);
   if (lds_partial) (void)dev_free(lds_partial);
   epet::blk_release(this);
+  epet::brk_release(this);
   if (tr) epet_matrix_destroy(tr);
 }
 

@@ -265,7 +265,10 @@ int epet_mlem_noalloc(epet_ctx* ctx, const epet_matrix* A, const float* y_dev,
                       const float* s_dev, float* x_dev, int niter, double* loglik_out);
 
 /* Autotuner of the multi-frame products epet_mlem runs for F frames on A and
- * its attached transpose.  Blocked products (the default): every shape of
+ * its attached transpose.  Bricks (generated matrices, where 64 neighbouring
+ * rows share enough columns): the splits of each direction are timed and the
+ * fastest kept; cfg = {64, splits_fwd, 64, splits_bwd} (rows per group).
+ * Blocked products (other matrices): every shape of
  * (rows per block rb in {128,256,512,1024}) x (frames per lane P in {4,8}) that
  * fits the workgroup's LDS is timed per direction and the fastest kept;
  * cfg = {rb_fwd, P_fwd, rb_bwd, P_bwd}.  Gather kernels
@@ -278,7 +281,9 @@ int epet_mlem_noalloc(epet_ctx* ctx, const epet_matrix* A, const float* y_dev,
 int epet_mlem_tune(epet_ctx* ctx, epet_matrix* A, int F, int* cfg, float* ms);
 
 /* The multi-frame path epet_mlem runs for F frames on A, as tuned: info (10
- * ints).  Blocked products: {2, P_fwd, lanes per row slot fwd, rows per block
+ * ints).  Bricks: {3, padded frames, parts of a stored value, rows per group
+ * fwd, splits fwd, entries per step fwd, entries per step bwd, rows per group
+ * bwd, splits bwd, 0}.  Blocked products: {2, P_fwd, lanes per row slot fwd, rows per block
  * fwd, splits fwd, P_bwd, lanes bwd, rows per block bwd, splits bwd, 0}.
  * Gather kernels: {1, P_fwd, R_fwd, 0, 0, P_bwd, R_bwd, 0, 0, 0}.  {0, ...}:
  * not tuned yet.  ms (2 floats, may be NULL) = the tuned times per launch. */
