@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -226,8 +227,10 @@ struct epet_matrix {
   // frame count in use) and its autotuned launch shape
   epet::BlkCopy* blk = nullptr;
   // bricks of the multi-frame products on the matrix cores
+  // (brk_state on the matrix itself: 0 not asked for yet, 1 built, -1 not to be)
   epet::BrkCopy* brk = nullptr;
-  bool brk_failed = false;
+  std::atomic<int> brk_state{0};
+  std::atomic<long long> brk_work{0};   // entries x frames multiplied before the bricks
   // multi-frame kernel configuration picked by the autotuner for mf_F frames
   // (rows per wavefront R, frames per lane tile P) and the times it measured
   int mf_F = 0, mf_fwd_R = 1, mf_fwd_P = 32, mf_bwd_R = 1, mf_bwd_P = 32;

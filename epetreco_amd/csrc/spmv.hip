@@ -579,8 +579,16 @@ static int launch_spmm(hipStream_t st, const epet_matrix* A, int op, int F, floa
   return EPET_OK;
 }
 
+int brk_spmm(epet_ctx* ctx, const epet_matrix* A, int op, int F, float alpha, const float* X,
+             float beta, float* Y, bool* done);
+
 int matrix_spmm(epet_ctx* ctx, const epet_matrix* A, int op, int F, float alpha, const float* X,
                 float beta, float* Y) {
+  if (!ctx->opt.batched_gather && !ctx->opt.batched_blocked) {
+    bool done = false;
+    EPET_TRY(brk_spmm(ctx, A, op, F, alpha, X, beta, Y, &done));
+    if (done) return EPET_OK;
+  }
   switch (A->value_type) {
     case EPET_VAL_F32: return launch_spmm<ValF32>(ctx->stream, A, op, F, alpha, X, beta, Y);
     case EPET_VAL_BF16: return launch_spmm<ValBF16>(ctx->stream, A, op, F, alpha, X, beta, Y);

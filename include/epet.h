@@ -215,7 +215,10 @@ int epet_csrmv(epet_ctx* ctx, int op, int m, int n, long long nnz,
 int epet_matrix_spmv(epet_ctx* ctx, const epet_matrix* A, int op, float alpha,
                      const float* x_dev, float beta, float* y_dev);
 /* Multi-vector product: X and Y are frame-minor (X[j*nrhs + f]), nrhs <= 64.
- * op N: Y(m x nrhs) = alpha*A*X + beta*Y; op T: Y(n x nrhs) = alpha*A^T X + beta*Y. */
+ * op N: Y(m x nrhs) = alpha*A*X + beta*Y; op T: Y(n x nrhs) = alpha*A^T X + beta*Y.
+ * A generated matrix with its transposed copy attached keeps bricks for the
+ * matrix cores (see epet_mlem) once products enough have been asked of it: that
+ * call synchronises, and sums are in another order from then on. */
 int epet_matrix_spmm(epet_ctx* ctx, const epet_matrix* A, int op, int nrhs,
                      float alpha, const float* X_dev, float beta, float* Y_dev);
 

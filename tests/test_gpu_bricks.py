@@ -142,3 +142,68 @@ def test_not_finite(gpu_ctx_factory, monkeypatch, what, F):
     assert np.array_equal(np.isnan(ll), np.isnan(llb)) and np.array_equal(np.isinf(ll), np.isinf(llb))
     ok = np.isfinite(llb)
     np.testing.assert_allclose(ll[ok], llb[ok], rtol=1e-6)
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("F", [2, 4, 8, 11, 32, 64])
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (-0.5, 1.5)])
+def test_products(gpu_ctx_factory, storage, F, alpha, beta):
+    """spmm on bricks (transposed copy attached) against FP64 on the stored values:
+    rtol 2e-5 of the sum of magnitudes, the bar of the other products."""
+    import scipy.sparse as sp
+    from epetreco_amd.api import OP_N, OP_T
+    ctx, A = _problem(gpu_ctx_factory, 15, 13, 17, 24, 6, 1, storage)
+    rp, col, val = decoded(A)
+    M = sp.csr_matrix((val.astype(np.float64), col, rp), shape=(A.m, A.n))
+    A.spmm(OP_N, torch.zeros(A.n, 64, device="cuda"))   # enough work for the bricks to be built
+    rng = np.random.default_rng(F)
+    for op, K, nin, nout in ((OP_N, M, A.n, A.m), (OP_T, M.T, A.m, A.n)):
+        X = rng.normal(size=(nin, F)).astype(np.float32)
+        Y0 = rng.normal(size=(nout, F)).astype(np.float32)
+        Y = torch.as_tensor(Y0, device="cuda")
+        A.spmm(op, torch.as_tensor(X, device="cuda"), Y, alpha=alpha, beta=beta)
+        want = alpha * (K @ X.astype(np.float64)) + beta * Y0
+        bar = 2e-5 * (abs(alpha) * (abs(K) @ np.abs(X)) + abs(beta * Y0)) + 1e-30
+        assert np.all(np.abs(Y.cpu().numpy() - want) <= bar)
+
+
+def test_products_on_two_streams_and_in_a_graph(gpu_ctx_factory):
+    """Calls on two streams share nothing; a captured call runs the kernels that
+    need no working memory, and replays give the eager result."""
+    from epetreco_amd.api import OP_N, OP_T, Context
+    ctx, A = _problem(gpu_ctx_factory, 15, 13, 17, 24, 6, 1, "f32")
+    A.spmm(OP_T, torch.zeros(A.m, 64, device="cuda"))
+    X = [torch.rand(A.m, 6, device="cuda") for _ in range(2)]
+    want = [A.spmm(OP_T, x).double() for x in X]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    ctxs = []
+    for st in streams:
+        with torch.cuda.stream(st):
+            ctxs.append(Context(0, st))
+    from epetreco_amd._lib import check, lib
+    import ctypes
+    outs = [[torch.zeros(A.n, 6, device="cuda") for _ in range(20)] for _ in range(2)]
+    torch.cuda.synchronize()
+    for k in range(20):
+        for i in range(2):
+            check(lib().epet_matrix_spmm(ctxs[i].handle, A.handle, OP_T, 6, 1.0,
+                                         ctypes.c_void_p(X[i].data_ptr()), 0.0,
+                                         ctypes.c_void_p(outs[i][k].data_ptr())))
+    torch.cuda.synchronize()
+    for i in range(2):
+        for o in outs[i]:
+            assert (o.double() - want[i]).norm() <= 1e-6 * want[i].norm()
+    # captured
+    g = torch.cuda.CUDAGraph()
+    y = torch.zeros(A.n, 6, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=streams[0]):
+        check(lib().epet_matrix_spmm(ctxs[0].handle, A.handle, OP_T, 6, 1.0,
+                                     ctypes.c_void_p(X[0].data_ptr()), 0.0,
+                                     ctypes.c_void_p(y.data_ptr())))
+    for _ in range(3):
+        y.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert (y.double() - want[0]).norm() <= 1e-6 * want[0].norm()
