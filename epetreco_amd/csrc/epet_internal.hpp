@@ -221,6 +221,8 @@ struct epet_matrix {
   void* lds_val = nullptr;
   uint16_t* lds_col16 = nullptr;
   float* lds_partial = nullptr;
+  int4* lds_plan = nullptr;   // rows of every wavefront of lds_wgs workgroups
+  int lds_wgs = 0;
   ColMap lds_map;
   bool lds_failed = false;
   // blocked multi-frame copy (register-accumulated products, one per padded

@@ -1,27 +1,38 @@
 // lds.hip -- LDS-tiled row products y = A x (and, over a transposed copy, the
 // back projection).
 //
-// The gathered vector x (n entries) is cut into tiles of LDS_TILE entries.
-// Workgroup (tile t, row range g) of 1024 threads copies tile t into LDS, then
-// its 16 wavefronts walk the rows of range g, R rows per wavefront at a time,
-// summing each row's entries whose column lies in tile t (an entry range given
-// by the per-matrix plan, since columns ascend within a row) with x read from
-// LDS.  The row's partial for tile t goes to partial[t m + r]; a reduction sums
-// the partials of every row in tile order (deterministic) and applies the row
-// scale, alpha/beta or the MLEM ratio.
+// The gathered vector x (n entries) is cut into tiles of LDS_TILE entries.  A
+// workgroup of 1024 threads copies one tile into LDS and sums, for its rows, the
+// entries whose column lies in that tile, with x read from LDS.  The row's
+// partial for tile t goes to partial[t m + r]; a reduction sums the partials of
+// every row in tile order (deterministic) and applies the row scale, alpha/beta
+// or the MLEM ratio.  With a single tile the product is written at once.
 //
 // The kernels read a tile-major copy of the matrix built once per matrix: the
 // entries of (tile t, row r) lie contiguously at lds_off[t m + r], rows of one
-// tile back to back, columns stored tile-local in 16 bits.  A cache line that
-// straddles two segments then belongs to neighbouring rows of the same
-// workgroup and is read from HBM once, and an FP32 entry costs 6 bytes.  HBM
-// sees the entry stream once, x once per workgroup, and 12 bytes of offset and
-// partial per (row, tile).
+// tile back to back, columns stored tile-local in 16 bits, every segment padded
+// to whole chunks of 8 entries.  So an FP32 entry costs 6 bytes, HBM sees the
+// entry stream once, x once per workgroup, and 12 bytes of offset and partial per
+// (row, tile).
+//
+// What bounds it is that stream, and keeping it in flight.  A wavefront therefore
+// runs through its rows' chunks as one stream, 64 chunks (a block) at a time
+// whatever the rows' lengths, three blocks requested ahead; a lane's chunk belongs
+// to one row, and the lanes' sums are added up by row with a segmented scan.
+// Before, R rows at a time had 64/R lanes each and one chunk per lane in flight:
+// lanes idle at every row's end, and a wait per pass.  The rows are dealt out so
+// that every wavefront has the same number of chunks (k_lds_plan).
+// Forward / back projection, FP32, 52^3 voxels, before -> now:
+//   1,100,000 rows, 979M entries   1163 -> 1055 / 1199 -> 1027 us (5.6 TB/s)
+//   100,000 rows, 88M entries       141 ->  107 /  212 ->  106 us
+//   11,250 rows, 4.6M entries        19 ->   11 us forward
+// (a large tensor is read at 6.2 TB/s on the same card.)
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "epet_block.hpp"
 #include "epet_internal.hpp"
@@ -34,129 +45,206 @@ void launch_row_plan(hipStream_t st, int m, int T, int TS, const int64_t* rowptr
 
 constexpr int LDS_BLOCK = 1024;
 constexpr int LDS_WAVES = LDS_BLOCK / WAVE;
+// blocks in flight per wavefront: 1 / 2 / 3 / 4 / 6 took 1131 / 1126 / 1126 / 1138 /
+// 1139 us forward and 1247 / 1167 / 1155 / 1172 / 1175 us back at 979M entries
+constexpr int LDS_DEPTH = 3;
+// Workgroups: as many per CU as give every wavefront LDS_MIN_BLOCKS blocks, at most
+// LDS_PER_CU.  More even out the card's unequal speeds, but each copies its 128 KB
+// tile before its first product, and one workgroup's LDS fills a CU.  At 979M
+// entries 8 / 16 / 32 / 64 per CU took 1122 / 1076 / 1055 / 1117 us forward; at
+// 88M, 4 / 8 / 12 / 16 blocks at least took 137 / 113 / 109 / 107 us.
+constexpr int LDS_MIN_BLOCKS = 16, LDS_PER_CU = 32;
+// A row's own cost in chunks: rows with next to no entries in a tile still take
+// their turn in a window of 64.  At 88M entries (the fifth tile nearly empty) 0 /
+// 0.25 / 0.5 / 1 / 2 / 4 took 235 / 136 / 117 / 111 / 110 / 119 us forward.
+constexpr int LDS_ROW_COST = 2;
 
-// A chunk of LDS_CHUNK entries of the tile-major copy: eight 16-bit columns
-// (one 16-byte load) and eight values (one or two 16-byte loads).
-template <typename VT> struct LdsChunk;
-template <> struct LdsChunk<ValF32> {
-  static __device__ __forceinline__ void load(const float* __restrict__ val, long long k,
-                                              float v[8]) {
-    const float4 a = *reinterpret_cast<const float4*>(val + k);
-    const float4 b = *reinterpret_cast<const float4*>(val + k + 4);
+// The values of a chunk of LDS_CHUNK entries of the tile-major copy (one or two
+// 16-byte loads; its eight 16-bit columns are a third).
+template <typename VT> struct LdsChunkRaw {
+  uint4 a;
+  __device__ __forceinline__ void load(const uint16_t* __restrict__ val, long long k) {
+    a = *reinterpret_cast<const uint4*>(val + k);
+  }
+  __device__ __forceinline__ void get(float v[8]) const {
+    const unsigned w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      if constexpr (std::is_same<VT, ValBF16>::value) {
+        v[2 * i] = __uint_as_float(w[i] << 16);
+        v[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
+      } else {
+        v[2 * i] = __half2float(__ushort_as_half((uint16_t)(w[i] & 0xFFFFu)));
+        v[2 * i + 1] = __half2float(__ushort_as_half((uint16_t)(w[i] >> 16)));
+      }
+    }
+  }
+};
+template <> struct LdsChunkRaw<ValF32> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* __restrict__ val, long long k) {
+    a = *reinterpret_cast<const float4*>(val + k);
+    b = *reinterpret_cast<const float4*>(val + k + 4);
+  }
+  __device__ __forceinline__ void get(float v[8]) const {
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
   }
 };
-template <> struct LdsChunk<ValBF16> {
-  static __device__ __forceinline__ void load(const uint16_t* __restrict__ val, long long k,
-                                              float v[8]) {
-    const uint4 a = *reinterpret_cast<const uint4*>(val + k);
-    const unsigned w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      v[2 * i] = __uint_as_float(w[i] << 16);
-      v[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
+
+// Where a row's sum goes: its tile's partial, or with one tile the result.
+struct LdsStore {
+  int direct;
+  const float* rowscale;
+  float alpha, beta;
+  __device__ __forceinline__ void store(float* __restrict__ out, int t, int m, long long r,
+                                        float s) const {
+    if (!direct) {
+      out[(long long)t * m + r] = s;
+      return;
     }
-  }
-};
-template <> struct LdsChunk<ValF16> {
-  static __device__ __forceinline__ void load(const uint16_t* __restrict__ val, long long k,
-                                              float v[8]) {
-    const uint4 a = *reinterpret_cast<const uint4*>(val + k);
-    const unsigned w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      v[2 * i] = __half2float(__ushort_as_half((uint16_t)(w[i] & 0xFFFFu)));
-      v[2 * i + 1] = __half2float(__ushort_as_half((uint16_t)(w[i] >> 16)));
-    }
+    const float v = alpha * (rowscale ? rowscale[r] : 1.0f) * s;
+    out[r] = beta == 0.0f ? v : v + beta * out[r];
   }
 };
 
-// R rows per wavefront (L = 64/R lanes per row), J chunks of LDS_CHUNK entries
-// per lane per pass; BWD = 1 marks the back projection over a transposed copy
-// (a separate instantiation, so that profiles tell the two products apart).
-template <typename VT, int R, int J, int BWD>
-__global__ __launch_bounds__(LDS_BLOCK) void k_rows_lds(int m, int n, int T, long long rows_per_wg,
+// Lane l's value of the lane d below it in the same row of 16 (0 shifted in).
+template <int D>
+__device__ __forceinline__ float dpp_shr(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x110 + D, 0xF, 0xF, true));
+}
+
+// Sums over the lanes of each segment up to and including the own lane: `before`
+// is the number of lanes below the own one that belong to its segment.
+__device__ __forceinline__ float segment_scan(float v, int before, int lane) {
+  const int in16 = lane & 15, b16 = std::min(before, in16);
+  float t;
+  t = dpp_shr<1>(v);
+  v += b16 >= 1 ? t : 0.0f;
+  t = dpp_shr<2>(v);
+  v += b16 >= 2 ? t : 0.0f;
+  t = dpp_shr<4>(v);
+  v += b16 >= 4 ? t : 0.0f;
+  t = dpp_shr<8>(v);
+  v += b16 >= 8 ? t : 0.0f;
+  // carries across the rows of 16: each row's last lane into the next row
+#pragma unroll
+  for (int row = 1; row < 4; row++) {
+    const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16 * row - 1));
+    if ((lane >> 4) == row && before > in16) v += c;
+  }
+  return v;
+}
+
+template <typename VT>
+struct LdsBlock {
+  uint4 c;
+  LdsChunkRaw<VT> v;
+};
+
+// D blocks of 64 chunks in flight per wavefront; BWD = 1 marks the back
+// projection over a transposed copy (a separate instantiation, so that profiles
+// tell the two products apart).  out: the partials, or with T = 1 the result.
+template <typename VT, int D, int BWD>
+__global__ __launch_bounds__(LDS_BLOCK) void k_rows_lds(int m, int n, const int4* __restrict__ plan,
                                                         const int64_t* __restrict__ off,
                                                         const uint16_t* __restrict__ col,
                                                         const typename VT::T* __restrict__ val,
                                                         const float* __restrict__ x,
-                                                        float* __restrict__ partial, ColMap mp) {
+                                                        float* __restrict__ out, LdsStore ep,
+                                                        ColMap mp) {
   extern __shared__ float xs[];
-  constexpr int L = WAVE / R;
-  const int t = blockIdx.x % T;
-  const long long g = blockIdx.x / T;
+  const int lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  // this wavefront's rows [wa, wb) of tile t and their chunks [q, qe)
+  const int4 unit = plan[(long long)blockIdx.x * LDS_WAVES + w];
+  const int t = unit.z;
+  if (t < 0) return;   // the whole workgroup
+  const long long wa = unit.x, wb = unit.y;
   const long long tb = (long long)t * LDS_TILE;
   const int cnt = (int)std::min<long long>(LDS_TILE, (long long)n - tb);
+  const int64_t* offt = off + (long long)t * m;
+  long long q = offt[wa] / LDS_CHUNK;
+  const long long qe = offt[wb] / LDS_CHUNK, qlast = std::max(0ll, qe - 1);
+  auto load = [&](long long qb) {
+    LdsBlock<VT> b;
+    const long long k = std::min(qb + lane, qlast) * LDS_CHUNK;   // past the end: not used
+    b.c = *reinterpret_cast<const uint4*>(col + k);
+    b.v.load(val, k);
+    return b;
+  };
+  LdsBlock<VT> buf[D];
+#pragma unroll
+  for (int j = 0; j < D; j++) buf[j] = load(q + (long long)j * WAVE);
+  // lane l owns row wr + l of the window: its chunks [s, e)
+  long long wr = wa;
+  auto bound = [&](long long r) { return offt[std::min(r, wb)] / LDS_CHUNK; };
+  long long s = bound(wr + lane), e = bound(wr + lane + 1);
+  long long ns = bound(wr + WAVE + lane), ne = bound(wr + WAVE + lane + 1);
   if (mp.nx == 0) {
     // tile copy: 16-byte loads when the tile start is 16-byte aligned
     const int c4 = ((reinterpret_cast<uintptr_t>(x + tb) & 15) == 0) ? (cnt >> 2) : 0;
-    for (int i = threadIdx.x; i < c4; i += LDS_BLOCK)
-      reinterpret_cast<float4*>(xs)[i] = reinterpret_cast<const float4*>(x + tb)[i];
+    const float4* x4 = reinterpret_cast<const float4*>(x + tb);
+    constexpr int N4 = LDS_TILE / 4 / LDS_BLOCK;
+    if (c4 == N4 * LDS_BLOCK) {   // a whole tile: all its loads at once
+      float4 r[N4];
+#pragma unroll
+      for (int i = 0; i < N4; i++) r[i] = x4[threadIdx.x + i * LDS_BLOCK];
+#pragma unroll
+      for (int i = 0; i < N4; i++) reinterpret_cast<float4*>(xs)[threadIdx.x + i * LDS_BLOCK] = r[i];
+    } else {
+#pragma unroll 4
+      for (int i = threadIdx.x; i < c4; i += LDS_BLOCK) reinterpret_cast<float4*>(xs)[i] = x4[i];
+    }
     for (int i = (c4 << 2) + threadIdx.x; i < cnt; i += LDS_BLOCK) xs[i] = x[tb + i];
   } else {
     // renumbered columns: tile entry i is column colmap_inv(tb + i) of x
     for (int i = threadIdx.x; i < cnt; i += LDS_BLOCK) xs[i] = x[colmap_inv(tb + i, mp)];
   }
   __syncthreads();
-  const int lane = lane_id(), gi = lane / L, l = lane % L;
-  const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  const long long r0 = g * rows_per_wg;
-  const long long r1 = std::min<long long>((long long)m, r0 + rows_per_wg);
+  if (wa >= wb) return;
   const unsigned last = (unsigned)(cnt - 1);
-  const long long step = (long long)LDS_WAVES * R;
-  const int64_t* offt = off + (long long)t * m;
-  // segment [s0, s1) of row rbx + gi in tile t (whole chunks); empty past the range
-  auto segment = [&](long long rbx, long long& s0, long long& s1) {
-    s0 = 0;
-    s1 = 0;
-    const long long r = rbx + gi;
-    if (r < r1) {
-      s0 = offt[r];
-      s1 = offt[r + 1];
-    }
-  };
-  long long rb = r0 + (long long)w * R;
-  long long n0, n1;
-  segment(rb, n0, n1);
-  for (; rb < r1; rb += step) {
-    const long long r = rb + gi;
-    const bool ok = r < r1;
-    const long long s0 = n0, s1 = n1;
-    segment(rb + step, n0, n1);   // the next segment's bounds, requested before this one's entries
-    float acc = 0.0f;
-    for (long long base = s0 + (long long)l * LDS_CHUNK; base < s1;
-         base += (long long)L * LDS_CHUNK * J) {
-      // J chunks: columns and values requested together (ordinary cached
-      // loads), chunks past the segment skipped
-      uint4 c[J];
-      float v[J][LDS_CHUNK];
-      bool in[J];
+  float acc = 0.0f;
+  for (;;) {
 #pragma unroll
-      for (int j = 0; j < J; j++) {
-        const long long k = base + (long long)j * L * LDS_CHUNK;
-        in[j] = k < s1;
-        const long long kc = in[j] ? k : base;
-        c[j] = *reinterpret_cast<const uint4*>(col + kc);
-        LdsChunk<VT>::load(val, kc, v[j]);
+    for (int j = 0; j < D; j++) {
+      const unsigned cw[4] = {buf[j].c.x, buf[j].c.y, buf[j].c.z, buf[j].c.w};
+      float v[LDS_CHUNK];
+      buf[j].v.get(v);
+      float a = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        // the clamp keeps LDS reads in range whatever the data
+        const unsigned lo = std::min(cw[i] & (i == 0 ? 0x7FFFu : 0xFFFFu), last);
+        const unsigned hi = std::min(cw[i] >> 16, last);
+        a += v[2 * i] * xs[lo];
+        a += v[2 * i + 1] * xs[hi];
       }
-#pragma unroll
-      for (int j = 0; j < J; j++) {
-        const unsigned cw[4] = {c[j].x, c[j].y, c[j].z, c[j].w};
-        float a = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          // the clamp keeps LDS reads in range whatever the data
-          const unsigned lo = std::min(cw[i] & 0xFFFFu, last), hi = std::min(cw[i] >> 16, last);
-          a += v[j][2 * i] * xs[lo];
-          a += v[j][2 * i + 1] * xs[hi];
-        }
-        acc += in[j] ? a : 0.0f;
+      // lanes of the own segment below the own lane
+      const unsigned long long heads = __ballot((cw[0] & 0x8000u) != 0);
+      const unsigned long long below = heads & (~0ull >> (63 - lane));
+      a = segment_scan(a, below ? lane - (63 - __clzll((long long)below)) : lane, lane);
+      buf[j] = load(q + (long long)D * WAVE);
+      const long long qn = q + WAVE;
+      for (;;) {
+        // the part of the own row in this block ends at lane min(e, qn) - 1 - q
+        const int at = (int)(std::min(e, qn) - 1 - q);
+        const float p = __shfl(a, at & (WAVE - 1), WAVE);
+        if (s < qn && e > q && s < e) acc += p;
+        if (lane_value_i64(e, WAVE - 1) > qn) break;   // the window goes on in the next block
+        const long long r = wr + lane;
+        if (r < wb) ep.store(out, t, m, r, acc);
+        wr += WAVE;
+        if (wr >= wb) return;
+        acc = 0.0f;
+        s = ns;
+        e = ne;
+        ns = bound(wr + WAVE + lane);
+        ne = bound(wr + WAVE + lane + 1);
       }
+      q = qn;
     }
-#pragma unroll
-    for (int o = L / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, L);
-    if (ok && l == 0) partial[(long long)t * m + r] = acc;
   }
 }
 
@@ -237,7 +325,8 @@ __global__ void k_lds_set_last(int64_t* __restrict__ off, long long i, long long
 }
 
 // one wavefront per (tile, row) segment: copy values and tile-local columns,
-// then zero entries (column 0, value 0) up to the padded length
+// then zero entries (the segment's last column, value 0) up to the padded length.
+// Bit 15 of a segment's first column marks it.
 template <typename T>
 __global__ __launch_bounds__(256) void k_lds_fill(int m, int T_, int mask,
                                                   const int64_t* __restrict__ rowptr,
@@ -259,10 +348,54 @@ __global__ __launch_bounds__(256) void k_lds_fill(int m, int T_, int mask,
     const long long dst = off[i], plen = off[i + 1] - dst;
     for (long long k = lane; k < plen; k += WAVE) {
       const bool in = k < len;
-      col16[dst + k] = in ? (uint16_t)(col[src + k] & mask) : (uint16_t)0;
+      const int c = col[src + (in ? k : len - 1)] & mask;
+      col16[dst + k] = (uint16_t)(k == 0 ? c | 0x8000 : c);
       val2[dst + k] = in ? val[src + k] : (T)0;
     }
   }
+}
+
+// ------------------------------------------------------------------ work split
+// Unit u = 16 wg + w: the rows (x, y) of tile z that wavefront w of workgroup wg
+// sums.  Tile t has max(1, ceil(cost / target)) workgroups, cost = chunks +
+// LDS_ROW_COST rows, and its cost is cut evenly over their wavefronts, each row
+// going to the wavefront its first chunk falls to; z = -1 past the last tile's
+// workgroups.
+__global__ __launch_bounds__(256) void k_lds_plan(int m, int T, long long target, long long nunits,
+                                                  const int64_t* __restrict__ off,
+                                                  int4* __restrict__ plan) {
+  const long long u = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= nunits) return;
+  long long wg = u / LDS_WAVES;
+  int t = 0;
+  long long c0 = 0, chunks = 0, wgs = 0;
+  for (; t < T; t++) {
+    c0 = off[(long long)t * m] / LDS_CHUNK;
+    chunks = off[(long long)(t + 1) * m] / LDS_CHUNK - c0 + (long long)LDS_ROW_COST * m;
+    wgs = std::max(1ll, (chunks + target - 1) / target);
+    if (wg < wgs) break;
+    wg -= wgs;
+  }
+  if (t == T) {
+    plan[u] = make_int4(0, 0, -1, 0);
+    return;
+  }
+  const int64_t* offt = off + (long long)t * m;
+  const long long k = wg * LDS_WAVES + u % LDS_WAVES, nk = wgs * LDS_WAVES;
+  // first row whose first chunk is at or past share j of the tile
+  auto row = [&](long long j) {
+    if (j == 0) return 0;
+    if (j == nk) return m;
+    const long long c = c0 + (long long)((double)chunks * (double)j / (double)nk);
+    int lo = 0, hi = m;
+    while (lo < hi) {
+      const int mid = lo + (hi - lo) / 2;
+      if (offt[mid] / LDS_CHUNK + (long long)LDS_ROW_COST * mid < c) lo = mid + 1;
+      else hi = mid;
+    }
+    return lo;
+  };
+  plan[u] = make_int4(row(k), row(k + 1), t, 0);
 }
 
 // ------------------------------------------------------------------ reductions
@@ -312,45 +445,30 @@ __global__ __launch_bounds__(256) void k_lds_ratio(int m, int T, const float* __
 }
 
 // ------------------------------------------------------------------ dispatch
-template <typename VT, int R, int J, int BWD>
-static void launch_rows_lds(epet_ctx* ctx, const epet_matrix* A, const float* x) {
+template <typename VT, int BWD>
+static void launch_rows_lds(epet_ctx* ctx, const epet_matrix* A, const float* x, float* out,
+                            const LdsStore& ep) {
+  constexpr int D = LDS_DEPTH;
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)k_rows_lds<VT, R, J, BWD>,
+    (void)hipFuncSetAttribute((const void*)k_rows_lds<VT, D, BWD>,
                               hipFuncAttributeMaxDynamicSharedMemorySize,
                               LDS_TILE * (int)sizeof(float));
     attr = true;
   }
-  // each workgroup owns its CU's LDS; several workgroups per CU in all, so
-  // that tiles and row ranges of unequal weight even out: 12 for the forward
-  // and 24 for the back projection at 52^3 (4 to 32 per CU were within a few
-  // percent of each other)
-  const long long per_cu = BWD ? 24 : 12;
-  const long long G = std::max<long long>(1, (per_cu * ctx->num_cus + A->lds_T - 1) / A->lds_T);
-  const long long rows_per_wg = std::max<long long>(LDS_WAVES * R, (A->m + G - 1) / G);
-  const long long ng = (A->m + rows_per_wg - 1) / rows_per_wg;
-  k_rows_lds<VT, R, J, BWD><<<(unsigned)(ng * A->lds_T), LDS_BLOCK, LDS_TILE * sizeof(float),
-                             ctx->stream>>>(A->m, A->n, A->lds_T, rows_per_wg, A->lds_off,
-                                            A->lds_col16, (const typename VT::T*)A->lds_val, x,
-                                            A->lds_partial, A->lds_map);
-}
-
-// Rows per wavefront from the mean segment length; one chunk per lane per pass
-// (at 52^3 two chunks per pass took 8.1 ms per MLEM iteration, one 6.9-7.2 ms).
-template <typename VT, int BWD>
-static void rows_lds_dispatch(epet_ctx* ctx, const epet_matrix* A, const float* x) {
-  const double seg = (double)A->nnz / std::max(1.0, (double)A->m * A->lds_T);
-  if (seg >= 384.0) launch_rows_lds<VT, 2, 1, BWD>(ctx, A, x);
-  else if (seg >= 48.0) launch_rows_lds<VT, 4, 1, BWD>(ctx, A, x);
-  else launch_rows_lds<VT, 16, 1, BWD>(ctx, A, x);
+  const size_t lds = sizeof(float) * (size_t)std::min(LDS_TILE, A->n);
+  k_rows_lds<VT, D, BWD><<<(unsigned)A->lds_wgs, LDS_BLOCK, lds, ctx->stream>>>(
+      A->m, A->n, A->lds_plan, A->lds_off, A->lds_col16,
+      (const typename VT::T*)A->lds_val, x, out, ep, A->lds_map);
 }
 
 template <int BWD>
-static void rows_lds(epet_ctx* ctx, const epet_matrix* A, const float* x) {
+static void rows_lds(epet_ctx* ctx, const epet_matrix* A, const float* x, float* out,
+                     const LdsStore& ep) {
   switch (A->value_type) {
-    case EPET_VAL_F32: rows_lds_dispatch<ValF32, BWD>(ctx, A, x); break;
-    case EPET_VAL_BF16: rows_lds_dispatch<ValBF16, BWD>(ctx, A, x); break;
-    default: rows_lds_dispatch<ValF16, BWD>(ctx, A, x); break;
+    case EPET_VAL_F32: launch_rows_lds<ValF32, BWD>(ctx, A, x, out, ep); break;
+    case EPET_VAL_BF16: launch_rows_lds<ValBF16, BWD>(ctx, A, x, out, ep); break;
+    default: launch_rows_lds<ValF16, BWD>(ctx, A, x, out, ep); break;
   }
 }
 
@@ -369,7 +487,9 @@ static void lds_release(epet_matrix* A) {
   A->lds_val = nullptr;
   A->lds_col16 = nullptr;
   A->lds_partial = nullptr;
-  A->lds_T = 0;
+  if (A->lds_plan) (void)dev_free(A->lds_plan);
+  A->lds_plan = nullptr;
+  A->lds_T = A->lds_wgs = 0;
 }
 
 // Tile-major copy of A for column tiles of TV columns (a power of two up to
@@ -377,7 +497,7 @@ static void lds_release(epet_matrix* A) {
 // columns.  Allocates and synchronises.  On an allocation failure returns
 // EPET_OK with *off == nullptr.
 int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int* T_out,
-                     int64_t** off_out, void** val_out, uint16_t** col_out) {
+                     long long* entries_out, int64_t** off_out, void** val_out, uint16_t** col_out) {
   *off_out = nullptr;
   *val_out = nullptr;
   *col_out = nullptr;
@@ -427,16 +547,16 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
             dev_malloc((void**)&cnt, sizeof(int) * (size_t)std::max(1ll, nseg)) == hipSuccess &&
             dev_malloc((void**)&off, sizeof(int64_t) * (size_t)(nseg + 1)) == hipSuccess;
   int rc = EPET_OK;
+  long long tot = 0;
   if (ok) {
     launch_row_plan(st, A->m, T, TV, A->rowptr, scol, toff);
     k_lds_counts<<<grid_for(nseg, 256, 1ll << 31), 256, 0, st>>>(A->m, T, toff, cnt);
-    long long tot = 0;
     rc = exclusive_scan_i32_to_i64(ctx, cnt, off, nseg, &tot);
     if (rc == EPET_OK && (tot < A->nnz || tot > A->nnz + (long long)(LDS_CHUNK - 1) * nseg))
       rc = fail(EPET_ERR_STATE, __FILE__, __LINE__, "tile-major copy: entry count mismatch");
     ok = rc == EPET_OK &&
-         dev_malloc((void**)&val, vb * (size_t)std::max(1ll, tot)) == hipSuccess &&
-         dev_malloc((void**)&col16, sizeof(uint16_t) * (size_t)std::max(1ll, tot)) == hipSuccess;
+         dev_malloc((void**)&val, vb * (size_t)std::max<long long>(LDS_CHUNK, tot)) == hipSuccess &&
+         dev_malloc((void**)&col16, sizeof(uint16_t) * (size_t)std::max<long long>(LDS_CHUNK, tot)) == hipSuccess;
     if (rc == EPET_OK && !ok) (void)hipGetLastError();
     if (ok) {
       k_lds_set_last<<<1, 64, 0, st>>>(off, nseg, tot);
@@ -466,6 +586,7 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
     return rc;
   }
   *T_out = T;
+  *entries_out = tot;
   *off_out = off;
   *val_out = val;
   *col_out = col16;
@@ -496,12 +617,28 @@ int lds_prepare_map(epet_ctx* ctx, epet_matrix* A, bool voxel_columns) {
   if (A->lds_off || A->lds_failed || !lds_wanted(ctx, A)) return EPET_OK;
   int T = 0;
   const ColMap mp = voxel_columns ? voxel_map(ctx, A) : ColMap{};
-  EPET_TRY(build_tile_major(ctx, A, LDS_TILE, mp, &T, &A->lds_off, &A->lds_val, &A->lds_col16));
+  long long entries = 0;
+  EPET_TRY(build_tile_major(ctx, A, LDS_TILE, mp, &T, &entries, &A->lds_off, &A->lds_val, &A->lds_col16));
   A->lds_map = mp;
-  if (A->lds_off && dev_malloc((void**)&A->lds_partial, sizeof(float) * (size_t)A->m * T) ==
-                        hipSuccess) {
-    A->lds_T = T;
-    return EPET_OK;
+  if (A->lds_off) {
+    const long long cost = entries / LDS_CHUNK + (long long)LDS_ROW_COST * A->m * T;
+    const long long per_cu =
+        cost / ((long long)LDS_MIN_BLOCKS * WAVE * LDS_WAVES * ctx->num_cus) + 1;
+    // whole rounds of the CUs, the tiles' own rounding up included
+    const long long budget = std::min<long long>(LDS_PER_CU, per_cu) * ctx->num_cus;
+    const long long target = 1 + cost / (budget > 2 * T ? budget - T : budget);
+    const long long wgs = T + cost / target;
+    if (wgs < (1ll << 31) &&
+        dev_malloc((void**)&A->lds_plan, sizeof(int4) * LDS_WAVES * (size_t)wgs) == hipSuccess &&
+        dev_malloc((void**)&A->lds_partial, sizeof(float) * (size_t)A->m * T) == hipSuccess) {
+      k_lds_plan<<<grid_for(wgs * LDS_WAVES, 256, 1ll << 31), 256, 0, ctx->stream>>>(
+          A->m, T, target, wgs * LDS_WAVES, A->lds_off, A->lds_plan);
+      EPET_HIP(hipGetLastError());
+      EPET_HIP(hipStreamSynchronize(ctx->stream));
+      A->lds_T = T;
+      A->lds_wgs = (int)wgs;
+      return EPET_OK;
+    }
   }
   (void)hipGetLastError();
   lds_release(A);
@@ -519,10 +656,15 @@ bool lds_ready(const epet_ctx* ctx, const epet_matrix* A) {
 // bwd: A is a transposed copy)
 int lds_spmv(epet_ctx* ctx, const epet_matrix* A, const float* x, float alpha, float beta,
              float* y, bool use_scale, bool bwd) {
-  if (bwd) rows_lds<1>(ctx, A, x);
-  else rows_lds<0>(ctx, A, x);
-  k_lds_reduce<<<grid_for(A->m, 256, 1ll << 31), 256, 0, ctx->stream>>>(
-      A->m, A->lds_T, A->lds_partial, use_scale ? A->rowscale : nullptr, alpha, beta, y);
+  const float* scale = use_scale ? A->rowscale : nullptr;
+  const bool direct = A->lds_T == 1;
+  const LdsStore ep{direct ? 1 : 0, scale, alpha, beta};
+  float* out = direct ? y : A->lds_partial;
+  if (bwd) rows_lds<1>(ctx, A, x, out, ep);
+  else rows_lds<0>(ctx, A, x, out, ep);
+  if (!direct)
+    k_lds_reduce<<<grid_for(A->m, 256, 1ll << 31), 256, 0, ctx->stream>>>(
+        A->m, A->lds_T, A->lds_partial, scale, alpha, beta, y);
   EPET_HIP(hipGetLastError());
   return EPET_OK;
 }
@@ -530,7 +672,7 @@ int lds_spmv(epet_ctx* ctx, const epet_matrix* A, const float* x, float alpha, f
 // MLEM forward step (capturable once prepared)
 int lds_fwd_ratio(epet_ctx* ctx, const epet_matrix* A, const float* x, const float* y, float* e,
                   int fold, const int* itp, double* loglik) {
-  rows_lds<0>(ctx, A, x);
+  rows_lds<0>(ctx, A, x, A->lds_partial, LdsStore{});
   k_lds_ratio<<<grid_for(A->m, 256, 16ll * ctx->num_cus), 256, 0, ctx->stream>>>(
       A->m, A->lds_T, A->lds_partial, A->rowscale, y, e, fold, itp, loglik);
   EPET_HIP(hipGetLastError());

@@ -542,6 +542,7 @@ epet_matrix::~epet_matrix() {
   if (lds_off) (void)dev_free(lds_off);
   if (lds_val) (void)dev_free(lds_val);
   if (lds_col16) (void)dev_free(lds_col16);
+  if (lds_plan) (void)dev_free(lds_plan);
   if (lds_partial) (void)dev_free(lds_partial);
   epet::blk_release(this);
   epet::brk_release(this);
