@@ -840,7 +840,9 @@ static int brk_build(epet_ctx* ctx, const epet_matrix* M, const std::vector<int>
   B->m = M->m;
   B->G = (int)((rows.size() + BRK_ROWS - 1) / BRK_ROWS);
   B->mpos = B->G * BRK_ROWS;
-  B->noct = (int)((cols.size() + 7) / 8);
+  // whole groups of positions: the forward product writes the ratios of a whole
+  // row group into the other direction's gathered vector
+  B->noct = (int)((cols.size() + BRK_ROWS - 1) / BRK_ROWS) * (BRK_ROWS / 8);
   B->npos = B->noct * 8;
   B->parts = brk_parts(M->value_type);
   const int nwords = (B->noct + 31) / 32;
@@ -1024,6 +1026,8 @@ static int brk_product(epet_ctx* ctx, const BrkCopy* B, const BrkCopy* o, int Fp
   EPET_CHECK(splits <= 1 || (B->partial && B->partial_len >= (long long)splits * B->mpos * Fp),
              EPET_ERR_STATE, "bricks: partial buffer missing");
   EPET_CHECK(brk_vec(B, Fp) && brk_vec(o, Fp), EPET_ERR_STATE, "bricks: gathered vector missing");
+  EPET_CHECK(mode != 0 || o->npos >= B->mpos, EPET_ERR_STATE,
+             "bricks: the gathered vector is shorter than the row groups");
   BrkArgs a{};
   a.F = m.F;
   a.splits = splits;

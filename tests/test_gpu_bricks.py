@@ -207,3 +207,23 @@ def test_products_on_two_streams_and_in_a_graph(gpu_ctx_factory):
         g.replay()
         torch.cuda.synchronize()
         assert (y.double() - want[0]).norm() <= 1e-6 * want[0].norm()
+
+
+@pytest.mark.parametrize("rows", [449, 456, 480, 511, 512])
+@pytest.mark.parametrize("F", [8, 50])
+def test_rows_that_fill_no_group(gpu_ctx_factory, oracle, rows, F):
+    """Row counts that leave the last group of 64 partly empty: the ratios of the
+    whole group are written, so the vector that holds them covers it."""
+    from epetreco_amd.geometry import MeasurementSetup, VoxelGrid
+    s = MeasurementSetup(-0.23, 0.23, 32, 2, 2, 2, 2, 0.2, 0.02, 0.02, 0.02)
+    g = VoxelGrid(-0.08, -0.01, -0.01, 0.01, 0.01, 0.01, 16, 2, 2)
+    ctx = gpu_ctx_factory(setup=s, grid=g, nrays=256, seed=4)
+    A = ctx.sm_build(np.arange(rows, dtype=np.int32)).attach_transpose()
+    Y, sens, X0 = _data(A, F, 7)
+    X, _ = _run(ctx, A, Y, sens, X0, 3, False)
+    assert ctx.batched_config(A, F)["path"].startswith("bricks")
+    rp, col, val = decoded(A)
+    X64 = oracle.mlem_f64_frames(A.m, A.n, val, rp, col, Y.cpu().numpy(), sens.cpu().numpy(),
+                                 X0.cpu().numpy().astype(np.float64), 3)
+    for f in range(F):
+        assert _rel(X[:, f], X64[:, f]) < 1e-5
