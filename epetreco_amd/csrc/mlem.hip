@@ -1,15 +1,20 @@
 // mlem.hip -- mlemOperations drop-ins and the fused MLEM iteration.
 //
-// One MLEM iteration (tests/reco.cu:209-300) is four launches on the context's
+// One MLEM iteration (tests/reco.cu:209-300) is a few launches on the context's
 // stream, replayable as one hipGraph (no memset nodes; every clear is a
 // kernel):
 //   1. k_fwd_ratio : yhat_i = sum_k a_ik x_k, e_i = y_i / yhat_i (0 where
 //                    yhat_i = 0), FP64 log-likelihood sum y log yhat - yhat
-//   2. back projection c += A^T e (spmv.hip kernels)
-//   3. k_update    : x_j <- x_j c_j / (s_j + [s_j == 0]), FP64 sum of x
-//   4. k_normalise : x_j <- x_j / sum x, c <- 0, next sum slot <- 0, it++
-// Device state (iteration counter, sums, log-likelihoods, frame flags) lives in
-// one small buffer so that the same graph serves every iteration.
+//   2. back projection c = A^T e (spmv.hip kernels)
+//   3. k_update    : x_j <- x_j c_j / (s_j + [s_j == 0]), FP64 sum of x, it++
+//   4. k_normalise : x_j <- x_j / sum x, next sum slot <- 0
+// (3 and 4 are one launch for small images, k_update_one).  Device state
+// (iteration counters, sums, log-likelihoods, frame flags) lives in one small
+// buffer so that the same graph serves every iteration.
+//
+// FP64 sums over a whole vector end in one atomic per workgroup on one address,
+// which the card takes one by one, 12 ns each: the kernels that end so run few
+// workgroups of 1024 threads (REDUCE_BLOCK).
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -93,6 +98,12 @@ __global__ __launch_bounds__(256) void k_scales(float* __restrict__ x, float alp
   if (i < n) x[i] = alpha * x[i];
 }
 
+constexpr int REDUCE_BLOCK = 1024;
+// workgroups of REDUCE_BLOCK threads for n elements: at most one per CU
+static unsigned reduce_grid(const epet_ctx* ctx, long long n) {
+  return grid_for(n, REDUCE_BLOCK, ctx->num_cus);
+}
+
 __device__ __forceinline__ double block_sum_f64(double v, double* s_w) {
   v = wave_sum(v);
   if (lane_id() == 0) s_w[wave_id()] = v;
@@ -103,9 +114,11 @@ __device__ __forceinline__ double block_sum_f64(double v, double* s_w) {
   return t;   // valid in thread 0
 }
 
-__global__ __launch_bounds__(256) void k_sum_f64(const float* __restrict__ x, long long n,
-                                                 double* __restrict__ out) {
-  __shared__ double s_w[256 / WAVE];
+// (with 256 threads and up to 2048 workgroups 28 us at 104^3 and 9 us at 52^3,
+// now 6 and 4)
+__global__ __launch_bounds__(REDUCE_BLOCK) void k_sum_f64(const float* __restrict__ x, long long n,
+                                                          double* __restrict__ out) {
+  __shared__ double s_w[REDUCE_BLOCK / WAVE];
   double acc = 0.0;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x)
@@ -135,7 +148,7 @@ struct MlemState {
 // scale, for a back projection through the transposed copy (which stores the
 // unscaled values).
 template <typename VT, int L>
-__global__ __launch_bounds__(256) void k_fwd_ratio(int m, const int64_t* __restrict__ rowptr,
+__global__ __launch_bounds__(REDUCE_BLOCK) void k_fwd_ratio(int m, const int64_t* __restrict__ rowptr,
                                                    const int* __restrict__ col,
                                                    const typename VT::T* __restrict__ val,
                                                    const float* __restrict__ rowscale,
@@ -144,11 +157,11 @@ __global__ __launch_bounds__(256) void k_fwd_ratio(int m, const int64_t* __restr
                                                    float* __restrict__ e, int fold,
                                                    const int* __restrict__ itp,
                                                    double* __restrict__ loglik) {
-  __shared__ double s_w[256 / WAVE];
+  __shared__ double s_w[REDUCE_BLOCK / WAVE];
   const int sub = threadIdx.x % L;
-  const long long stride = (long long)gridDim.x * (256 / L);
+  const long long stride = (long long)gridDim.x * (REDUCE_BLOCK / L);
   double ll = 0.0;
-  for (long long r = (long long)blockIdx.x * (256 / L) + threadIdx.x / L; r < m; r += stride) {
+  for (long long r = (long long)blockIdx.x * (REDUCE_BLOCK / L) + threadIdx.x / L; r < m; r += stride) {
     const long long b = rowptr[r], end = rowptr[r + 1];
     float a0 = 0.0f, a1 = 0.0f;
     long long k = b + sub;
@@ -175,7 +188,7 @@ __global__ __launch_bounds__(256) void k_fwd_ratio(int m, const int64_t* __restr
 
 // Single frame, long rows: one wavefront per row with vector loads.
 template <typename VT>
-__global__ __launch_bounds__(256) void k_fwd_ratio_vec(int m, const int64_t* __restrict__ rowptr,
+__global__ __launch_bounds__(REDUCE_BLOCK) void k_fwd_ratio_vec(int m, const int64_t* __restrict__ rowptr,
                                                        const int* __restrict__ col,
                                                        const typename VT::T* __restrict__ val,
                                                        const float* __restrict__ rowscale,
@@ -184,12 +197,12 @@ __global__ __launch_bounds__(256) void k_fwd_ratio_vec(int m, const int64_t* __r
                                                        float* __restrict__ e, int fold,
                                                        const int* __restrict__ itp,
                                                        double* __restrict__ loglik) {
-  __shared__ double s_w[256 / WAVE];
+  __shared__ double s_w[REDUCE_BLOCK / WAVE];
   const int lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane(wave_id());
-  const long long nw = (long long)gridDim.x * (256 / WAVE);
+  const long long nw = (long long)gridDim.x * (REDUCE_BLOCK / WAVE);
   double ll = 0.0;
-  long long r = (long long)blockIdx.x * (256 / WAVE) + wv;
+  long long r = (long long)blockIdx.x * (REDUCE_BLOCK / WAVE) + wv;
   long long pb = r < m ? row_bounds_load(rowptr, r, lane) : 0;
   for (; r < m; r += nw) {
     const long long b = lane_value_i64(pb, 0), end = lane_value_i64(pb, 1);
@@ -242,58 +255,145 @@ __global__ __launch_bounds__(256) void k_fwd_ratio_mf(int m, int F,
   }
 }
 
+// Every thread stays on one frame: a workgroup's first (REDUCE_BLOCK / F) F
+// threads take elements f, f + F, .. of the frame-minor arrays, stepping by a
+// multiple of F, so that a sum is kept in a register (an LDS atomic per element
+// and a 64-bit remainder took 45 us for 32 frames of 52^3, now 22).
+struct FrameStep {
+  int f, width;          // own frame; threads in use
+  long long i, step;     // first element, stride
+  long long j, jstep;    // their voxels
+  __device__ __forceinline__ FrameStep(int F) {
+    width = REDUCE_BLOCK / F * F;
+    f = threadIdx.x % F;
+    i = (long long)blockIdx.x * width + threadIdx.x;
+    step = (long long)gridDim.x * width;
+    j = (long long)blockIdx.x * (width / F) + threadIdx.x / F;
+    jstep = step / F;
+  }
+};
+
+__device__ __forceinline__ float mlem_factor(float x, float c, float s) {
+  s += (float)(s == 0.0f);   // mlemOperations.hpp:48-50
+  return x * c / s;
+}
+
+// Workgroup sums of v per frame in s_sum[F] (zero on entry; barriers inside)
+__device__ __forceinline__ void frame_sums(double v, int F, const FrameStep& q, double* s_sum) {
+  if (F == 1) {
+    v = wave_sum(v);
+    if (lane_id() == 0) atomicAdd(&s_sum[0], v);
+  } else if ((int)threadIdx.x < q.width) {
+    atomicAdd(&s_sum[q.f], v);
+  }
+  __syncthreads();
+}
+
+// The counters are two, so that no launch only counts: itp[0] is read by the
+// forward step and k_normalise and advanced by k_update, itp[1] is read by
+// k_update and advanced by k_normalise.
+
 // x <- x c / (s + [s==0]) for active frames, FP64 sum per frame into slot it&1
-// (grid-stride; per-frame partial sums in LDS, one global atomic per
-// workgroup and frame)
-__global__ __launch_bounds__(256) void k_update(float* __restrict__ x, const float* __restrict__ c,
-                                                const float* __restrict__ s, long long n, int F,
-                                                const int* __restrict__ itp,
-                                                double* __restrict__ sum,
-                                                const int* __restrict__ active) {
+// (one global atomic per workgroup and frame)
+__global__ __launch_bounds__(REDUCE_BLOCK) void k_update(float* __restrict__ x,
+                                                         const float* __restrict__ c,
+                                                         const float* __restrict__ s, long long n,
+                                                         int F, int* __restrict__ itp,
+                                                         double* __restrict__ sum,
+                                                         const int* __restrict__ active) {
   __shared__ double s_sum[64];
   if (threadIdx.x < 64) s_sum[threadIdx.x] = 0.0;
   __syncthreads();
-  const int slot = (*itp) & 1;
-  const long long tot = n * F;
-  double v1 = 0.0;   // single-frame running sum
-  for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < tot;
-       idx += (long long)gridDim.x * blockDim.x) {
-    const long long j = (F == 1) ? idx : idx / F;
-    const int f = (F == 1) ? 0 : (int)(idx % F);
-    float dvs = s[j];
-    dvs += (float)(dvs == 0.0f);   // mlemOperations.hpp:48-50
-    float xn = x[idx];
-    if (!active || active[f]) { xn = xn * c[idx] / dvs; x[idx] = xn; }
-    if (F == 1) v1 += xn;
-    else atomicAdd(&s_sum[f], (double)xn);
-  }
-  if (F == 1) {
-    v1 = wave_sum(v1);
-    if (lane_id() == 0) atomicAdd(&s_sum[0], v1);
-  }
-  __syncthreads();
-  if (threadIdx.x < F) unsafeAtomicAdd(&sum[slot * F + threadIdx.x], s_sum[threadIdx.x]);
-}
-
-__global__ __launch_bounds__(256) void k_normalise(float* __restrict__ x, float* __restrict__ c,
-                                                   long long n, int F, const int* __restrict__ itp,
-                                                   double* __restrict__ sum,
-                                                   const int* __restrict__ active) {
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int slot = (*itp) & 1;
-  if (idx < n * (long long)F) {
-    const int f = (F == 1) ? 0 : (int)(idx % F);
-    if (!active || active[f]) {
-      const double S = sum[slot * F + f];
-      x[idx] = x[idx] * (float)(1.0 / S);   // reco.cu:280-281
+  const int slot = itp[1] & 1;
+  const FrameStep q(F);
+  double v = 0.0;
+  if ((int)threadIdx.x < q.width) {
+    const bool act = !active || active[q.f];
+#pragma unroll 4
+    for (long long i = q.i, j = q.j; j < n; i += q.step, j += q.jstep) {
+      float xn = x[i];
+      if (act) {
+        xn = mlem_factor(xn, c[i], s[j]);
+        x[i] = xn;
+      }
+      v += xn;
     }
-    c[idx] = 0.0f;
   }
-  if (idx < F) sum[(slot ^ 1) * F + idx] = 0.0;
+  frame_sums(v, F, q, s_sum);
+  if ((int)threadIdx.x < F) unsafeAtomicAdd(&sum[slot * F + threadIdx.x], s_sum[threadIdx.x]);
+  if (blockIdx.x == 0 && threadIdx.x == 0) itp[0] += 1;
 }
 
-__global__ void k_advance(int* itp) {
-  if (threadIdx.x == 0) *itp += 1;
+// c <- 0 where the next back projection adds to it (c not null)
+__global__ __launch_bounds__(REDUCE_BLOCK) void k_normalise(float* __restrict__ x,
+                                                            float* __restrict__ c, long long n,
+                                                            int F, int* __restrict__ itp,
+                                                            double* __restrict__ sum,
+                                                            const int* __restrict__ active) {
+  const int slot = (itp[0] - 1) & 1;
+  const FrameStep q(F);
+  if ((int)threadIdx.x < q.width) {
+    const bool act = !active || active[q.f];
+    const float r = (float)(1.0 / sum[slot * F + q.f]);   // reco.cu:280-281
+#pragma unroll 4
+    for (long long i = q.i, j = q.j; j < n; i += q.step, j += q.jstep) {
+      if (act) x[i] *= r;
+      if (c) c[i] = 0.0f;
+    }
+  }
+  if (blockIdx.x == 0) {
+    if ((int)threadIdx.x < F) sum[(slot ^ 1) * F + threadIdx.x] = 0.0;
+    if (threadIdx.x == 0) itp[1] += 1;
+  }
+}
+
+// Both by one workgroup, for images of up to UPDATE_ONE elements: no atomics on
+// memory and one launch less (4,096 voxels: 5.5 us against 5.6 us and a launch, and
+// its time grows with the image: 16 elements a thread at the limit).
+constexpr long long UPDATE_ONE = 16384;
+__global__ __launch_bounds__(REDUCE_BLOCK) void k_update_one(float* __restrict__ x,
+                                                             float* __restrict__ c,
+                                                             const float* __restrict__ s,
+                                                             long long n, int F, bool clear,
+                                                             int* __restrict__ itp,
+                                                             const int* __restrict__ active) {
+  __shared__ double s_sum[64];
+  if (threadIdx.x < 64) s_sum[threadIdx.x] = 0.0;
+  __syncthreads();
+  const FrameStep q(F);
+  const bool mine = (int)threadIdx.x < q.width;
+  const bool act = mine && (!active || active[q.f]);
+  double v = 0.0;
+  if (mine)
+#pragma unroll 4
+    for (long long i = q.i, j = q.j; j < n; i += q.step, j += q.jstep) {
+      float xn = x[i];
+      if (act) {
+        xn = mlem_factor(xn, c[i], s[j]);
+        x[i] = xn;
+      }
+      if (clear) c[i] = 0.0f;
+      v += xn;
+    }
+  frame_sums(v, F, q, s_sum);
+  if (act) {
+    const float r = (float)(1.0 / s_sum[q.f]);   // reco.cu:280-281
+#pragma unroll 4
+    for (long long i = q.i, j = q.j; j < n; i += q.step, j += q.jstep) x[i] *= r;
+  }
+  if (threadIdx.x == 0) itp[0] += 1;
+}
+
+// The state of a run before its first iteration: doubles and image 0, counters 0,
+// frames active.
+__global__ __launch_bounds__(256) void k_mlem_init(double* __restrict__ d, long long nd,
+                                                   int* __restrict__ itp, int F,
+                                                   float* __restrict__ c, long long nv) {
+  const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long step = (long long)gridDim.x * blockDim.x;
+  for (long long i = i0; i < nd; i += step) d[i] = 0.0;
+  for (long long i = i0; i < nv; i += step) c[i] = 0.0f;
+  if (i0 < 2 + F) itp[i0] = i0 < 2 ? 0 : 1;
 }
 
 __global__ void k_fill_i32_one(int* p, int v) {
@@ -321,16 +421,17 @@ static int launch_fwd_ratio(hipStream_t st, int ncu, const epet_matrix* A, int F
   if (m == 0) return EPET_OK;
   if (F == 1) {
     const int L = A->lanes_fwd > 0 ? A->lanes_fwd : pick_lanes(A->nnz, m);
-    const long long cap = 16ll * ncu;
+    // two workgroups fill a CU
+    const long long rows = REDUCE_BLOCK / L, g = std::min<long long>((m + rows - 1) / rows, 2ll * ncu);
     if (L == 64 && A->lanes_fwd == 0) {
-      k_fwd_ratio_vec<VT><<<(unsigned)std::min<long long>((m + 3) / 4, cap), 256, 0, st>>>(
+      k_fwd_ratio_vec<VT><<<(unsigned)g, REDUCE_BLOCK, 0, st>>>(
           m, A->rowptr, A->col, v, A->rowscale, x, y, e, fold, itp, loglik);
       EPET_HIP(hipGetLastError());
       return EPET_OK;
     }
 #define EPET_FR(LL)                                                                         \
-  k_fwd_ratio<VT, LL><<<(unsigned)std::min<long long>(((long long)m + 256 / LL - 1) / (256 / LL), cap), \
-                        256, 0, st>>>(m, A->rowptr, A->col, v, A->rowscale, x, y, e, fold, itp, loglik)
+  k_fwd_ratio<VT, LL><<<(unsigned)g, REDUCE_BLOCK, 0, st>>>(m, A->rowptr, A->col, v, A->rowscale, \
+                                                            x, y, e, fold, itp, loglik)
     switch (L) {
       case 64: EPET_FR(64); break;
       case 32: EPET_FR(32); break;
@@ -364,6 +465,7 @@ static int mlem_iteration(epet_ctx* ctx, const epet_matrix* A, int F, const floa
                           double* loglik, const int* active, bool prepared_only = false) {
   hipStream_t st = ctx->stream;
   int rc;
+  bool adds = false;   // whether the back projection adds to c
   if (F > 1 && A->tr) {
     const MfArgs a{F, x, y, e, c, itp, loglik};
     rc = use_brk(ctx, A, F)   ? brk_iteration(ctx, A, a)
@@ -381,6 +483,7 @@ static int mlem_iteration(epet_ctx* ctx, const epet_matrix* A, int F, const floa
       default: rc = launch_fwd_ratio<ValF16>(st, ctx->num_cus, A, F, x, y, e, fold, itp, loglik); break;
     }
     if (rc != EPET_OK) return rc;
+    adds = !via_tr;
     if (via_tr) rc = matrix_bp_transpose(ctx, A->tr, 1.0f, e, 0.0f, c);
     else if (F == 1 && prepared_only) rc = matrix_spmv_t_prepared(ctx, A, 1.0f, e, 1.0f, c);
     else if (F == 1) rc = matrix_spmv(ctx, A, EPET_OP_T, 1.0f, e, 1.0f, c);
@@ -388,12 +491,31 @@ static int mlem_iteration(epet_ctx* ctx, const epet_matrix* A, int F, const floa
   }
   if (rc != EPET_OK) return rc;
   const long long nv = (long long)A->n * F;
-  k_update<<<grid_for(nv, 256, 4ll * ctx->num_cus), 256, 0, st>>>(x, c, s, A->n, F, itp, sum, active);
-  k_normalise<<<grid_for(std::max<long long>(nv, F), 256, 1ll << 31), 256, 0, st>>>(x, c, A->n, F,
-                                                                                   itp, sum, active);
-  k_advance<<<1, 64, 0, st>>>(itp);
+  if (nv <= UPDATE_ONE) {
+    k_update_one<<<1, REDUCE_BLOCK, 0, st>>>(x, c, s, A->n, F, adds, itp, active);
+  } else {
+    // one, two and four workgroups per CU: 34, 25 and 28 us at 8 frames of 104^3
+    const unsigned g = grid_for(nv, REDUCE_BLOCK, 2ll * ctx->num_cus);
+    k_update<<<g, REDUCE_BLOCK, 0, st>>>(x, c, s, A->n, F, itp, sum, active);
+    k_normalise<<<g, REDUCE_BLOCK, 0, st>>>(x, adds ? c : nullptr, A->n, F, itp, sum, active);
+  }
   EPET_HIP(hipGetLastError());
   return EPET_OK;
+}
+
+// Working arrays of a run: state and c cleared, s <- s_in / sum(s_in)
+// (reco.cu:182-183).  d[0] is the sum of s_in.
+static hipError_t mlem_start(epet_ctx* ctx, int n, int F, const float* s_in, double* d, long long nd,
+                             int* itp, float* c, float* s) {
+  hipStream_t st = ctx->stream;
+  const long long nv = (long long)n * F;
+  k_mlem_init<<<grid_for(std::max(nv, nd), 256, 16ll * ctx->num_cus), 256, 0, st>>>(d, nd, itp, F,
+                                                                                     c, nv);
+  if (n > 0) {
+    k_sum_f64<<<reduce_grid(ctx, n), REDUCE_BLOCK, 0, st>>>(s_in, n, d);
+    k_scale_by_sum<<<grid_for(n, 256, 1ll << 31), 256, 0, st>>>(s, s_in, n, d);
+  }
+  return hipGetLastError();
 }
 
 // ------------------------------------------------------ allocation-free MLEM
@@ -482,7 +604,7 @@ int epet_sum(epet_ctx* ctx, const float* x, long long n, double* out) {
   double* d = nullptr;
   EPET_HIP(tmp.alloc(&d, sizeof(double)));
   k_zero_f64<<<1, 64, 0, ctx->stream>>>(d, 1);
-  if (n > 0) k_sum_f64<<<grid_for(n, 256, 2048), 256, 0, ctx->stream>>>(x, n, d);
+  if (n > 0) k_sum_f64<<<reduce_grid(ctx, n), REDUCE_BLOCK, 0, ctx->stream>>>(x, n, d);
   EPET_HIP(hipGetLastError());
   return read_pinned(ctx, out, d, sizeof(double));
 }
@@ -503,18 +625,16 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
     ctx->stream = own;
   }
   hipStream_t st = ctx->stream;
-  // buffers: e (m F), c (n F), s (n), state
-  float *e = nullptr, *c = nullptr, *s = nullptr;
-  int* ibuf = nullptr;      // [it, active[F]]
-  double* dbuf = nullptr;   // [ssum, sum[2F], loglik[niter F]]
+  // one block: e (m F), c (n F), s (n), doubles [ssum, sum[2F], loglik[niter F]],
+  // ints [it, it of the update, active[F]]
   const size_t nd = 1 + 2 * (size_t)F + (size_t)std::max(1, niter) * F;
+  const size_t e_b = align256(sizeof(float) * (size_t)A->m * F);
+  const size_t c_b = align256(sizeof(float) * (size_t)nv), s_b = align256(sizeof(float) * (size_t)A->n);
+  const size_t d_b = align256(sizeof(double) * nd), i_b = align256(sizeof(int) * (2 + F));
+  unsigned char* block = nullptr;
   int rc = EPET_OK;
   auto cleanup = [&]() {
-    if (e) (void)hipFreeAsync(e, st);
-    if (c) (void)hipFreeAsync(c, st);
-    if (s) (void)hipFreeAsync(s, st);
-    if (ibuf) (void)hipFreeAsync(ibuf, st);
-    if (dbuf) (void)hipFreeAsync(dbuf, st);
+    if (block) (void)hipFreeAsync(block, st);
     (void)hipStreamSynchronize(st);
     if (own) { (void)hipStreamDestroy(own); ctx->stream = saved; }
   };
@@ -527,26 +647,17 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
       return rc;                                                                         \
     }                                                                                    \
   } while (0)
-  EPET_MLEM_HIP(tmp_malloc((void**)&e, sizeof(float) * std::max<long long>(1, (long long)A->m * F), st));
-  EPET_MLEM_HIP(tmp_malloc((void**)&c, sizeof(float) * std::max<long long>(1, nv), st));
-  EPET_MLEM_HIP(tmp_malloc((void**)&s, sizeof(float) * std::max(1, A->n), st));
-  EPET_MLEM_HIP(tmp_malloc((void**)&ibuf, sizeof(int) * (1 + F), st));
-  EPET_MLEM_HIP(tmp_malloc((void**)&dbuf, sizeof(double) * nd, st));
-  int* itp = ibuf;
-  int* active = ibuf + 1;
+  EPET_MLEM_HIP(tmp_malloc((void**)&block, e_b + c_b + s_b + d_b + i_b, st));
+  float* e = (float*)block;
+  float* c = (float*)(block + e_b);
+  float* s = (float*)(block + e_b + c_b);
+  double* dbuf = (double*)(block + e_b + c_b + s_b);
+  int* itp = (int*)(block + e_b + c_b + s_b + d_b);
+  int* active = itp + 2;
   double* ssum = dbuf;
   double* sum = dbuf + 1;
   double* ll = dbuf + 1 + 2 * F;
-  k_zero_f64<<<grid_for((long long)nd, 256), 256, 0, st>>>(dbuf, (int)nd);
-  k_fill_f32<<<grid_for(nv, 256, 1ll << 31), 256, 0, st>>>(c, nv, 0.0f);
-  std::vector<int> hi(1 + F, 1);
-  hi[0] = 0;
-  EPET_MLEM_HIP(hipMemcpyAsync(ibuf, hi.data(), sizeof(int) * (1 + F), hipMemcpyHostToDevice, st));
-  // s <- s / sum(s)  (reco.cu:182-183)
-  k_sum_f64<<<grid_for(A->n, 256, 2048), 256, 0, st>>>(s_in, A->n, ssum);
-  k_scale_by_sum<<<grid_for(A->n, 256, 1ll << 31), 256, 0, st>>>(s, s_in, A->n, ssum);
-  EPET_MLEM_HIP(hipGetLastError());
-  EPET_MLEM_HIP(hipStreamSynchronize(st));
+  EPET_MLEM_HIP(mlem_start(ctx, A->n, F, s_in, dbuf, (long long)nd, itp, c, s));
 
   // back-projection plan (allocates) and multi-frame tuning before any capture
   if (F == 1) {
@@ -578,7 +689,6 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
     rc = mf_tune(ctx, const_cast<epet_matrix*>(A), a, 2);
     if (rc != EPET_OK) { cleanup(); return rc; }
   }
-  k_fill_f32<<<grid_for(nv, 256, 1ll << 31), 256, 0, st>>>(c, nv, 0.0f);
   const bool stopping = tol > 0.0 && frame_iters != nullptr;
   std::vector<int> act(F, 1), iters(F, 0);
   std::vector<double> hll((size_t)std::max(1, niter) * F, 0.0);
@@ -666,18 +776,8 @@ int epet_mlem_noalloc(epet_ctx* ctx, const epet_matrix* A, const float* y, const
   float* e = (float*)(base + L.e);
   float* c = (float*)(base + L.c);
   float* s = (float*)(base + L.s);
-  const int n = A->n;
-  // the array keeps the previous call's contents: clear with kernels
-  const int nd = 3 + std::max(1, niter);
-  k_zero_f64<<<grid_for(nd, 256), 256, 0, st>>>(dbuf, nd);
-  k_fill_i32_one<<<1, 64, 0, st>>>(itp, 0);
-  k_fill_f32<<<grid_for(std::max(1, n), 256, 1ll << 31), 256, 0, st>>>(c, n, 0.0f);
-  // s <- s / sum(s)  (reco.cu:182-183)
-  if (n > 0) {
-    k_sum_f64<<<grid_for(n, 256, 2048), 256, 0, st>>>(s_in, n, ssum);
-    k_scale_by_sum<<<grid_for(n, 256, 1ll << 31), 256, 0, st>>>(s, s_in, n, ssum);
-  }
-  EPET_HIP(hipGetLastError());
+  // the array keeps the previous call's contents: cleared by the start's kernels
+  EPET_HIP(mlem_start(ctx, A->n, 1, s_in, dbuf, 3 + std::max(1, niter), itp, c, s));
   for (int it = 0; it < niter; it++)
     EPET_TRY(mlem_iteration(ctx, A, 1, y, s, x, e, c, itp, sum, ll, nullptr, true));
   if (loglik_out && niter > 0) {
