@@ -1,8 +1,7 @@
 // mlem.hip -- mlemOperations drop-ins and the fused MLEM iteration.
 //
 // One MLEM iteration (tests/reco.cu:209-300) is a few launches on the context's
-// stream, replayable as one hipGraph (no memset nodes; every clear is a
-// kernel):
+// stream:
 //   1. k_fwd_ratio : yhat_i = sum_k a_ik x_k, e_i = y_i / yhat_i (0 where
 //                    yhat_i = 0), FP64 log-likelihood sum y log yhat - yhat
 //   2. back projection c = A^T e (spmv.hip kernels)
@@ -10,7 +9,7 @@
 //   4. k_normalise : x_j <- x_j / sum x, next sum slot <- 0
 // (3 and 4 are one launch for small images, k_update_one).  Device state
 // (iteration counters, sums, log-likelihoods, frame flags) lives in one small
-// buffer so that the same graph serves every iteration.
+// buffer, so that the host waits for nothing between iterations.
 //
 // FP64 sums over a whole vector end in one atomic per workgroup on one address,
 // which the card takes one by one, 12 ns each: the kernels that end so run few
@@ -457,7 +456,7 @@ static int launch_fwd_ratio(hipStream_t st, int ncu, const epet_matrix* A, int F
   return EPET_OK;
 }
 
-// One MLEM iteration on `st` (capturable).  prepared_only: the single-frame
+// One MLEM iteration on the context's stream.  prepared_only: the single-frame
 // back projection uses the plan A already holds and builds none (no
 // allocation).
 static int mlem_iteration(epet_ctx* ctx, const epet_matrix* A, int F, const float* y,
@@ -616,14 +615,13 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
   EPET_CHECK(F >= 1 && F <= 64, EPET_ERR_UNSUPPORTED, "frames must be in [1, 64]");
   EPET_CHECK(niter >= 0, EPET_ERR_ARG, "negative iteration count");
   const long long nv = (long long)A->n * F;
-  hipStream_t own = nullptr;
-  hipStream_t saved = ctx->stream;
-  if (use_graph && ctx->stream == nullptr) {
-    // capture needs a non-null stream; order it after the caller's null-stream work
-    EPET_HIP(hipStreamSynchronize(nullptr));
-    EPET_HIP(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
-    ctx->stream = own;
-  }
+  // The iterations are launched directly, use_graph or not: an iteration is 3 to 7
+  // launches of 5 us and more each, which the host keeps ahead of.  Replaying a
+  // captured iteration took 60 us more a call (capture, instantiation, a stream of
+  // its own) and 5 to 9 us more an iteration (9,000 rows, 16^3, 1 and 5 frames, 10
+  // iterations: 401 against 271 us and 673 against 528; 50: 1441 against 1090 and
+  // 2766 against 2381; 150,000 rows, 52^3, 13 frames, 3: 1955 against 1859).
+  (void)use_graph;
   hipStream_t st = ctx->stream;
   // one block: e (m F), c (n F), s (n), doubles [ssum, sum[2F], loglik[niter F]],
   // ints [it, it of the update, active[F]]
@@ -636,7 +634,6 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
   auto cleanup = [&]() {
     if (block) (void)hipFreeAsync(block, st);
     (void)hipStreamSynchronize(st);
-    if (own) { (void)hipStreamDestroy(own); ctx->stream = saved; }
   };
 #define EPET_MLEM_HIP(call)                                                              \
   do {                                                                                   \
@@ -659,7 +656,7 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
   double* ll = dbuf + 1 + 2 * F;
   EPET_MLEM_HIP(mlem_start(ctx, A->n, F, s_in, dbuf, (long long)nd, itp, c, s));
 
-  // back-projection plan (allocates) and multi-frame tuning before any capture
+  // back-projection plan (allocates) and multi-frame tuning
   if (F == 1) {
     rc = lds_prepare_map(ctx, const_cast<epet_matrix*>(A), true);
     if (rc == EPET_OK && bp_use_transpose(ctx, A)) rc = lds_prepare(ctx, A->tr);
@@ -692,24 +689,9 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
   const bool stopping = tol > 0.0 && frame_iters != nullptr;
   std::vector<int> act(F, 1), iters(F, 0);
   std::vector<double> hll((size_t)std::max(1, niter) * F, 0.0);
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  if (use_graph && niter > 0) {
-    EPET_MLEM_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    rc = mlem_iteration(ctx, A, F, y, s, x, e, c, itp, sum, ll, active);
-    hipError_t ce = hipStreamEndCapture(st, &graph);
-    if (rc != EPET_OK) { cleanup(); return rc; }
-    EPET_MLEM_HIP(ce);
-    EPET_MLEM_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-  }
   for (int it = 0; it < niter; it++) {
-    if (exec) {
-      hipError_t ge = hipGraphLaunch(exec, st);
-      if (ge != hipSuccess) { rc = fail(EPET_ERR_HIP, __FILE__, __LINE__, "hipGraphLaunch"); break; }
-    } else {
-      rc = mlem_iteration(ctx, A, F, y, s, x, e, c, itp, sum, ll, active);
-      if (rc != EPET_OK) break;
-    }
+    rc = mlem_iteration(ctx, A, F, y, s, x, e, c, itp, sum, ll, active);
+    if (rc != EPET_OK) break;
     if (stopping) {
       // per-frame stop on the relative log-likelihood change
       if (hipMemcpyAsync(hll.data() + (size_t)it * F, ll + (size_t)it * F, sizeof(double) * F,
@@ -738,8 +720,6 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
       if (!any) break;
     }
   }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
   if (rc == EPET_OK && loglik_out && niter > 0) {
     if (hipMemcpyAsync(loglik_out, ll, sizeof(double) * (size_t)niter * F, hipMemcpyDeviceToHost,
                        st) != hipSuccess ||
