@@ -19,6 +19,7 @@ constexpr int GEN_BLOCK = 256;
 constexpr int MAX_SLABS = 512;        // x planes of the traversal path
 constexpr int BITMAP_WORDS = 4096;    // 131072 voxel bits per row in LDS
 constexpr float MARK_EPS = 2e-3f;     // traversal margin, in voxel widths
+constexpr float WIN_EPS = 4e-3f;      // of windows from rounder sums
 constexpr float REJECT_MARGIN2 = 1.0404f;  // (1.02)^2 on the voxel half diagonal
 
 // ------------------------------------------------------------------ rays
@@ -363,17 +364,21 @@ __global__ __launch_bounds__(GEN_BLOCK) void k_sm_rows(Geo g, const int* __restr
 // so that cell order is voxel order) and walks the rays one after the other,
 // one lane per plane of the axis the rays run along (x or z): the lane adds the
 // ray's exact length to the few voxels of its plane that the ray's rectangle
-// (MARK_EPS wider) holds.  Planes are disjoint, so no two lanes add to one
+// (MARK_EPS wider) holds, from the corner where the ray comes in, stepping over
+// whichever face it leaves by: the intervals between faces are met in order, so
+// no voxel with a length is passed over.  Planes are disjoint, so no two lanes add to one
 // voxel, and a wavefront's LDS operations keep their order, so every sum is the
 // reference's.  A plane parameter (box face - start) / direction depends only
 // on (ray, axis, plane): one table per ray in LDS replaces six correctly
 // rounded divisions per (voxel, ray).  Adding a ray that does not cross a voxel
 // adds exactly 0, so leaving it out keeps the sum.
 //
-// Bound by the chain of LDS reads and VALU work of one ray after the other.
-// Channels of 916 entries (52^3, 64 rays): 40,000 took 7.86 ms in k_sm_rows and
-// take 2.12 ms here, 100,000 18.6 and 5.2 ms; 11,250 of 57 entries (16^3, 8 rays)
-// 275 and 59 us.
+// Bound by VALU work (68% busy) and, at 10 workgroups per CU by their LDS, the chain
+// of LDS reads of one ray after the other.  Channels of 916 entries (52^3, 64 rays):
+// 40,000 took 7.86 ms in k_sm_rows, 100,000 18.6; walked with divisions and every
+// voxel of the rectangles tried 2.11 and 5.1 ms; now 1.49 and 4.0 ms (divisions 0.3,
+// steps 0.15, windows from sums 0.15 of the 0.62 ms).  11,250 of 57 entries (16^3, 8
+// rays): 275, 59, 48 us.
 //
 // A ray parallel to an axis meets every voxel of that axis (the reference
 // ignores the axis then), so its windows span it.  Rows it does not take are
@@ -385,6 +390,27 @@ struct WalkWin {      // window of an x-plane
   int wz;             // cells per y line (0: no cells)
   int y, z;           // low | high << 16, inclusive
 };
+
+// n / d, correctly rounded, from y = 1 / d correctly rounded: two corrections by the
+// exact remainder (Markstein, IBM J. Res. Dev. 34, 1990), half the instructions of
+// a division.  For d and n in walk_plain's range.
+__device__ __forceinline__ float walk_quot(float n, float d, float y) {
+  float q = n * y;
+  q = __builtin_fmaf(__builtin_fmaf(-q, d, n), y, q);
+  return __builtin_fmaf(__builtin_fmaf(-q, d, n), y, q);
+}
+// Whether quotients (a - p) / d over a grid's faces a keep clear of overflow and
+// of remainders that are not exact: origin, edges and p are 0 or at least 2^-60, so
+// that a - p is a multiple of 2^-83, and all are at most 2^30 (2^31 a whole grid).
+__device__ __forceinline__ bool walk_plain(float v, bool zero_too) {
+  const float a = fabsf(v);
+  return (zero_too && a == 0.0f) || (a >= 0x1p-60f && a <= 0x1p+30f);
+}
+
+// voxel index of a coordinate in voxels, kept within an int's range
+__device__ __forceinline__ int walk_index(float v) {
+  return (int)floorf(__builtin_amdgcn_fmed3f(v, -1.0f, 65536.0f));
+}
 
 template <int NW>
 __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restrict__ list,
@@ -401,7 +427,8 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
   const int no = max(nx, nz) + 1;
   float4* rp = walk_lds;                                  // nrays: start, length
   float4* rd = rp + nrays;                                // nrays: direction
-  WalkWin* win = reinterpret_cast<WalkWin*>(rd + nrays);  // nx
+  float4* rq = rd + nrays;                                // nrays: 1 / direction, plain
+  WalkWin* win = reinterpret_cast<WalkWin*>(rq + nrays);  // nx
   int* off = reinterpret_cast<int*>(win + nx);            // nx + 1: first cell of a plane
   float* tab = reinterpret_cast<float*>(off + nx + 1);    // per wavefront: y faces, then x or z faces
   float* cell = tab + NW * (ny + 1 + no);                 // ncells
@@ -422,26 +449,61 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
     const float d0 = ray[3] - ray[0], d1 = ray[4] - ray[1], d2 = ray[5] - ray[2];
     rp[r] = make_float4(ray[0], ray[1], ray[2], absolute3(d0, d1, d2));
     rd[r] = make_float4(d0, d1, d2, d0 == 0.0f ? 0.0f : 1.0f / d0);
+    bool plain = true;
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      plain = plain && walk_plain(ray[c], true) && walk_plain(ray[c + 3] - ray[c], false) &&
+              walk_plain(g.go[c], true) && walk_plain(g.gd[c], false) &&
+              g.gd[c] * (float)g.gn[c] <= 0x1p+31f;
+    rq[r] = make_float4(1.0f / d0, 1.0f / d1, 1.0f / d2, plain ? 1.0f : 0.0f);
   }
   __syncthreads();
   // the axis the rays run along, by the first ray (any choice gives the same sums)
   const bool along_x = fabsf(rd[0].x) >= fabsf(rd[0].z);
-  for (int r = tid; r < nrays; r += BLOCK)
-    if ((along_x ? rd[r].x : rd[r].z) == 0.0f) atomicOr(&s_flag, 1);
+  const float iy_d = 1.0f / g.gd[1], iz_d = 1.0f / g.gd[2];
+  // y and z in voxels at the x faces, as first value and step (in the cells' LDS),
+  // for rays not too steep: sums of up to 1024 voxels and the grid's edge lose less
+  // than WIN_EPS - MARK_EPS to rounding
+  if (4 * nrays > ncells && tid == 0) s_flag = 2;
   __syncthreads();
-  if (s_flag) {   // uniform
+  for (int r = tid; r < nrays; r += BLOCK) {
+    const float4 p = rp[r], d = rd[r], iv = rq[r];
+    if ((along_x ? d.x : d.z) == 0.0f) atomicOr(&s_flag, 1);
+    const float t0 = (g.go[0] - p.x) * iv.x, dt = g.gd[0] * iv.x;
+    const float my = dt * d.y * iy_d, mz = dt * d.z * iz_d;
+    if (!(iv.w != 0.0f && fmaxf(fabsf(my), fabsf(mz)) * (float)nx <= 1024.0f)) atomicOr(&s_flag, 2);
+    if (4 * nrays <= ncells) {
+      cell[4 * r] = (p.y + t0 * d.y - g.go[1]) * iy_d;
+      cell[4 * r + 1] = my;
+      cell[4 * r + 2] = (p.z + t0 * d.z - g.go[2]) * iz_d;
+      cell[4 * r + 3] = mz;
+    }
+  }
+  __syncthreads();
+  const bool steep_rays = s_flag & 2;
+  if (s_flag & 1) {   // uniform
     if (tid == 0) row_cnt[at] = WALK_GENERAL;
     return;
   }
 
   // windows: bounding boxes of the rays' rectangles in every x-plane
   int ncell = 0;
-  const float iy_d = 1.0f / g.gd[1], iz_d = 1.0f / g.gd[2];
   for (int base = 0; base < nx; base += BLOCK) {
     const int i = base + tid;
     float y0 = 1e30f, y1 = -1e30f, z0 = 1e30f, z1 = -1e30f;
     const float xlo = g.go[0] + (float)i * g.gd[0], xhi = g.go[0] + (float)(i + 1) * g.gd[0];
-    for (int r = 0; r < nrays; r++) {
+    for (int r = 0; !steep_rays && r < nrays; r++) {
+      const float ya = __builtin_fmaf((float)i, cell[4 * r + 1], cell[4 * r]);
+      const float za = __builtin_fmaf((float)i, cell[4 * r + 3], cell[4 * r + 2]);
+      const float yb = ya + cell[4 * r + 1], zb = za + cell[4 * r + 3];
+      y0 = fminf(y0, fminf(ya, yb)); y1 = fmaxf(y1, fmaxf(ya, yb));
+      z0 = fminf(z0, fminf(za, zb)); z1 = fmaxf(z1, fmaxf(za, zb));
+    }
+    if (!steep_rays) {
+      y0 -= WIN_EPS; y1 += WIN_EPS; z0 -= WIN_EPS; z1 += WIN_EPS;
+      if (!(y1 >= 0.0f && z1 >= 0.0f && y0 < (float)ny && z0 < (float)nz)) y1 = -1e30f;
+    }
+    for (int r = 0; steep_rays && r < nrays; r++) {
       const float4 p = rp[r], d = rd[r];
       float ta = (xlo - p.x) * d.w, tb = (xhi - p.x) * d.w;
       if (d.x == 0.0f) {   // every x-plane: the ray's way through the grid's z range
@@ -478,6 +540,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
     if (tid == 0) row_cnt[at] = WALK_LEFT;
     return;
   }
+  __syncthreads();
   for (int k = tid; k < ncell; k += BLOCK) cell[k] = 0.0f;
   __syncthreads();
 
@@ -490,11 +553,80 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
   const int i = w * WAVE + lane;      // this lane's plane
   const bool own = i < nd;
   const WalkWin wx = win[along_x && own ? i : 0];
+  // y and other indices this lane may meet (none past the last plane)
+  const int ly = along_x ? wx.y & 0xFFFF : 0, hy = !own ? -1 : along_x ? wx.y >> 16 : ny - 1;
+  const int lo_o = along_x ? wx.z & 0xFFFF : 0, hi_o = !own ? -1 : along_x ? wx.z >> 16 : nother - 1;
+  // faces of this lane's plane and of its places in the tables
+  const float fa = god + (float)i * gdd, fb = god + (float)(i + 1) * gdd;
+  const float fy = g.go[1] + (float)lane * g.gd[1], fo = goo + (float)lane * gdo;
   if (w * WAVE < nd) {
     for (int r = 0; r < nrays; r++) {
       const float4 p = rp[r], d = rd[r];
       const float pd = along_x ? p.x : p.z, dd = along_x ? d.x : d.z;
       const float po = along_x ? p.z : p.x, d_o = along_x ? d.z : d.x;
+      const float4 iv = rq[r];
+      if (__builtin_amdgcn_readfirstlane(iv.w != 0.0f)) {
+        const float idd = along_x ? iv.x : iv.z, ido = along_x ? iv.z : iv.x;
+        if (lane <= ny) taby[lane] = walk_quot(fy - p.y, d.y, iv.y);
+        if (lane <= nother) tabo[lane] = walk_quot(fo - po, d_o, ido);
+        for (int k = lane + WAVE; k <= ny; k += WAVE)
+          taby[k] = walk_quot((g.go[1] + (float)k * g.gd[1]) - p.y, d.y, iv.y);
+        for (int k = lane + WAVE; k <= nother; k += WAVE)
+          tabo[k] = walk_quot((goo + (float)k * gdo) - po, d_o, ido);
+        __builtin_amdgcn_wave_barrier();
+        const float a = walk_quot(fa - pd, dd, idd), b = walk_quot(fb - pd, dd, idd);
+        const float lo = fminf(a, b), hi = fmaxf(a, b);
+        // voxel coordinates where the ray enters and leaves the plane
+        const float my = d.y * iy_d, cy = (p.y - g.go[1]) * iy_d;
+        const float mo = d_o * io_d, co = (po - goo) * io_d;
+        const float ya = __builtin_fmaf(lo, my, cy), yb = __builtin_fmaf(hi, my, cy);
+        const float oa = __builtin_fmaf(lo, mo, co), ob = __builtin_fmaf(hi, mo, co);
+        // the plane's rectangle, and with x-planes the part of it in the window
+        const int y0 = max(ly, walk_index(fminf(ya, yb) - MARK_EPS));
+        const int y1 = min(hy, walk_index(fmaxf(ya, yb) + MARK_EPS));
+        const int o0 = max(lo_o, walk_index(fminf(oa, ob) - MARK_EPS));
+        const int o1 = min(hi_o, walk_index(fmaxf(oa, ob) + MARK_EPS));
+        const int uy = d.y > 0.0f ? 1 : 0, uo = d_o > 0.0f ? 1 : 0;   // uniform
+        if (y0 <= y1 && o0 <= o1) {
+          // table places of the faces the ray leaves by, and of the last ones
+          int ay = (uy ? y0 : y1) + uy, ao = (uo ? o0 : o1) + uo + ny + 1;
+          const float end = fminf(hi, fminf(taby[(uy ? y1 : y0) + uy], tabo[(uo ? o1 : o0) + uo]));
+          const int sy = 2 * uy - 1, so = 2 * uo - 1;
+          float yin = taby[ay - sy], yout = taby[ay], oin = taby[ao - so], oout = taby[ao];
+          // cell of the voxel with x-planes; its x plane else
+          int c = along_x ? wx.base + (ay - uy) * wx.wz + ao - uo - ny - 1 : ao - uo - ny - 1;
+          const int cy_step = along_x ? sy * wx.wz : 0;
+          for (;;) {
+            // a voxel's length, by the reference's maxima and minima (end instead of
+            // hi: beyond it lies no voxel of the rectangle)
+            const float out = fminf(yout, oout);
+            const float lo2 = fmaxf(fmaxf(lo, yin), oin), hi2 = fminf(end, out);
+            if (lo2 < hi2) {
+              if (along_x) {
+                cell[c] += (hi2 - lo2) * p.w;
+              } else {
+                const WalkWin v = win[c];
+                const int iy = ay - uy;
+                if (iy >= (v.y & 0xFFFF) && iy <= v.y >> 16 && i >= (v.z & 0xFFFF) && i <= v.z >> 16)
+                  cell[v.base + iy * v.wz + i] += (hi2 - lo2) * p.w;
+              }
+            }
+            if (!(out < end)) break;
+            const bool by_y = yout <= oout;
+            ay += by_y ? sy : 0;
+            ao += by_y ? 0 : so;
+            c += by_y ? cy_step : so;
+            const float next = taby[by_y ? ay : ao];
+            yin = by_y ? yout : yin;
+            oin = by_y ? oin : oout;
+            yout = by_y ? next : yout;
+            oout = by_y ? oout : next;
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+        continue;
+      }
+      // rays parallel to an axis, or with components out of walk_plain's range
       for (int k = lane; k <= ny; k += WAVE) taby[k] = ((g.go[1] + (float)k * g.gd[1]) - p.y) / d.y;
       for (int k = lane; k <= nother; k += WAVE) tabo[k] = ((goo + (float)k * gdo) - po) / d_o;
       __builtin_amdgcn_wave_barrier();
@@ -626,7 +758,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
 // LDS of k_sm_walk for `cells` cells
 static size_t walk_lds_bytes(const Geo& g, int nw, int cells) {
   const size_t no = (size_t)std::max(g.gn[0], g.gn[2]) + 1;
-  return 32 * (size_t)g.nrays + sizeof(WalkWin) * g.gn[0] + sizeof(int) * (g.gn[0] + 1) +
+  return 48 * (size_t)g.nrays + sizeof(WalkWin) * g.gn[0] + sizeof(int) * (g.gn[0] + 1) +
          sizeof(float) * (nw * ((size_t)g.gn[1] + 1 + no) + cells);
 }
 
