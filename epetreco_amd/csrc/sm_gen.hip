@@ -412,6 +412,15 @@ __device__ __forceinline__ int walk_index(float v) {
   return (int)floorf(__builtin_amdgcn_fmed3f(v, -1.0f, 65536.0f));
 }
 
+// block_rank, without its barriers where the workgroup is one wavefront: they would
+// wait for the entries written before.  (Writing the cells with a value first and
+// reading them back for the candidate test cost a launch on a few wide rows 500 us,
+// two round trips to memory for every 64 cells.)
+template <int NW>
+__device__ __forceinline__ int walk_rank(bool flag, int* s_wave, int* total) {
+  return NW == 1 ? wave_rank(flag, total) : block_rank<NW * WAVE>(flag, s_wave, total);
+}
+
 template <int NW>
 __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restrict__ list,
                                                       int row0, int rowcap, int keep_zeros,
@@ -671,29 +680,13 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
   pixel_centres(g, ci, p0, p1);
   int kept = 0;
   if (!keep_zeros) {
-    // the cells with a value, then their voxels, the candidate test and the mean
+    // the cells with a value: their voxels, the candidate test and the mean
     for (int base = 0; base < ncell; base += BLOCK) {
-      const int k = base + tid;
-      const float a = k < ncell ? cell[k] : 0.0f;
-      int tot;
-      const int r = block_rank<BLOCK>(a != 0.0f, s_wave, &tot);
-      if (a != 0.0f && kept + r < rowcap) { ocol[kept + r] = k; oval[kept + r] = a; }
-      kept += tot;
-    }
-    if (kept > rowcap) {
-      if (tid == 0) row_cnt[at] = -kept;
-      return;   // uniform
-    }
-    const int nval = kept;
-    kept = 0;
-    __syncthreads();   // the list is visible to the whole workgroup
-    for (int base = 0; base < nval; base += BLOCK) {
-      const int k = base + tid;
+      const int c = base + tid;
+      float a = c < ncell ? cell[c] : 0.0f;
       int v = -1;
-      float a = 0.0f;
-      if (k < nval) {
-        const int c = ocol[k];
-        a = oval[k] / (float)nrays;
+      if (a != 0.0f) {
+        a /= (float)nrays;
         int lo = 0, hi = nx - 1;   // plane of cell c: last x with off[x] <= c
         while (lo < hi) {
           const int mid = (lo + hi + 1) >> 1;
@@ -703,11 +696,10 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
         const int rel = c - off[lo];
         v = (lo * ny + (q.y & 0xFFFF) + rel / q.wz) * nz + (q.z & 0xFFFF) + rel % q.wz;
       }
-      __syncthreads();   // every read of this part of the list precedes the writes
       const bool keep = v >= 0 && a != 0.0f && is_candidate(g, p0, p1, v);
       int tot;
-      const int r = block_rank<BLOCK>(keep, s_wave, &tot);
-      if (keep) { ocol[kept + r] = v; oval[kept + r] = a; }
+      const int r = walk_rank<NW>(keep, s_wave, &tot);
+      if (keep && kept + r < rowcap) { ocol[kept + r] = v; oval[kept + r] = a; }
       kept += tot;
     }
   } else {
@@ -737,7 +729,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
         const int v = (ix * ny + iy) * nz + iz;
         const bool keep = k < box && is_candidate(g, p0, p1, v);
         int tot;
-        const int r = block_rank<BLOCK>(keep, s_wave, &tot);
+        const int r = walk_rank<NW>(keep, s_wave, &tot);
         if (keep && kept + r < rowcap) {
           const bool in = iy >= (q.y & 0xFFFF) && iy <= q.y >> 16 && iz >= (q.z & 0xFFFF) &&
                           iz <= q.z >> 16;
@@ -747,12 +739,8 @@ __global__ __launch_bounds__(NW * WAVE) void k_sm_walk(Geo g, const int* __restr
         kept += tot;
       }
     }
-    if (kept > rowcap) {
-      if (tid == 0) row_cnt[at] = -kept;
-      return;
-    }
   }
-  if (tid == 0) row_cnt[at] = kept;
+  if (tid == 0) row_cnt[at] = kept > rowcap ? -kept : kept;
 }
 
 // LDS of k_sm_walk for `cells` cells
