@@ -7,6 +7,7 @@
 
 #include "epet_block.hpp"
 #include "epet_internal.hpp"
+#include "epet_rows.hpp"
 
 namespace epet {
 
@@ -429,6 +430,73 @@ __global__ __launch_bounds__(TR_BLOCK) void k_tr_count(int m, int n, int T, int 
   for (int i = threadIdx.x; i < c1 - c0; i += TR_BLOCK) cnt[blk * n + c0 + i] = tr_c[i];
 }
 
+// Column sums in FP64: workgroup (tile, row block) adds its entries into doubles in
+// LDS and then each column once to memory.  s is zero before.  100,000 rows of 885
+// entries, 52^3 columns: 1.17 ms with an atomic in memory per entry, 0.35 ms so.
+constexpr int CS_TILE = 16384;   // doubles of a workgroup, 128 KB
+template <typename VT>
+__global__ __launch_bounds__(TR_BLOCK) void k_colsum_tiles(int m, int n, int T, int rows_per_block,
+                                                           const int64_t* __restrict__ rowptr,
+                                                           const int* __restrict__ col,
+                                                           const typename VT::T* __restrict__ val,
+                                                           const float* __restrict__ scale,
+                                                           double* __restrict__ s) {
+  extern __shared__ double cs_sum[];
+  __shared__ int64_t s_lo[TR_BLOCK];
+  __shared__ int s_n[TR_BLOCK];
+  const int t = blockIdx.x % T;
+  const long long blk = blockIdx.x / T;
+  const int c0 = t * CS_TILE, c1 = min(n, c0 + CS_TILE);
+  for (int i = threadIdx.x; i < c1 - c0; i += TR_BLOCK) cs_sum[i] = 0.0;
+  const long long r0 = blk * rows_per_block, r1 = min((long long)m, r0 + rows_per_block);
+  for (long long rb = r0; rb < r1; rb += TR_BLOCK) {
+    __syncthreads();
+    tr_bounds(rowptr, col, rb + threadIdx.x, r1, c0, c1, s_lo, s_n);
+    __syncthreads();
+    const int nr = (int)min((long long)TR_BLOCK, r1 - rb);
+    for (int i = wave_id(); i < nr; i += TR_BLOCK / WAVE) {
+      const int64_t lo = s_lo[i];
+      const int len = s_n[i];
+      const float sc = scale ? scale[rb + i] : 1.0f;
+      for (int k = lane_id(); k < len; k += 4 * WAVE) {
+        int c[4];   // four entries requested together
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const bool in = k + j * WAVE < len;
+          c[j] = in ? col[lo + k + j * WAVE] : -1;
+          v[j] = in ? VT::get_cached(val, lo + k + j * WAVE) : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (c[j] >= 0) unsafeAtomicAdd(&cs_sum[c[j] - c0], (double)(v[j] * sc));
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < c1 - c0; i += TR_BLOCK)
+    if (cs_sum[i] != 0.0) unsafeAtomicAdd(&s[c0 + i], cs_sum[i]);
+}
+
+template <typename VT>
+static int launch_colsum_tiles(epet_ctx* ctx, const epet_matrix* A, double* s) {
+  const int T = (A->n + CS_TILE - 1) / CS_TILE;
+  // four workgroups per CU in turn, and rows enough for each to make up for adding
+  // its columns to memory
+  const int want = std::max(1, 4 * ctx->num_cus / T);
+  const int rpb = std::max(16, (A->m + want - 1) / want);
+  const long long grid = (long long)((A->m + rpb - 1) / rpb) * T;
+  const size_t lds = sizeof(double) * (size_t)std::min(A->n, CS_TILE);
+  if (lds > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)k_colsum_tiles<VT>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              CS_TILE * (int)sizeof(double));
+  k_colsum_tiles<VT><<<(unsigned)grid, TR_BLOCK, lds, ctx->stream>>>(
+      A->m, A->n, T, rpb, A->rowptr, A->col, (const typename VT::T*)A->val, A->rowscale, s);
+  EPET_HIP(hipGetLastError());
+  return EPET_OK;
+}
+
 // cnt[blk n + c] -> entries of column c before block blk; total[c] = all of them
 __global__ __launch_bounds__(256) void k_tr_prefix(int n, int B, uint32_t* __restrict__ cnt,
                                                    int* __restrict__ total) {
@@ -823,6 +891,16 @@ int epet_matrix_colsum_f64(epet_ctx* ctx, const epet_matrix* A, double* s) {
   EPET_CHECK(ctx && A && s, EPET_ERR_ARG, "null argument");
   hipStream_t st = ctx->stream;
   k_fill_f64<<<grid_for(A->n, 256, 1ll << 31), 256, 0, st>>>(s, A->n);
+  // sums in LDS where a column has entries enough to make up for adding it to memory
+  // once per row block (3 a column: 14.0 us against 9.9; 13: 120 against 202; 125: 18
+  // against 50)
+  if (A->m > 0 && A->n > 0 && A->cols_strict && A->nnz >= 8ll * A->n) {
+    switch (A->value_type) {
+      case EPET_VAL_F32: return launch_colsum_tiles<ValF32>(ctx, A, s);
+      case EPET_VAL_BF16: return launch_colsum_tiles<ValBF16>(ctx, A, s);
+      default: return launch_colsum_tiles<ValF16>(ctx, A, s);
+    }
+  }
   if (A->m)
     k_colsum_f64<<<A->m, 256, 0, st>>>(A->rowptr, A->col, A->val, A->value_type, A->rowscale,
                                        A->m, s);
