@@ -33,8 +33,7 @@ def _lengths(kind, m, rng):
     return np.full(m, 200)
 
 
-@pytest.mark.parametrize("storage", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("m,n,kind", [
+SHAPES = [
     (1, 4097, "even"),             # one row, less than one window
     (333, 100, "even"),            # one tile, shorter than 128 KB
     (700, 32768, "uneven"),        # exactly one tile
@@ -42,7 +41,11 @@ def _lengths(kind, m, rng):
     (500, 100001, "uneven"),       # four tiles
     (1000, 70000, "one_long"),     # windows of empty rows
     (3000, 40000, "even"),
-])
+]
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("m,n,kind", SHAPES)
 def test_product(gpu_ctx_factory, storage, m, n, kind):
     import scipy.sparse as sp
     from epetreco_amd.api import OP_N, VAL_BF16, VAL_F16, Matrix
@@ -66,3 +69,38 @@ def test_product(gpu_ctx_factory, storage, m, n, kind):
         want = alpha * (M @ xh) + beta * Y0
         bar = 2e-5 * (abs(alpha) * (abs(M) @ np.abs(xh)) + abs(beta * Y0)) + 1e-30
         assert np.all(np.abs(y.cpu().numpy() - want) <= bar)
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("m,n,kind", SHAPES)
+@pytest.mark.parametrize("projected", [True, False])
+def test_back_projection(gpu_ctx_factory, storage, m, n, kind, projected):
+    """Without a transposed copy (k_bp_tiled), before and after a forward product;
+    weights of 0 and an infinity."""
+    import scipy.sparse as sp
+    from epetreco_amd.api import OP_N, OP_T, VAL_BF16, VAL_F16, Matrix
+    rng = np.random.default_rng(m + n)
+    rp, col, val = _csr(rng, m, n, _lengths(kind, m, rng))
+    ctx = gpu_ctx_factory()
+    A = Matrix.from_csr(ctx, torch.as_tensor(rp), torch.as_tensor(col), torch.as_tensor(val), n)
+    if storage != "f32":
+        A = A.convert({"bf16": VAL_BF16, "f16": VAL_F16}[storage])
+    prp, pcol, pval = decoded(A)
+    M = sp.csr_matrix((pval.astype(np.float64), pcol, prp), shape=(m, n)).T.tocsr()
+    if projected:
+        A.spmv(OP_N, torch.ones(n, device="cuda"))
+    x = rng.normal(size=m).astype(np.float32)
+    x[::5] = 0.0
+    Y0 = rng.normal(size=n).astype(np.float32)
+    for alpha, beta in ((1.0, 0.0), (-0.5, 1.5)):
+        y = torch.as_tensor(Y0, device="cuda")
+        A.spmv(OP_T, torch.as_tensor(x, device="cuda"), y, alpha=alpha, beta=beta)
+        want = alpha * (M @ x.astype(np.float64)) + beta * Y0
+        bar = 2e-5 * (abs(alpha) * (abs(M) @ np.abs(x)) + abs(beta * Y0)) + 1e-30
+        assert np.all(np.abs(y.cpu().numpy() - want) <= bar)
+    x[m // 2] = np.inf                # only the voxels of that row become infinite
+    y = A.spmv(OP_T, torch.as_tensor(x, device="cuda")).cpu().numpy()
+    row = pcol[prp[m // 2]:prp[m // 2 + 1]]
+    hit = np.zeros(n, bool)
+    hit[row[pval[prp[m // 2]:prp[m // 2 + 1]] > 0]] = True
+    assert np.all(np.isinf(y[hit])) and np.all(np.isfinite(y[~hit]))
