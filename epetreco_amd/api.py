@@ -389,6 +389,12 @@ class Matrix:
         self.ctx.synchronize()
         return trp, tc[:self.nnz], tv[:self.nnz], ts
 
+    def _out(self, shape, beta: float) -> torch.Tensor:
+        # with beta = 0 the products write every element and read none, so a fill would
+        # be a launch for nothing (a matrix without rows or columns launches nothing)
+        make = torch.empty if beta == 0.0 and self.m > 0 and self.n > 0 else torch.zeros
+        return make(shape, dtype=torch.float32, device=self.ctx.device)
+
     def spmv(self, op: int, x: torch.Tensor, y: Optional[torch.Tensor] = None,
              alpha: float = 1.0, beta: float = 0.0, ctx: Optional[Context] = None) -> torch.Tensor:
         """y = alpha op(A) x + beta y (on `ctx`, the matrix's own context by default)."""
@@ -397,7 +403,7 @@ class Matrix:
             raise EpetError(EPET_ERR_ARG, f"unknown operation {op}")
         nin, nout = (self.n, self.m) if op == OP_N else (self.m, self.n)
         if y is None:
-            y = torch.zeros(nout, dtype=torch.float32, device=self.ctx.device)
+            y = self._out(nout, beta)
         _check_vec(x, nin, "x", self.ctx.device)
         _check_vec(y, nout, "y", self.ctx.device)
         check(lib().epet_matrix_spmv(ctx.handle, self._h, op, alpha, _p(x), beta, _p(y)))
@@ -412,7 +418,7 @@ class Matrix:
         F = X.shape[1]
         nin, nout = (self.n, self.m) if op == OP_N else (self.m, self.n)
         if Y is None:
-            Y = torch.zeros((nout, F), dtype=torch.float32, device=self.ctx.device)
+            Y = self._out((nout, F), beta)
         if Y.dim() != 2 or Y.shape[1] != F:
             raise EpetError(EPET_ERR_ARG, f"Y {tuple(Y.shape)} must have {F} frames")
         _check_vec(X, nin * F, "X", self.ctx.device)
