@@ -589,6 +589,230 @@ __global__ __launch_bounds__(TR_BLOCK) void k_tr_fill(int m, int n, int T, int t
   }
 }
 
+// The same in two steps for longer rows.  What bounds k_tr_fill is its writes, 4
+// bytes here and there over the whole of the transposed arrays (4.5 GB leave L2 for
+// 0.7 GB of entries).  So the entries go first to the bucket of their TR_BUCKET
+// columns, whose room is that of its columns in the result: entries of one row and
+// bucket lie together (3 at 52^3), rows of a block follow one another, and one
+// counter per bucket serves a workgroup for whole rows.  A workgroup then sorts a
+// bucket in LDS, with the columns' next positions in its lanes and the rank of an
+// entry among the 64 of a wavefront by ballots, and writes it in whole lines.
+// Entries (rows of them), k_tr_fill against both steps: 2.7M (133) 90 and 78 us; 8.9M
+// (885) 382 and 237; 89M (885) 3.24 and 1.71 ms; 87M (2,884, 104^3) 5.09 and 2.04.
+// Writing pairs from k_tr_fill and splitting them took 2.48 ms for the 89M, buckets
+// of 32 columns placed straight in memory 2.32.
+constexpr int TR_BUCKET = 8, TR_BITS = 3;
+constexpr int TRP_BLOCK = 512;
+constexpr size_t TR_PAIR_BYTES = (size_t)1 << 30;   // of pairs
+
+template <typename V> struct alignas(8) TrPair {
+  unsigned key;   // row * TR_BUCKET + column in the bucket
+  V val;
+};
+
+// first position of (bucket, row block blk) in pairs and result
+__device__ __forceinline__ long long tr_bucket_start(long long n, long long blk, int bucket,
+                                                     const uint32_t* __restrict__ cnt,
+                                                     const int64_t* __restrict__ tptr) {
+  const long long c0 = (long long)bucket * TR_BUCKET, c1 = min(n, c0 + TR_BUCKET);
+  long long p = tptr[c0];
+  for (long long c = c0; c < c1; c++) p += cnt[blk * n + c];
+  return p;
+}
+
+template <typename V, typename P>
+__global__ __launch_bounds__(TRP_BLOCK) void k_tr_bucket(int m, int n, int T, int tile,
+                                                         int rows_per_block,
+                                                         const int64_t* __restrict__ rowptr,
+                                                         const int* __restrict__ col,
+                                                         const V* __restrict__ val,
+                                                         const uint32_t* __restrict__ cnt,
+                                                         const int64_t* __restrict__ tptr,
+                                                         TrPair<V>* __restrict__ out) {
+  extern __shared__ unsigned char tr_raw[];
+  P* cur = reinterpret_cast<P*>(tr_raw);       // next position of the tile's buckets
+  __shared__ int64_t s_lo[TRP_BLOCK];
+  __shared__ int s_n[TRP_BLOCK];
+  const int t = blockIdx.x % T;
+  const long long blk = blockIdx.x / T;
+  const int c0 = t * tile, c1 = min(n, c0 + tile);   // tile: whole buckets
+  const int b0 = c0 / TR_BUCKET, nb = (c1 - c0 + TR_BUCKET - 1) / TR_BUCKET;
+  for (int i = threadIdx.x; i < nb; i += TRP_BLOCK)
+    cur[i] = (P)tr_bucket_start(n, blk, b0 + i, cnt, tptr);
+  const int lane = lane_id();
+  const long long r0 = blk * rows_per_block, r1 = min((long long)m, r0 + rows_per_block);
+  // one entry per thread: runs of one bucket take their places together
+  auto place = [&](bool in, int c, V v, int r) {
+    const int b = in ? (c >> TR_BITS) - b0 : -1;
+    const int left = __shfl_up(b, 1, WAVE);
+    const bool head = in && (lane == 0 || left != b);
+    const unsigned long long heads = __ballot(head), live = __ballot(in);
+    if (live == 0) return;
+    // the run's head, its length, and the own place in it (lanes in use come first)
+    const unsigned long long below = heads & (~0ull >> (63 - lane));
+    const int h = 63 - __clzll((long long)(below | 1ull));
+    const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1);
+    P base = 0;
+    if (head) {
+      const int next = above ? lane + __ffsll((long long)above) : __popcll(live);
+      base = (P)atomicAdd(&cur[b], (P)(next - lane));
+    }
+    base = __shfl(base, h, WAVE);
+    if (in) out[(long long)base + (lane - h)] = TrPair<V>{(unsigned)r * TR_BUCKET + (c & (TR_BUCKET - 1)), v};
+  };
+  for (long long rb = r0; rb < r1; rb += TRP_BLOCK) {
+    __syncthreads();
+    tr_bounds(rowptr, col, rb + threadIdx.x, r1, c0, c1, s_lo, s_n);
+    __syncthreads();
+    const int nr = (int)min((long long)TRP_BLOCK, r1 - rb);
+    int cn[TR_AHEAD];
+    V vn[TR_AHEAD];
+    auto request = [&](int i0) {
+#pragma unroll
+      for (int j = 0; j < TR_AHEAD; j++) {
+        cn[j] = -1;
+        if (i0 + j < nr && (int)threadIdx.x < s_n[i0 + j]) {
+          cn[j] = col[s_lo[i0 + j] + threadIdx.x];
+          vn[j] = val[s_lo[i0 + j] + threadIdx.x];
+        }
+      }
+    };
+    request(0);
+    for (int i0 = 0; i0 < nr; i0 += TR_AHEAD) {
+      int c[TR_AHEAD];
+      V v[TR_AHEAD];
+#pragma unroll
+      for (int j = 0; j < TR_AHEAD; j++) {
+        c[j] = cn[j];
+        v[j] = vn[j];
+      }
+      request(i0 + TR_AHEAD);
+#pragma unroll
+      for (int j = 0; j < TR_AHEAD; j++) {
+        if (i0 + j >= nr) break;
+        const int r = (int)(rb + i0 + j), len = s_n[i0 + j];
+        place(c[j] >= 0, c[j], v[j], r);
+        for (int k = threadIdx.x + TRP_BLOCK; k - (int)threadIdx.x < len; k += TRP_BLOCK) {
+          const bool in = k < len;
+          place(in, in ? col[s_lo[i0 + j] + k] : -1, in ? val[s_lo[i0 + j] + k] : V(0), r);
+        }
+        // the next row's places come after this row's: wait for LDS alone
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      }
+    }
+  }
+}
+
+// Workgroup = bucket, each wavefront a part of the row blocks: entries in order to
+// their places, in LDS where the bucket fits (then the result is written in whole
+// lines), else in memory.
+constexpr int TR_WAVES = 4;
+constexpr int TR_ROOM = 6144;    // entries of a bucket in LDS
+template <typename V>
+__global__ __launch_bounds__(TR_WAVES * WAVE) void k_tr_place(int n, int B,
+                                                              const uint32_t* __restrict__ cnt,
+                                                              const int64_t* __restrict__ tptr,
+                                                              const TrPair<V>* __restrict__ in,
+                                                              int* __restrict__ orow,
+                                                              V* __restrict__ oval) {
+  __shared__ int s_row[TR_ROOM];
+  __shared__ V s_val[TR_ROOM];
+  const int lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const long long c0 = (long long)blockIdx.x * TR_BUCKET;
+  const long long first = tptr[c0], size = tptr[min((long long)n, c0 + TR_BUCKET)] - first;
+  const bool fits = size <= TR_ROOM;
+  const long long blk0 = (long long)B * w / TR_WAVES, blk1 = (long long)B * (w + 1) / TR_WAVES;
+  const long long c = c0 + (lane & (TR_BUCKET - 1));
+  // this lane's column: its next position in the bucket
+  long long next = 0, a = 0, z = 0;
+  if (c < n) {
+    const long long p = tptr[c];
+    a = blk0 < B ? cnt[blk0 * n + c] : tptr[c + 1] - p;
+    z = blk1 < B ? cnt[blk1 * n + c] : tptr[c + 1] - p;
+    next = p - first + a;
+  }
+  // the part's entries: from all columns' entries before it to those before its end
+#pragma unroll
+  for (int off = TR_BUCKET / 2; off > 0; off >>= 1) {
+    a += __shfl_xor(a, off, WAVE);
+    z += __shfl_xor(z, off, WAVE);
+  }
+  const long long e0 = first + a, e1 = first + z;
+  TrPair<V> q = e0 + lane < e1 ? in[e0 + lane] : TrPair<V>{0u, V(0)};
+  for (long long k = e0; k < e1; k += WAVE) {
+    const TrPair<V> p = q;
+    const bool live = k + lane < e1;
+    const long long kn = min(k + WAVE + lane, e1 - 1);
+    q = in[kn];                               // the next 64, requested before these are placed
+    const unsigned cl = p.key & (TR_BUCKET - 1);
+    unsigned long long same = __ballot(live), own = same;
+#pragma unroll
+    for (int b = 0; b < TR_BITS; b++) {
+      const unsigned long long bit = __ballot((cl >> b) & 1u);
+      same &= (cl >> b) & 1u ? bit : ~bit;
+      own &= (lane >> b) & 1 ? bit : ~bit;
+    }
+    const long long at = __shfl(next, (int)cl, WAVE) + __popcll(same & ((1ull << lane) - 1ull));
+    if (live) {
+      const int r = (int)(p.key >> TR_BITS);
+      if (fits) {
+        s_row[at] = r;
+        s_val[at] = p.val;
+      } else {
+        orow[first + at] = r;
+        oval[first + at] = p.val;
+      }
+    }
+    next += __popcll(own);
+  }
+  __syncthreads();
+  if (fits)
+    for (int i = threadIdx.x; i < (int)size; i += TR_WAVES * WAVE) {
+      orow[first + i] = s_row[i];
+      oval[first + i] = s_val[i];
+    }
+}
+
+// Places the entries by buckets; *done = false where that does not apply: rows too
+// short to occupy a workgroup (57 entries: no gain), keys beyond 32 bits, counters
+// beyond LDS, pairs of more than TR_PAIR_BYTES, or no memory for them.
+template <typename V, typename P>
+static int tr_by_buckets(epet_ctx* ctx, const epet_matrix* A, int rpb, int B, const uint32_t* cnt,
+                         const int64_t* tptr, int* orow, void* oval, bool* done) {
+  *done = false;
+  const int nbuckets = (int)(((long long)A->n + TR_BUCKET - 1) / TR_BUCKET);
+  if (A->nnz < 128ll * A->m || A->m >= (1 << (32 - TR_BITS))) return EPET_OK;
+  const int per_wg = 48 * 1024 / (int)sizeof(P);
+  // two workgroups per CU (one to eight made no difference)
+  const int fit = (nbuckets + per_wg - 1) / per_wg;
+  int T = std::max(fit, std::min(16, std::max(1, 512 / B)));
+  if (fit > 16) return EPET_OK;
+  const int tile = (nbuckets + T - 1) / T * TR_BUCKET;
+  T = (A->n + tile - 1) / tile;
+  hipStream_t st = ctx->stream;
+  // A block that is kept for the next matrix once freed: 0.7 GB from the pool of
+  // temporaries, which keeps less, took 35 ms longer a reconstruction.
+  const size_t bytes = sizeof(TrPair<V>) * (size_t)A->nnz;
+  if (bytes > TR_PAIR_BYTES) return EPET_OK;
+  struct Block {
+    void* p = nullptr;
+    ~Block() { (void)dev_free(p); }            // waits for the device
+  } block;
+  if (dev_malloc(&block.p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return EPET_OK;
+  }
+  TrPair<V>* pairs = (TrPair<V>*)block.p;
+  k_tr_bucket<V, P><<<(unsigned)(B * T), TRP_BLOCK, sizeof(P) * (size_t)(tile / TR_BUCKET), st>>>(
+      A->m, A->n, T, tile, rpb, A->rowptr, A->col, (const V*)A->val, cnt, tptr, pairs);
+  k_tr_place<V><<<(unsigned)nbuckets, TR_WAVES * WAVE, 0, st>>>(A->n, B, cnt, tptr, pairs, orow,
+                                                                (V*)oval);
+  EPET_HIP(hipGetLastError());
+  *done = true;
+  return EPET_OK;
+}
+
 template <typename V, typename P>
 static void launch_tr_fill(hipStream_t st, int grid, int m, int n, int T, int tile, int rpb,
                            const int64_t* rowptr, const int* col, const void* val,
@@ -947,14 +1171,27 @@ int epet_matrix_transpose(epet_ctx* ctx, epet_matrix* A) {
   k_set_last_i64<<<1, 64, 0, st>>>(T->rowptr + A->n, (int64_t)A->nnz);
   if (any) {
     const int g = B * nt;
-    if (A->value_type == EPET_VAL_F32) {
+    bool done = false;
+    if (A->value_type == EPET_VAL_F32 && wide)
+      EPET_TRY((tr_by_buckets<float, unsigned long long>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
+                                                   &done)));
+    else if (A->value_type == EPET_VAL_F32)
+      EPET_TRY((tr_by_buckets<float, unsigned>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
+                                         &done)));
+    else if (wide)
+      EPET_TRY((tr_by_buckets<uint16_t, unsigned long long>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
+                                                      &done)));
+    else
+      EPET_TRY((tr_by_buckets<uint16_t, unsigned>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
+                                            &done)));
+    if (!done && A->value_type == EPET_VAL_F32) {
       if (wide)
         launch_tr_fill<float, uint64_t>(st, g, A->m, A->n, nt, tile, rpb, A->rowptr, A->col, A->val,
                                         cnt, T->rowptr, T->col, T->val);
       else
         launch_tr_fill<float, uint32_t>(st, g, A->m, A->n, nt, tile, rpb, A->rowptr, A->col, A->val,
                                         cnt, T->rowptr, T->col, T->val);
-    } else {
+    } else if (!done) {
       if (wide)
         launch_tr_fill<uint16_t, uint64_t>(st, g, A->m, A->n, nt, tile, rpb, A->rowptr, A->col,
                                            A->val, cnt, T->rowptr, T->col, T->val);
