@@ -45,9 +45,12 @@ __global__ __launch_bounds__(256) void k_unpack_keys(const uint64_t* __restrict_
 
 // One read of the (row, col) pairs: bitwise AND and OR over all keys (digits
 // where they agree are constant), and whether any key is below the one before
-// it (out[2]).  Bound by the 8 bytes per pair it reads.  A workgroup reduces
+// it (out[2]).  Bound by the 8 bytes per pair it reads: a lane takes four pairs by
+// two 16-byte loads, the key before them comes from the lane before (40M pairs: 113
+// us, 147 with two 4-byte reads of every pair).  A workgroup reduces
 // before its three atomics: with two 64-bit atomics per wavefront on one cache
 // line, 40M pairs took 411 us here.
+typedef int coo_i4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ __launch_bounds__(256) void k_coo_scan(const int* __restrict__ row,
                                                   const int* __restrict__ col, long long n,
                                                   unsigned long long* __restrict__ out) {
@@ -55,8 +58,31 @@ __global__ __launch_bounds__(256) void k_coo_scan(const int* __restrict__ row,
   __shared__ int s_f[256 / WAVE];
   uint64_t a = ~0ull, o = 0ull;
   bool below = false;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
+  const long long nq = n / 4;
+  const int lane = lane_id();
+  for (long long q0 = (long long)blockIdx.x * 256 + wave_id() * WAVE; q0 < nq;
+       q0 += (long long)gridDim.x * 256) {
+    const bool in = q0 + lane < nq;
+    const long long q = in ? q0 + lane : nq - 1;
+    const coo_i4 r = *reinterpret_cast<const coo_i4*>(row + 4 * q);
+    const coo_i4 c = *reinterpret_cast<const coo_i4*>(col + 4 * q);
+    const long long before = q0 > 0 ? 4 * q0 - 1 : 0;
+    const uint64_t first = coo_key(row[before], col[before]);
+    uint64_t k[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      k[i] = coo_key(r[i], c[i]);
+      a &= k[i];
+      o |= k[i];
+      if (i > 0) below |= k[i] < k[i - 1];
+    }
+    uint64_t prev = __shfl_up(k[3], 1, WAVE);
+    if (lane == 0) prev = first;
+    below |= in && k[0] < prev;
+  }
+  // the last 0 to 3 pairs
+  if (blockIdx.x == 0 && threadIdx.x < (unsigned)(n - 4 * nq)) {
+    const long long i = 4 * nq + threadIdx.x;
     const uint64_t k = coo_key(row[i], col[i]);
     a &= k;
     o |= k;
@@ -169,6 +195,7 @@ __global__ __launch_bounds__(256) void k_fill_i32(int* __restrict__ p, long long
 // entry serialises on the row's counter (40M entries of 2,001 sorted rows:
 // 32.8 ms, with runs 0.1 ms, near the read of the ids).
 constexpr int HIST_SPAN = 16 * WAVE;
+constexpr int HIST_AHEAD = 8;   // loads of a wavefront in flight (40M sorted ids: 47 us, with one 61)
 __global__ __launch_bounds__(256) void k_row_hist(const int* __restrict__ rowid, long long nnz,
                                                   int m, int* __restrict__ cnt,
                                                   int* __restrict__ bad) {
@@ -183,25 +210,36 @@ __global__ __launch_bounds__(256) void k_row_hist(const int* __restrict__ rowid,
     const long long b = span * HIST_SPAN;
     const long long e = b + HIST_SPAN < nnz ? b + HIST_SPAN : nnz;
     int cur = 0, run = 0;   // wavefront-uniform: the run that reaches the end of the last 64
-    for (long long base = b; base < e; base += WAVE) {
-      const bool in = base + lane < e;
-      const int r = in ? rowid[base + lane] : 0;
-      const int n = (int)(e - base < WAVE ? e - base : WAVE);
-      if (run > 0 && __all(!in || r == cur)) {
-        run += n;
-        continue;
+    for (long long at = b; at < e; at += HIST_AHEAD * WAVE) {
+      int ahead[HIST_AHEAD];
+#pragma unroll
+      for (int j = 0; j < HIST_AHEAD; j++) {
+        const long long i = at + j * WAVE + lane;
+        ahead[j] = rowid[i < e ? i : e - 1];
       }
-      if (run > 0 && lane == 0) add(cur, run);
-      // runs within these n entries; the last one is carried on
-      const int prev = __shfl_up(r, 1, WAVE);
-      const unsigned long long heads = __ballot(in && (lane == 0 || r != prev));
-      const int last = 63 - __clzll((long long)heads);
-      if (in && lane != last && ((heads >> lane) & 1)) {
-        const unsigned long long after = heads & (~0ull << lane << 1);
-        add(r, __ffsll((long long)after) - 1 - lane);
+#pragma unroll
+      for (int j = 0; j < HIST_AHEAD; j++) {
+        const long long base = at + j * WAVE;
+        if (base >= e) break;
+        const bool in = base + lane < e;
+        const int r = ahead[j];
+        const int n = (int)(e - base < WAVE ? e - base : WAVE);
+        if (run > 0 && __all(!in || r == cur)) {
+          run += n;
+          continue;
+        }
+        if (run > 0 && lane == 0) add(cur, run);
+        // runs within these n entries; the last one is carried on
+        const int prev = __shfl_up(r, 1, WAVE);
+        const unsigned long long heads = __ballot(in && (lane == 0 || r != prev));
+        const int last = 63 - __clzll((long long)heads);
+        if (in && lane != last && ((heads >> lane) & 1)) {
+          const unsigned long long after = heads & (~0ull << lane << 1);
+          add(r, __ffsll((long long)after) - 1 - lane);
+        }
+        cur = __shfl(r, last, WAVE);
+        run = n - last;
       }
-      cur = __shfl(r, last, WAVE);
-      run = n - last;
     }
     if (run > 0 && lane == 0) add(cur, run);
   }
@@ -886,7 +924,7 @@ int epet_cooSort(epet_ctx* ctx, float* val, int* row, int* col, long long N) {
   StreamTemps tmp(st);
   EPET_HIP(tmp.alloc(&scan, sizeof(unsigned long long) * 3));
   k_init_scan<<<1, 64, 0, st>>>(scan);
-  k_coo_scan<<<grid_for(N, 256, 8ll * ctx->num_cus), 256, 0, st>>>(row, col, N, scan);
+  k_coo_scan<<<grid_for((N + 3) / 4, 256, 8ll * ctx->num_cus), 256, 0, st>>>(row, col, N, scan);
   EPET_HIP(hipGetLastError());
   unsigned long long ao[3];
   EPET_TRY(read_pinned(ctx, ao, scan, sizeof(ao)));
