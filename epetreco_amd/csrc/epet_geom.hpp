@@ -127,6 +127,35 @@ __device__ __forceinline__ bool is_candidate(const Geo& g, const float p0[3],
   return distance_pl(p0, p1, c) < g.sumRadii;
 }
 
+// The same predicate for many voxels of one channel.  sqrt(q) / |ab| < R, with q as
+// distance_pl computes it, is decided by q against R^2 |ab|^2 where the two differ by
+// more than 1e-5, and by the root and the quotient, both correctly rounded, only
+// between: all roundings on the way from q and to the bounds add up to less than 1e-6.
+struct CandidateTest {
+  float a[3], ab[3], len, lo, hi;
+  __device__ __forceinline__ CandidateTest(const Geo& g, const float p0[3], const float p1[3]) {
+#pragma unroll
+    for (int d = 0; d < 3; d++) { a[d] = p0[d]; ab[d] = p1[d] - p0[d]; }
+    len = absolute3(ab[0], ab[1], ab[2]);
+    const float rl = g.sumRadii * len;
+    const bool plain = rl > 1e-15f && rl < 1e15f;    // squares far from the ends of the range
+    lo = plain ? rl * rl * (1.0f - 1e-5f) : -1.0f;
+    hi = plain ? rl * rl * (1.0f + 1e-5f) : __builtin_inff();
+  }
+  __device__ __forceinline__ bool operator()(const Geo& g, int ix, int iy, int iz) const {
+    const float p0 = g.go[0] + ((float)ix + 0.5f) * g.gd[0] - a[0];
+    const float p1 = g.go[1] + ((float)iy + 0.5f) * g.gd[1] - a[1];
+    const float p2 = g.go[2] + ((float)iz + 0.5f) * g.gd[2] - a[2];
+    const float c0 = ab[1] * p2 - ab[2] * p1;
+    const float c1 = ab[2] * p0 - ab[0] * p2;
+    const float c2 = ab[0] * p1 - ab[1] * p0;
+    const float q = (c0 * c0 + c1 * c1) + c2 * c2;
+    if (q < lo) return true;
+    if (q > hi) return false;
+    return sqrtf(q) / len < g.sumRadii;
+  }
+};
+
 // Voxel box corners (getSystemMatrixDeviceOnly.cu:166-175).
 __device__ __forceinline__ void voxel_box(const Geo& g, int v, float box[6]) {
   int id[3];
