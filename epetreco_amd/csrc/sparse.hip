@@ -46,22 +46,23 @@ __global__ __launch_bounds__(256) void k_unpack_keys(const uint64_t* __restrict_
 // One read of the (row, col) pairs: bitwise AND and OR over all keys (digits
 // where they agree are constant), and whether any key is below the one before
 // it (out[2]).  Bound by the 8 bytes per pair it reads: a lane takes four pairs by
-// two 16-byte loads, the key before them comes from the lane before (40M pairs: 113
-// us, 147 with two 4-byte reads of every pair).  A workgroup reduces
-// before its three atomics: with two 64-bit atomics per wavefront on one cache
-// line, 40M pairs took 411 us here.
+// two 16-byte loads, the key before them comes from the lane before (with two
+// 4-byte reads of every pair, 40M pairs took 30 us more).  The atomics on one cache
+// line are taken one by one, so few large workgroups reduce before theirs: 40M
+// pairs 99 us, 113 with 2,048 workgroups of 256 threads, 411 with atomics per wavefront.
+constexpr int SCAN_BLOCK = 1024;
 typedef int coo_i4 __attribute__((ext_vector_type(4), aligned(4)));
-__global__ __launch_bounds__(256) void k_coo_scan(const int* __restrict__ row,
+__global__ __launch_bounds__(SCAN_BLOCK) void k_coo_scan(const int* __restrict__ row,
                                                   const int* __restrict__ col, long long n,
                                                   unsigned long long* __restrict__ out) {
-  __shared__ unsigned long long s_a[256 / WAVE], s_o[256 / WAVE];
-  __shared__ int s_f[256 / WAVE];
+  __shared__ unsigned long long s_a[SCAN_BLOCK / WAVE], s_o[SCAN_BLOCK / WAVE];
+  __shared__ int s_f[SCAN_BLOCK / WAVE];
   uint64_t a = ~0ull, o = 0ull;
   bool below = false;
   const long long nq = n / 4;
   const int lane = lane_id();
-  for (long long q0 = (long long)blockIdx.x * 256 + wave_id() * WAVE; q0 < nq;
-       q0 += (long long)gridDim.x * 256) {
+  for (long long q0 = (long long)blockIdx.x * SCAN_BLOCK + wave_id() * WAVE; q0 < nq;
+       q0 += (long long)gridDim.x * SCAN_BLOCK) {
     const bool in = q0 + lane < nq;
     const long long q = in ? q0 + lane : nq - 1;
     const coo_i4 r = *reinterpret_cast<const coo_i4*>(row + 4 * q);
@@ -101,13 +102,14 @@ __global__ __launch_bounds__(256) void k_coo_scan(const int* __restrict__ row,
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 256 / WAVE; w++) {
+    for (int w = 1; w < SCAN_BLOCK / WAVE; w++) {
       a &= s_a[w];
       o |= s_o[w];
+      s_f[0] |= s_f[w];
     }
     atomicAnd(&out[0], (unsigned long long)a);
     atomicOr(&out[1], (unsigned long long)o);
-    if (s_f[0] | s_f[1] | s_f[2] | s_f[3]) atomicOr(&out[2], 1ull);
+    if (s_f[0]) atomicOr(&out[2], 1ull);
   }
 }
 
@@ -924,7 +926,7 @@ int epet_cooSort(epet_ctx* ctx, float* val, int* row, int* col, long long N) {
   StreamTemps tmp(st);
   EPET_HIP(tmp.alloc(&scan, sizeof(unsigned long long) * 3));
   k_init_scan<<<1, 64, 0, st>>>(scan);
-  k_coo_scan<<<grid_for((N + 3) / 4, 256, 8ll * ctx->num_cus), 256, 0, st>>>(row, col, N, scan);
+  k_coo_scan<<<grid_for((N + 3) / 4, SCAN_BLOCK, 2ll * ctx->num_cus), SCAN_BLOCK, 0, st>>>(row, col, N, scan);
   EPET_HIP(hipGetLastError());
   unsigned long long ao[3];
   EPET_TRY(read_pinned(ctx, ao, scan, sizeof(ao)));
