@@ -601,23 +601,43 @@ __global__ __launch_bounds__(256) void k_blk_gather(float* __restrict__ Gp,
   Gp[i] = (c >= 0 && f < F) ? G[(long long)c * F + f] : 0.0f;
 }
 
-// Split reductions, in split order.  Forward: the MLEM ratio (in row-position
-// order) and the FP64 log-likelihood (one atomic per workgroup and frame); back
-// projection: the image.
-__global__ __launch_bounds__(256) void k_blk_reduce(BlkArgs a) {
+// Split reductions.  Forward: the MLEM ratio (in row-position order) and the FP64
+// log-likelihood (one atomic per workgroup and frame); back projection: the image.
+// W = 1: a thread adds an element's partial sums in split order.  A few rows over
+// many column tiles have hundreds of splits and few elements, which that left to
+// wait for one load after the other (120 rows over 641,424 voxels, 14 frames, 627
+// splits: 153 us); W wavefronts then share 64 elements (8 us).
+constexpr int BLK_WIDE = 16, BLK_WIDE_SPLITS = 32;
+template <int W>
+__global__ __launch_bounds__(W == 1 ? 256 : W * WAVE) void k_blk_reduce(BlkArgs a) {
+  constexpr int ITEMS = W == 1 ? 256 : WAVE;
   __shared__ double s_ll[64];
+  __shared__ float s_part[W][WAVE];
   if (threadIdx.x < 64) s_ll[threadIdx.x] = 0.0;
   __syncthreads();
   const long long tot = (long long)a.m_pad * a.F;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
-       i += (long long)gridDim.x * blockDim.x) {
+  for (long long i0 = (long long)blockIdx.x * ITEMS; i0 < tot; i0 += (long long)gridDim.x * ITEMS) {
+    const long long i = i0 + threadIdx.x % ITEMS;
     const long long p = i / a.F;
     const int f = (int)(i % a.F);
-    const int orig = a.rowperm[p];
-    if (orig < 0) continue;
+    const int orig = i < tot ? a.rowperm[p] : -1;
     float s = 0.0f;
-    for (int sp = 0; sp < a.splits; sp++)
-      s += a.partial[(((long long)sp * a.m_pad + p) << a.lgFp) + f];
+    if (orig >= 0) {
+      const float* part = a.partial + (p << a.lgFp) + f;
+      const long long step = (long long)a.m_pad << a.lgFp;
+#pragma unroll 4
+      for (int sp = W == 1 ? 0 : wave_id(); sp < a.splits; sp += W) s += part[sp * step];
+    }
+    if (W > 1) {
+      s_part[wave_id()][lane_id()] = s;
+      __syncthreads();
+      s = 0.0f;
+      if (wave_id() == 0)
+        for (int w = 0; w < W; w++) s += s_part[w][lane_id()];
+      __syncthreads();
+      if (wave_id() != 0) continue;
+    }
+    if (orig < 0) continue;
     const long long o = (long long)orig * a.F + f;
     if (a.mode == 1) {
       a.out[o] = s;
@@ -1101,8 +1121,12 @@ static int blk_launch(epet_ctx* ctx, const BlkCopy* B, int P, int rb, int splits
   kern<<<grid, BLK_THREADS, 0, ctx->stream>>>(a);
   if (splits > 1) {
     a.mode = mode;
-    k_blk_reduce<<<grid_for((long long)B->m_pad * F, 256, 16ll * ctx->num_cus), 256, 0,
-                   ctx->stream>>>(a);
+    const long long items = (long long)B->m_pad * F;
+    if (splits > BLK_WIDE_SPLITS)
+      k_blk_reduce<BLK_WIDE><<<grid_for(items, WAVE, 16ll * ctx->num_cus), BLK_WIDE * WAVE, 0,
+                               ctx->stream>>>(a);
+    else
+      k_blk_reduce<1><<<grid_for(items, 256, 16ll * ctx->num_cus), 256, 0, ctx->stream>>>(a);
   }
   EPET_HIP(hipGetLastError());
   return EPET_OK;
