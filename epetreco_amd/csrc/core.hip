@@ -53,12 +53,14 @@ int ctx_scratch(epet_ctx* ctx, size_t bytes, void** out) {
 // again: a reconstruction allocates and frees tens of blocks of up to hundreds
 // of MB, and at a few GB per 25 ms the driver's clearing of freed memory falls
 // behind (passes of 22 ms stalled for 50 to 130 ms now and then); a small build
-// spent 250 of 370 us in allocations.  At most DEV_KEEP bytes per device are
-// kept, for as long as a context on the device is open; they are given back
+// spent 250 of 370 us in allocations.  At most DEV_KEEP bytes per device, a twentieth
+// of the card, are kept (with 4 GB, closing series of 150,000 rows of 899 entries at
+// 52^3, 5 GB each, or of 99,000 of 2,794 stalled for 50 to 200 ms now and then; with
+// 16 GB none of 16 did), for as long as a context on the device is open; they are given back
 // when the last one closes and when an allocation fails.  A block is kept only
 // once the device has finished all work (which hipFree waits for as well), so
 // any thread or stream may take it.
-constexpr size_t DEV_KEEP = (size_t)4 << 30;
+constexpr size_t DEV_KEEP = (size_t)16 << 30;
 constexpr size_t TMP_KEEP = (size_t)1 << 30;   // stream-ordered temporaries
 constexpr int DEV_MAX = 64;
 
