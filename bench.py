@@ -139,7 +139,7 @@ def batched_bytes(nnz, m, V, F, sval, scaled):
 
 
 def batched_traffic(workload, storage):
-    """HBM bytes per batched iteration of the blocked products (both
+    """HBM bytes per batched iteration of the multi-frame products (both
     directions, the split reduction and the gather) from the committed counter
     summary, or None."""
     path = os.path.join(ROOT, "profiles", f"traffic_batched_{workload}.json")
@@ -281,7 +281,7 @@ def series_104(frames=8, niter=30, chunk=400_000):
     results = {}
     for key, vt in (("fp16_row_scale", VAL_F16), ("bf16_row_scale", VAL_BF16)):
         # rebuilt (deterministic generation) rather than uploaded: a generated
-        # matrix carries its channel ids and grid, which order the blocked copies
+        # matrix carries its channel ids and grid, which order the multi-frame copies
         A32 = ctx.sm_build(rows)
         M = A32.convert(vt)
         A32.close()
@@ -289,7 +289,7 @@ def series_104(frames=8, niter=30, chunk=400_000):
         M.attach_transpose()
         X = torch.full((V, F), 1.0 / V, device="cuda")
         t0 = time.time()
-        ctx.mlem(M, Yd, s, X, 1, use_graph=True)          # blocked copies and tuning
+        ctx.mlem(M, Yd, s, X, 1, use_graph=True)          # multi-frame copies and tuning
         torch.cuda.synchronize()
         prep_s = time.time() - t0
         X.fill_(1.0 / V)
@@ -411,7 +411,7 @@ def main():
         t0 = time.perf_counter()
         cfg, tms = ctx.mlem_tune(M, F)
         torch.cuda.synchronize()
-        say(f"tuned in {time.perf_counter() - t0:.2f} s (incl. blocked copies): {cfg} {tms}")
+        say(f"tuned in {time.perf_counter() - t0:.2f} s (incl. copies): {cfg} {tms}")
         ctx.mlem(M, Yp, prob.s, Xp, 3, use_graph=False)
         torch.cuda.synchronize()
         src = torch.ones(1 << 28, device="cuda")
@@ -518,7 +518,7 @@ def main():
                                 "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                                 "frac": B_it / ms_it / 1e6 / HBM_PEAK_GBPS,
                                 "algorithmic_bytes": B_it, "traffic": tr,
-                                "scope": "one F-frame MLEM iteration (graph replay, all kernels)"}}
+                                "scope": "one F-frame MLEM iteration (all kernels)"}}
             say(f"    {B_it / 1e9:.1f} GB algorithmic per iteration: {B_it / ms_it / 1e6:.0f} GB/s, "
                 f"{B_it / ms_it / 1e6 / HBM_PEAK_GBPS:.1%} of 8 TB/s"
                 + (f"; counters {tr / 1e9:.1f} GB" if tr else ""))
