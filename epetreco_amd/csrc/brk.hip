@@ -566,8 +566,7 @@ __global__ __launch_bounds__(256) void k_brk_reduce(BrkArgs a) {
     if (f >= a.F) continue;
     const int o = a.rowperm[p];
     if (o < 0) continue;
-    float s = 0.0f;
-    for (int sp = 0; sp < a.splits; sp++) s += a.partial[((long long)sp * a.mpos + p) * FP + f];
+    const float s = sum_ahead(a.partial + i, a.splits, (long long)a.mpos * FP);
     const float sc = a.rowscale ? a.rowscale[o] : 1.0f;
     if (a.mode == 1) {
       brk_store(a, (long long)o * a.F + f, s, sc);

@@ -434,8 +434,7 @@ __global__ __launch_bounds__(256) void k_lds_reduce(int m, int T, const float* _
                                                     float* __restrict__ y) {
   const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= m) return;
-  float s = 0.0f;
-  for (int t = 0; t < T; t++) s += partial[(long long)t * m + r];
+  const float s = sum_ahead(partial + r, T, m);
   const float v = alpha * (rowscale ? rowscale[r] : 1.0f) * s;
   y[r] = beta == 0.0f ? v : v + beta * y[r];
 }
@@ -455,11 +454,10 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_lds_ratio(int m, int T, const flo
   double ll = 0.0;
   for (long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x; r < m;
        r += (long long)gridDim.x * blockDim.x) {
-    float s = 0.0f;
-    for (int t = 0; t < T; t++) s += partial[(long long)t * m + r];
+    const float yi = y[r];   // requested with the partials
+    const float s = sum_ahead(partial + r, T, m);
     const float sc = rowscale ? rowscale[r] : 1.0f;
     const float yh = s * sc;
-    const float yi = y[r];
     const float ev = yh > 0.0f ? yi / yh : 0.0f;
     e[r] = fold ? ev * sc : ev;
     if (yh > 0.0f) ll += (double)yi * log((double)yh) - (double)yh;
