@@ -891,19 +891,19 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
     rows = std::max<long long>(1, std::min<long long>(rows, 1 << 17));
     rows = std::min<long long>(rows, m - r0);
     if (rows > maxrows) {
-      if (cnt) (void)hipFreeAsync(cnt, ctx->stream);
+      // one block for all three: each allocation and its end cost the host a few us,
+      // which builds of some hundred rows (40 us of kernels) notice
       if (off) (void)hipFreeAsync(off, ctx->stream);
-      if (left_d) (void)hipFreeAsync(left_d, ctx->stream);
-      cnt = nullptr;
       off = nullptr;
-      left_d = nullptr;
-      if (tmp_malloc((void**)&cnt, sizeof(int) * rows, ctx->stream) != hipSuccess ||
-          tmp_malloc((void**)&left_d, sizeof(int) * rows, ctx->stream) != hipSuccess ||
-          tmp_malloc((void**)&off, sizeof(int64_t) * (rows + 1), ctx->stream) != hipSuccess) {
+      const size_t off_b = sizeof(int64_t) * (rows + 1), cnt_b = sizeof(int) * rows;
+      if (tmp_malloc((void**)&off, off_b + 2 * cnt_b, ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
+        off = nullptr;
         rc = fail(EPET_ERR_ALLOC, __FILE__, __LINE__, "row counts");
         break;
       }
+      cnt = (int*)((char*)off + off_b);
+      left_d = (int*)((char*)off + off_b + cnt_b);
       maxrows = (int)rows;
     }
     void* scr = nullptr;
@@ -915,9 +915,11 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
     // rows that the one before left
     std::vector<int> hc(rows), left, general;
     auto counts = [&]() -> int {   // the rows' counts, and which rows have none yet
-      if (hipMemcpyAsync(hc.data(), cnt, sizeof(int) * rows, hipMemcpyDeviceToHost, ctx->stream) !=
-              hipSuccess ||
-          hipStreamSynchronize(ctx->stream) != hipSuccess)
+      if (sizeof(int) * rows <= 4096) {
+        EPET_TRY(read_pinned(ctx, hc.data(), cnt, sizeof(int) * rows));
+      } else if (hipMemcpyAsync(hc.data(), cnt, sizeof(int) * rows, hipMemcpyDeviceToHost, ctx->stream) !=
+                     hipSuccess ||
+                 hipStreamSynchronize(ctx->stream) != hipSuccess)
         return fail(EPET_ERR_HIP, __FILE__, __LINE__, "row count readback");
       left.clear();
       general.clear();
@@ -971,9 +973,7 @@ static int generate_rows(epet_ctx* ctx, const Geo& g, const int* list, int m,
     if (rc != EPET_OK) break;
     r0 += (int)rows;
   }
-  if (cnt) (void)hipFreeAsync(cnt, ctx->stream);
   if (off) (void)hipFreeAsync(off, ctx->stream);
-  if (left_d) (void)hipFreeAsync(left_d, ctx->stream);
   return rc;
 }
 
