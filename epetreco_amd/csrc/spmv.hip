@@ -179,9 +179,9 @@ __global__ __launch_bounds__(256) void k_spmv_n_vec(int m, const int64_t* __rest
 }
 
 // ------------------------------------------------------------------ tiled back projection
-// The image is cut into tiles of BP_TILE consecutive voxel ids (64 KB of LDS).
+// The image is cut into tiles of BP_TILE consecutive voxel ids (128 KB of LDS).
 // Workgroup (row block, tile) accumulates a_ij e_i of its rows' entries inside
-// the tile with LDS float atomics and writes the tile into its row block's
+// the tile with LDS double atomics and writes the tile into its row block's
 // partial image; a reduction sums the partial images.  Entry ranges of every
 // (row, tile) come from a per-matrix plan of tile-boundary offsets.
 constexpr int BP_TILE = 16384;
@@ -216,13 +216,15 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_tiled(int m, int n, int T, int 
                                                        const uint32_t* __restrict__ toff,
                                                        const float* __restrict__ e, float alpha,
                                                        float* __restrict__ partial) {
-  __shared__ float acc[BP_TILE];
+  // FP64: a block's sums come in any order, and have to round to the same floats
+  // (11,250 rows of 405 entries, 52^3: 58 us, with floats 51)
+  __shared__ double acc[BP_TILE];
   const int t = blockIdx.y;
   const long long r0 = (long long)blockIdx.x * rows_per_block;
   const long long r1 = min((long long)m, r0 + rows_per_block);
   const int tile0 = t * BP_TILE;
   const int tn = min(BP_TILE, n - tile0);
-  for (int j = threadIdx.x; j < BP_TILE; j += BP_BLOCK) acc[j] = 0.0f;
+  for (int j = threadIdx.x; j < BP_TILE; j += BP_BLOCK) acc[j] = 0.0;
   __syncthreads();
   const int sub = threadIdx.x & 31;          // 32 lanes per row segment
   const int seg = threadIdx.x >> 5;          // 32 segments per workgroup
@@ -259,12 +261,12 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_tiled(int m, int n, int T, int 
       // compare keeps LDS indices in range even for an inconsistent plan
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        if (k + 32 * i < hi && j[i] < BP_TILE) atomicAdd(&acc[j[i]], v[i] * ev);
+        if (k + 32 * i < hi && j[i] < BP_TILE) unsafeAtomicAdd(&acc[j[i]], (double)(v[i] * ev));
     }
   }
   __syncthreads();
   float* out = partial + (size_t)blockIdx.x * n + tile0;
-  for (int j = threadIdx.x; j < tn; j += BP_BLOCK) out[j] = acc[j];
+  for (int j = threadIdx.x; j < tn; j += BP_BLOCK) out[j] = (float)acc[j];
 }
 
 // y[j] = beta * y[j] + sum over row blocks of partial[b][j]: 64 columns per
