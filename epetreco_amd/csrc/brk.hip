@@ -1115,6 +1115,25 @@ int brk_prepare(epet_ctx* ctx, epet_matrix* A, int F) {
   return EPET_OK;
 }
 
+// Whether Y = A X is the faster one by the rows (k_spmm_n) than on bricks.  Bricks
+// take 33 to 35 us of launches and working memory and 2 to 4 ps an entry, whatever
+// the frames up to 16.  By the rows, a row is a wavefront's, F of its entries' frames
+// at a time, so that few long rows wait for one load after the other (0.4 us each);
+// else an entry and frame take 2 to 3 ps, 0.7 to 0.8 where the gathered vector stays
+// near.  Rows / bricks in us, FP32: 9,001 rows, 0.49M entries, 16^3 voxels, 8 frames
+// 6 / 34; 0.90M, 64 frames 46 / 39; 700 rows, 0.60M, 52^3, 4 frames 17 / 33, 16 frames
+// 83 / 33; 4.4M, 2 frames 32 / 51, 4 frames 55 / 51; 48.8M, 2 frames 197 / 156.
+// The back projection by the rows adds with float atomics, several times further from
+// the exact sums (4e-7 against 1.1e-7, 50,000 rows of 899 entries), and stays on bricks.
+static bool brk_rows_faster(const epet_matrix* A, int F) {
+  const double e = 1e-6 * (double)A->nnz;
+  int P = 2;
+  while (P < F) P *= 2;
+  const double serial = 0.4 / WAVE * P * (double)A->nnz / A->m;
+  const double rows = 5.0 + std::max(serial, e * F * (A->n < 32768 ? 0.8 : 3.0));
+  return rows < 35.0 + e * (1.5 + 0.7 * brk_parts(A->value_type));
+}
+
 // Y = alpha op(A) X + beta Y on bricks: *done = false where they do not apply.
 // The bricks are built for a matrix with a transposed copy (a program that
 // back-projects several frames again and again) once its products come to
@@ -1150,6 +1169,7 @@ int brk_spmm(epet_ctx* ctx, const epet_matrix* cA, int op, int F, float alpha, c
     EPET_TRY(brk_build_both(ctx, A));
     if (A->brk_state.load() != 1) return EPET_OK;
   }
+  if (op == EPET_OP_N && brk_rows_faster(A, F)) return EPET_OK;
   const BrkCopy* B = op == EPET_OP_N ? A->brk : A->tr->brk;
   const int Fp = brk_pad(F);
   // about 14,000 wavefronts (3.5 rounds of 16 per CU) measured best over the

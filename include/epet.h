@@ -218,7 +218,8 @@ int epet_matrix_spmv(epet_ctx* ctx, const epet_matrix* A, int op, float alpha,
  * op N: Y(m x nrhs) = alpha*A*X + beta*Y; op T: Y(n x nrhs) = alpha*A^T X + beta*Y.
  * A generated matrix with its transposed copy attached keeps bricks for the
  * matrix cores (see epet_mlem) once products enough have been asked of it: that
- * call synchronises, and sums are in another order from then on. */
+ * call synchronises, and sums are in another order from then on (op N only where it
+ * is large enough to gain by them). */
 int epet_matrix_spmm(epet_ctx* ctx, const epet_matrix* A, int op, int nrhs,
                      float alpha, const float* X_dev, float beta, float* Y_dev);
 
