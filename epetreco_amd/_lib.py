@@ -35,6 +35,7 @@ SIGNATURES = {
     "epet_ctx_destroy": (ctypes.c_int, [P]),
     "epet_ctx_set_stream": (ctypes.c_int, [P, P]),
     "epet_ctx_synchronize": (ctypes.c_int, [P]),
+    "epet_release_cached": (ctypes.c_int, [P]),
     "epet_set_geometry": (ctypes.c_int, [P, P, P]),
     "epet_set_nrays": (ctypes.c_int, [P, ctypes.c_int]),
     "epet_set_seed": (ctypes.c_int, [P, ctypes.c_uint64]),

@@ -93,6 +93,11 @@ class Context:
     def synchronize(self):
         check(lib().epet_ctx_synchronize(self._h))
 
+    def release_cached(self):
+        """Gives the device memory that the library keeps for its next matrices back
+        (up to 18 GB), for torch and other allocators in the process."""
+        check(lib().epet_release_cached(self._h))
+
     # -- geometry (device_constant_memory.hpp:14-26) ------------------------
     def set_geometry(self, setup: MeasurementSetup, grid: VoxelGrid, nrays: int = None,
                      seed: int = None):

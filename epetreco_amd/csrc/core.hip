@@ -57,7 +57,8 @@ int ctx_scratch(epet_ctx* ctx, size_t bytes, void** out) {
 // of the card, are kept (with 4 GB, closing series of 150,000 rows of 899 entries at
 // 52^3, 5 GB each, or of 99,000 of 2,794 stalled for 50 to 200 ms now and then; with
 // 16 GB none of 16 did), for as long as a context on the device is open; they are given back
-// when the last one closes and when an allocation fails.  A block is kept only
+// when the last one closes, when an allocation here fails, and by epet_release_cached,
+// for other allocators in the process.  A block is kept only
 // once the device has finished all work (which hipFree waits for as well), so
 // any thread or stream may take it.
 constexpr size_t DEV_KEEP = (size_t)16 << 30;
@@ -223,6 +224,19 @@ static void dev_close(int dev) {
   (void)hipDeviceSynchronize();
   if (pool) (void)hipMemPoolDestroy(pool);
   dev_trim(d);
+}
+
+// gives back what is kept on `dev` (current) and not in use
+static hipError_t dev_release(int dev) {
+  if (dev >= DEV_MAX) return hipSuccess;
+  DevBlocks& d = dev_blocks()[dev];
+  // temporaries freed on any stream are back in the pool then
+  const hipError_t e = hipDeviceSynchronize();
+  if (e != hipSuccess) return e;
+  dev_trim(d);
+  // a last context that closes takes the pool away under the same lock
+  std::lock_guard<std::mutex> lock(d.mu);
+  return d.pool ? hipMemPoolTrimTo(d.pool, 0) : hipSuccess;
 }
 
 int ctx_geo(epet_ctx* ctx, Geo* g) {
@@ -430,6 +444,18 @@ int epet_ctx_destroy(epet_ctx* ctx) {
   dev_close(ctx->device);
   if (cur != ctx->device && cur >= 0) (void)hipSetDevice(cur);
   delete ctx;
+  return EPET_OK;
+}
+
+int epet_release_cached(epet_ctx* ctx) {
+  EPET_CHECK(ctx, EPET_ERR_ARG, "null context");
+  EPET_HIP(hipStreamSynchronize(ctx->stream));
+  int cur = -1;
+  EPET_HIP(hipGetDevice(&cur));
+  if (cur != ctx->device) EPET_HIP(hipSetDevice(ctx->device));
+  const hipError_t e = dev_release(ctx->device);
+  if (cur != ctx->device) EPET_HIP(hipSetDevice(cur));
+  EPET_HIP(e);
   return EPET_OK;
 }
 

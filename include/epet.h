@@ -78,6 +78,12 @@ int epet_ctx_destroy(epet_ctx* ctx);
 int epet_ctx_set_stream(epet_ctx* ctx, void* stream);
 int epet_ctx_synchronize(epet_ctx* ctx);
 
+/* Freed device memory of matrices and calls (up to 16 GB of blocks and 2 GB of
+ * temporaries per device) is kept for the next ones while a context on the device is
+ * open.  This gives all of it back to the driver, for other allocators in the
+ * process; it waits for the device. */
+int epet_release_cached(epet_ctx* ctx);
+
 /* Geometry, rays per channel and Philox seed of the context.  Replaces the
  * cudaMemcpyToSymbol uploads of setup_const / grid_const / nrays_const
  * (device_constant_memory.hpp:14-26, tests/reco.cu:64-72).  The per-angle
