@@ -169,6 +169,22 @@ hipError_t dev_free(void* p) {
   return e;
 }
 
+// A caller may have given a block from epet_malloc to hipFree and have another one at
+// its address: forgets the block that was there unless this one is as large.
+static void dev_check(void* p) {
+  DevLive& l = dev_live();
+  std::lock_guard<std::mutex> lock(l.mu);
+  auto it = l.block.find(p);
+  if (it == l.block.end()) return;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess || base != p ||
+      size < it->second.second) {
+    (void)hipGetLastError();
+    l.block.erase(it);
+  }
+}
+
 // stream-ordered temporaries, from a pool that keeps up to TMP_KEEP bytes
 // between calls (the device's default pool gives them back at every
 // synchronisation)
@@ -544,6 +560,7 @@ int epet_free(epet_ctx* ctx, void* ptr) {
   EPET_CHECK(ctx, EPET_ERR_ARG, "null context");
   if (ptr) {
     EPET_HIP(hipStreamSynchronize(ctx->stream));
+    dev_check(ptr);
     EPET_HIP(dev_free(ptr));
   }
   return EPET_OK;
