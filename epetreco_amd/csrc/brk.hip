@@ -960,19 +960,38 @@ static int brk_vec_ensure(epet_ctx* ctx, BrkCopy* B, int Fp, bool* ok) {
   return EPET_OK;
 }
 
-static bool brk_partial_ensure(BrkCopy* B, int splits, int Fp) {
-  if (splits <= 1) return true;
-  const long long need = (long long)splits * B->mpos * Fp;
+// Room for `need` partial sums; a block that is there stays when there is no memory
+// for a larger one.
+static bool brk_partial_ensure(BrkCopy* B, long long need) {
   if (need <= B->partial_len) return true;
-  if (B->partial) (void)dev_free(B->partial);
-  B->partial = nullptr;
-  B->partial_len = 0;
-  if (dev_malloc((void**)&B->partial, sizeof(float) * (size_t)need) != hipSuccess) {
+  float* p = nullptr;
+  if (dev_malloc((void**)&p, sizeof(float) * (size_t)need) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
+  if (B->partial) (void)dev_free(B->partial);
+  B->partial = p;
   B->partial_len = need;
   return true;
+}
+static long long brk_partials(const BrkCopy* B, int splits, int Fp) {
+  return splits > 1 ? (long long)splits * B->mpos * Fp : 0;
+}
+// The partial sums of the launch shapes in use alone (what tuning asked for beyond
+// them is given back; no memory for the smaller block leaves the larger).
+static void brk_partial_fit(BrkCopy* B) {
+  long long need = 0;
+  for (int s = 0; s < 4; s++)
+    if (B->tuned[s]) need = std::max(need, brk_partials(B, B->splits[s], 8 << s));
+  if (need >= B->partial_len) return;
+  float* p = nullptr;
+  if (need > 0 && dev_malloc((void**)&p, sizeof(float) * (size_t)need) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  (void)dev_free(B->partial);
+  B->partial = p;
+  B->partial_len = need;
 }
 
 template <int NA, int FP>
@@ -1022,7 +1041,7 @@ static int brk_launch(epet_ctx* ctx, const BrkCopy* B, int Fp, BrkArgs& a) {
 // mode 1 the back projection.
 static int brk_product(epet_ctx* ctx, const BrkCopy* B, const BrkCopy* o, int Fp, int splits,
                        int mode, const MfArgs& m, const float* rowscale) {
-  EPET_CHECK(splits <= 1 || (B->partial && B->partial_len >= (long long)splits * B->mpos * Fp),
+  EPET_CHECK(splits <= 1 || (B->partial && B->partial_len >= brk_partials(B, splits, Fp)),
              EPET_ERR_STATE, "bricks: partial buffer missing");
   EPET_CHECK(brk_vec(B, Fp) && brk_vec(o, Fp), EPET_ERR_STATE, "bricks: gathered vector missing");
   EPET_CHECK(mode != 0 || o->npos >= B->mpos, EPET_ERR_STATE,
@@ -1215,9 +1234,7 @@ bool brk_ready(const epet_matrix* A, int F) {
   if (!brk_built(A, F)) return false;
   const int s = brk_slot(brk_pad(F));
   for (const BrkCopy* B : {A->brk, A->tr->brk})
-    if (B->tuned[s] != F ||
-        (B->splits[s] > 1 && B->partial_len < (long long)B->splits[s] * B->mpos * brk_pad(F)))
-      return false;
+    if (B->tuned[s] != F || B->partial_len < brk_partials(B, B->splits[s], brk_pad(F))) return false;
   return true;
 }
 
@@ -1232,7 +1249,17 @@ int brk_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& m) {
 }
 
 // Splits of a group's steps, per direction: enough wavefronts to fill the chip
-// against partial sums to add, by time.
+// against partial sums to add, by time.  Tried are splits of two batches of steps
+// and more, up to BRK_TRY_WAVES wavefronts, 16 rounds of 16 per CU: the fastest had
+// 2,256 (9,001 rows, 16^3 voxels) to 35,152 (99,000 rows back, 104^3), and each takes
+// as many partial sums: 64 frames of 3.3M rows in 64 parts, the limit by steps alone,
+// would take 55 GB to find that one part is best.
+constexpr long long BRK_TRY_WAVES = 65536;
+static int brk_most_splits(const BrkCopy* B) {
+  int most = 1;
+  while (most < 64 && B->nsteps >= 8ll * B->G * most && 2ll * B->G * most <= BRK_TRY_WAVES) most *= 2;
+  return most;
+}
 int brk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& m, int reps) {
   const int Fp = brk_pad(m.F), s = brk_slot(Fp);
   BrkCopy* dirs[2] = {A->brk, A->tr->brk};
@@ -1245,10 +1272,9 @@ int brk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& m, int reps) {
   for (int d = 0; d < 2 && rc == EPET_OK; d++) {
     BrkCopy* B = dirs[d];
     float best = 1e30f;
-    for (int splits = 1; splits <= 64 && rc == EPET_OK; splits *= 2) {
-      // no finer than two batches of steps each
-      if (splits > 1 && B->nsteps < 4ll * B->G * splits) break;
-      if (!brk_partial_ensure(B, splits, Fp)) break;
+    int most = brk_most_splits(B);
+    while (most > 1 && !brk_partial_ensure(B, brk_partials(B, most, Fp))) most /= 2;
+    for (int splits = 1; splits <= most && rc == EPET_OK; splits *= 2) {
       auto run = [&]() {
         MfArgs q = m;
         q.loglik = nullptr;
@@ -1271,6 +1297,7 @@ int brk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& m, int reps) {
     }
     B->ms[s] = best;
     B->tuned[s] = m.F;
+    brk_partial_fit(B);
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
