@@ -29,6 +29,12 @@
 // three bfloat16 (8 of its 24 significant bits each, by truncation), a stored
 // value of two (FP16) or one (BF16).  All part products are added, each exact, so
 // the sums differ from FP32 fused multiply-adds only in the order of additions.
+// By itself that would hold down to 2^-110 alone: a bfloat16 has no bits below
+// 2^-133, an FP32 number has them down to 2^-149 (at 2^-120 the three parts miss 1e-4
+// of it).  So k_brk_gather writes the vector times BRK_UP, and the sums are multiplied
+// by 1 / BRK_UP (a factor in the main loop instead took 1 to 4% of the product).  The
+// ratios that the forward product hands to the back projection are not scaled, as they
+// may be large.
 // Measured against 64 bits (relative 2-norm of the images, 2 to 10 iterations of
 // the four series in perf/cases.py): 1.9e-7 to 3.6e-7, with k_blk 2.9e-7 to 3.9e-7.
 // The parts of the gathered vector are columns of the other operand: 8 frames x 3
@@ -38,8 +44,9 @@
 // what a step waits for.
 //
 // Cells without an entry multiply the gathered vector by 0, which is not 0 for
-// an infinity or NaN: frames that hold one are recomputed from the same bricks
-// entry by entry.
+// an infinity or NaN: frames that hold one are recomputed from the same bricks and
+// the caller's vector entry by entry, and so are frames with numbers above BRK_BIG,
+// whose scaled sums could leave the range, and with ratios below BRK_SMALL.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -68,6 +75,9 @@ constexpr int BRK_LL = 64;         // copies of the log-likelihood sums
 // an entry.  At 92 to 110 entries a step bricks still won (16^3, 8 rays, 5 frames:
 // 17 and 23 us against 27 and 32); below 80 k_blk is kept.
 constexpr int BRK_MIN_ENTRIES = 80;
+
+// scaled sums stay below 2^96 times a row's sum of magnitudes
+constexpr float BRK_UP = 0x1p+24f, BRK_BIG = 0x1p+72f, BRK_SMALL = 0x1p-100f;
 
 typedef __bf16 brk_bf8 __attribute__((ext_vector_type(8)));
 typedef float brk_f16v __attribute__((ext_vector_type(16)));
@@ -98,7 +108,7 @@ struct BrkCopy {
   int64_t* gent = nullptr;          // G: first entry of a group
   unsigned* rec = nullptr;          // BRK_REC (nsteps / 2)
   uint16_t* val = nullptr;          // parts x (nent + BRK_TAIL)
-  unsigned long long* flag = nullptr;   // frames of the gathered vector with an infinity or NaN
+  unsigned long long* flag = nullptr;   // frames of the gathered vector to do entry by entry
   double* ll = nullptr;             // BRK_LL x 64 log-likelihood sums (zero between iterations)
   float* partial = nullptr;         // splits x mpos x Fp
   long long partial_len = 0;
@@ -137,6 +147,10 @@ struct BrkArgs {
   const uint16_t* val;
   long long vstride;           // between the parts of val
   const float* x;              // gathered vector
+  float down;                  // 1 / its factor
+  const float* xin;            // the vector it was gathered from, its columns by position
+  const int* colinv;           // and a scale per column (or null); xin null: x is unscaled
+  const float* xscale;
   const unsigned long long* flag;
   unsigned long long* clear;   // flag word of the other direction, cleared here (or null)
   const int* rowperm;
@@ -176,16 +190,35 @@ template <int FP>
 __device__ __forceinline__ size_t brk_at(long long pos, int f) {
   return ((size_t)(pos >> 2) * FP + f) * 4 + (size_t)(pos & 3);
 }
-__device__ __forceinline__ bool brk_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
+// Numbers that the split of a scaled and of an unscaled vector holds
+__device__ __forceinline__ bool brk_fits_up(float v) { return fabsf(v) <= BRK_BIG; }
+__device__ __forceinline__ bool brk_fits(float v) {
+  return v == 0.0f || (fabsf(v) >= BRK_SMALL && fabsf(v) <= 3.402823466e38f);
+}
+// Flags the lanes' frames (lane l: frame base + l % FP, all lanes at once) by one
+// atomic per wavefront and only where they are not flagged yet: atomics on one address
+// take 12 ns each.
+template <int FP>
+__device__ __forceinline__ void brk_flag(unsigned long long* flag, bool set, int base) {
+  unsigned long long m = __ballot(set);
+  if (m == 0) return;
+  if (FP <= 32) m |= m >> 32;
+  if (FP <= 16) m |= m >> 16;
+  if (FP <= 8) m |= m >> 8;
+  if (FP < 64) m &= (1ull << (FP & 63)) - 1ull;
+  m <<= base;
+  if (lane_id() == 0 && (m & ~__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0)
+    atomicOr(flag, m);
+}
 
 __device__ __forceinline__ void brk_store(const BrkArgs& a, long long at, float sum, float scale) {
   const float v = a.alpha * scale * sum;
   a.out[at] = a.beta == 0.0f ? v : v + a.beta * a.out[at];
 }
 
-// The gathered vector (times a scale per column, if any) in position order: one
-// thread per (four positions, frame).  Clears the other direction's flags and
-// sets this one's for frames with an infinity or NaN.
+// The gathered vector (times a scale per column, if any) times BRK_UP in position
+// order: one thread per (four positions, frame).  Clears the other direction's flags
+// and sets this one's.
 template <int FP>
 __global__ __launch_bounds__(256) void k_brk_gather(float* __restrict__ xs,
                                                     const float* __restrict__ X,
@@ -197,17 +230,20 @@ __global__ __launch_bounds__(256) void k_brk_gather(float* __restrict__ xs,
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const int f = (int)(i % FP);
   const long long q = i / FP;
-  if (q >= nquad || f >= F) return;
-  float v[4];
+  bool out = false;
+  if (q < nquad && f < F) {
+    float v[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int c = colinv[q * 4 + j];
-    v[j] = c >= 0 ? X[(long long)c * F + f] : 0.0f;
-    if (scale && c >= 0) v[j] *= scale[c];
+    for (int j = 0; j < 4; j++) {
+      const int c = colinv[q * 4 + j];
+      v[j] = c >= 0 ? X[(long long)c * F + f] : 0.0f;
+      if (scale && c >= 0) v[j] *= scale[c];
+      out |= !brk_fits_up(v[j]);
+      v[j] *= BRK_UP;
+    }
+    *reinterpret_cast<float4*>(xs + brk_at<FP>(q * 4, f)) = make_float4(v[0], v[1], v[2], v[3]);
   }
-  *reinterpret_cast<float4*>(xs + brk_at<FP>(q * 4, f)) = make_float4(v[0], v[1], v[2], v[3]);
-  if (!(brk_finite(v[0]) && brk_finite(v[1]) && brk_finite(v[2]) && brk_finite(v[3])))
-    atomicOr(flag, 1ull << f);
+  brk_flag<FP>(flag, out, 0);
 }
 
 // ------------------------------------------------------------------ main kernel
@@ -445,7 +481,15 @@ __global__ __launch_bounds__(BRK_WAVES * WAVE) void k_brk(BrkArgs a) {
           acc[i][0][r] += __shfl_xor(acc[i][0][r], 16, WAVE);
         }
     }
-    // frames with an infinity or NaN in the gathered vector: entry by entry
+    if (a.down != 1.0f) {
+#pragma unroll
+      for (int i = 0; i < BRK_SUB; i++)
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[i][c][r] *= a.down;
+    }
+    // frames with numbers that the split does not hold: entry by entry
     const unsigned long long bad = *a.flag & (a.F >= 64 ? ~0ull : (1ull << a.F) - 1ull);
     if (bad) {
       for (int f = 0; f < a.F; f++) {
@@ -462,7 +506,16 @@ __global__ __launch_bounds__(BRK_WAVES * WAVE) void k_brk(BrkArgs a) {
               float v = 0.0f;
               for (int k = NA - 1; k >= 0; k--)
                 v += brk_bf(reinterpret_cast<const uint16_t*>(vp + k * vs)[at]);
-              sum[i] += v * a.x[brk_at<FP>((long long)hd.x * 8 + j, f)];
+              const long long pos = (long long)hd.x * 8 + j;
+              float x;
+              if (a.xin) {
+                const int col = a.colinv[pos];
+                x = a.xin[(long long)col * a.F + f];
+                if (a.xscale) x *= a.xscale[col];
+              } else {
+                x = a.x[brk_at<FP>(pos, f)];
+              }
+              sum[i] += v * x;
               at++;
             }
           }
@@ -508,10 +561,10 @@ __global__ __launch_bounds__(BRK_WAVES * WAVE) void k_brk(BrkArgs a) {
           if (r % Q == q && o >= 0 && f < a.F) brk_store(a, (long long)o * a.F + f, acc[i][c][r], sc);
         }
     } else {
-      bool bad_e = false;
 #pragma unroll
       for (int c = 0; c < NC; c++) {
         const int f = 32 * c + f0;
+        bool out = false;
 #pragma unroll
         for (int o8 = 0; o8 < 4; o8++) {            // octet o8 of the group, positions 4 h .. 4 h + 3
           float w[4];
@@ -526,7 +579,7 @@ __global__ __launch_bounds__(BRK_WAVES * WAVE) void k_brk(BrkArgs a) {
               ev = yh > 0.0f ? yi / yh : 0.0f;
               if (yh > 0.0f && q == 0) ll[c] += (double)yi * log((double)yh) - (double)yh;
               if (a.fold) ev *= sc;
-              bad_e |= !brk_finite(ev);
+              out |= !brk_fits(ev);
             }
             w[r4] = ev;
           }
@@ -534,8 +587,7 @@ __global__ __launch_bounds__(BRK_WAVES * WAVE) void k_brk(BrkArgs a) {
             *reinterpret_cast<float4*>(a.oute + brk_at<FP>(p0 + 8 * o8 + 4 * h, f)) =
                 make_float4(w[0], w[1], w[2], w[3]);
         }
-        if (bad_e) atomicOr(a.oflag, 1ull << f);
-        bad_e = false;
+        brk_flag<(FP < 32 ? FP : 32)>(a.oflag, out, 32 * c);
       }
     }
     }
@@ -559,6 +611,7 @@ __global__ __launch_bounds__(256) void k_brk_reduce(BrkArgs a) {
   if (threadIdx.x < 64) s_ll[threadIdx.x] = 0.0;
   __syncthreads();
   const long long tot = (long long)a.mpos * FP;
+  bool out = false;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
        i += (long long)gridDim.x * blockDim.x) {
     const long long p = i / FP;
@@ -577,9 +630,10 @@ __global__ __launch_bounds__(256) void k_brk_reduce(BrkArgs a) {
     float ev = yh > 0.0f ? yi / yh : 0.0f;
     if (yh > 0.0f) atomicAdd(&s_ll[f], (double)yi * log((double)yh) - (double)yh);
     if (a.fold) ev *= sc;
-    if (!brk_finite(ev)) atomicOr(a.oflag, 1ull << f);
+    out |= !brk_fits(ev);
     a.oute[brk_at<FP>(p, f)] = ev;
   }
+  if (a.mode == 0) brk_flag<FP>(a.oflag, out, 0);   // a thread stays on its frame
   if (a.mode == 0 && a.ll) {
     __syncthreads();
     if ((int)threadIdx.x < a.F)
@@ -822,7 +876,7 @@ static std::vector<int> brk_voxel_positions(const MatGeo& g) {
 // ------------------------------------------------------------------ build (host)
 // Bricks of M with row positions `rows` and column positions `cols` (-1: none).
 // EPET_OK with *out == nullptr when memory is short, or (*unfit) the sizes are
-// beyond the kernel's or the bricks are too empty to pay.
+// beyond the kernel's, or the bricks too empty to pay.
 static int brk_build(epet_ctx* ctx, const epet_matrix* M, const std::vector<int>& rows,
                      const std::vector<int>& cols, BrkCopy** out, bool* unfit) {
   *out = nullptr;
@@ -1055,7 +1109,10 @@ static int brk_product(epet_ctx* ctx, const BrkCopy* B, const BrkCopy* o, int Fp
   a.partial = B->partial;
   a.itp = m.itp;
   a.alpha = 1.0f;
+  a.down = mode == 0 ? 1.0f / BRK_UP : 1.0f;   // the image by k_brk_gather, the ratio as it is
   if (mode == 0) {
+    a.xin = m.x;
+    a.colinv = B->colinv;
     a.oute = brk_vec(o, Fp)->x;
     a.oflag = o->flag;
     a.rowscale = rowscale;
@@ -1214,6 +1271,10 @@ int brk_spmm(epet_ctx* ctx, const epet_matrix* cA, int op, int F, float alpha, c
   a.splits = splits;
   a.mode = 1;
   a.x = xs;
+  a.down = 1.0f / BRK_UP;
+  a.xin = X;
+  a.colinv = B->colinv;
+  a.xscale = op == EPET_OP_T ? A->rowscale : nullptr;
   a.flag = flag;
   a.partial = reinterpret_cast<float*>(w + 256 + xb);
   a.out = Y;

@@ -1,0 +1,109 @@
+"""Bricks over the whole range of FP32: gathered vectors with numbers down to the
+smallest, infinities and NaN, and vectors of small and huge numbers at once.
+
+Tolerance against FP64: a row has a few hundred entries, so its FP32 sums keep a
+relative error of some 1e-7 of the sum of magnitudes; bar 2e-6, where a vector of
+numbers near 2^-120 that lost the bits below 2^-133 misses 1e-4.  Results below the
+normal numbers are multiples of 2^-149: 2^-148 beside that for each of up to 64
+partial sums (2^-142).  MLEM
+divides by such sums once per iteration: same bar for one iteration."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import decoded, env_ctx
+from test_gpu_spmm_routes import product, scan, with_bricks
+
+pytestmark = pytest.mark.gpu
+
+
+def _sparse(A):
+    import scipy.sparse as sp
+    rp, col, val = decoded(A)
+    return sp.csr_matrix((val.astype(np.float64), col, rp), shape=(A.m, A.n))
+
+
+def _agree(got, K, X, what):
+    X = X.cpu().numpy().astype(np.float64)
+    want = K @ X
+    bar = 2e-6 * (abs(K) @ np.abs(X)) + 2.0 ** -142
+    worst = np.max(np.abs(got.cpu().numpy() - want) / bar)
+    assert worst <= 1.0, (what, worst)
+
+
+@pytest.fixture(scope="module", params=["f32", "bf16", "f16"])
+def bricks(request, gpu_ctx_factory):
+    ctx, A = scan(gpu_ctx_factory, 51, 49, 53, 64, 6001, request.param)
+    with_bricks(ctx, A)
+    return ctx, A, _sparse(A)
+
+
+@pytest.mark.parametrize("F", [8, 13, 40])
+@pytest.mark.parametrize("exponent", [-99, -101, -112, -116, -120, -126, -133])
+def test_small_numbers(bricks, F, exponent):
+    from epetreco_amd.api import OP_N, OP_T
+    ctx, A, M = bricks
+    rng = np.random.default_rng(F)
+    for op, K, n in ((OP_N, M, A.n), (OP_T, M.T, A.m)):
+        X = torch.as_tensor((rng.normal(size=(n, F)) * 2.0 ** exponent).astype(np.float32), device="cuda")
+        _agree(product(ctx, A, op, X), K, X, (op, exponent))
+
+
+@pytest.mark.parametrize("F", [8, 20])
+@pytest.mark.parametrize("low,high", [(-120, 0), (-140, 45), (-118, 60), (-118, 71), (-118, 100)])
+def test_small_and_large_numbers(bricks, F, low, high):
+    """One frame small throughout, one with magnitudes from small to large, the others
+    ordinary: each as exact as by itself."""
+    from epetreco_amd.api import OP_N, OP_T
+    ctx, A, M = bricks
+    rng = np.random.default_rng(F)
+    for op, K, n in ((OP_N, M, A.n), (OP_T, M.T, A.m)):
+        x = rng.normal(size=(n, F))
+        x[:, 1] *= 2.0 ** low
+        x[:, F - 2] *= 2.0 ** rng.uniform(low, high, n)
+        X = torch.as_tensor(x.astype(np.float32), device="cuda")
+        _agree(product(ctx, A, op, X), K, X, (op, low, high))
+
+
+@pytest.mark.parametrize("F", [8, 20])
+def test_infinities_and_nan(bricks, monkeypatch, F):
+    """Where the row kernel has an infinity or NaN, so have bricks, and nowhere else."""
+    from epetreco_amd.api import OP_N, OP_T
+    ctx, A, M = bricks
+    rows_only = env_ctx(monkeypatch, EPET_BATCHED="gather")
+    for op, K, n in ((OP_N, M, A.n), (OP_T, M.T, A.m)):
+        X = torch.rand(n, F, device="cuda") + 0.5
+        X[n // 2, 0] = float("inf")
+        X[n // 3, 2] = float("nan")
+        X[n // 3, 3] = -float("inf")
+        X[n // 3 + 1, 3] = float("inf")
+        X[:, 4] *= 2.0 ** -119
+        X[n // 2, 4] = float("inf")
+        got, want = product(ctx, A, op, X), product(rows_only, A, op, X)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        ok = want.isfinite()
+        assert ok.any(0).all() and (~ok).any(0)[[0, 2, 3, 4]].all()
+        bar = torch.as_tensor(4e-6 * (abs(K) @ np.abs(np.nan_to_num(X.cpu().numpy().astype(np.float64),
+                                                                   nan=0.0, posinf=0.0, neginf=0.0))) +
+                              2.0 ** -142, device="cuda")
+        assert ((got.double() - want.double()).abs() <= bar)[ok].all()
+
+
+@pytest.mark.parametrize("F", [5, 16, 33])
+def test_mlem_of_a_small_image(bricks, oracle, F):
+    """An image of magnitude 2^-120 to start from (a caller may hand over any), data such
+    that the ratios are finite: 1 iteration."""
+    ctx, A, M = bricks
+    rng = np.random.default_rng(F)
+    Y = (rng.poisson(4.0, (A.m, F)) * 2.0 ** -14).astype(np.float32)
+    X0 = rng.uniform(0.5, 1.5, (A.n, F)).astype(np.float32)
+    X0[:, 1] *= np.float32(2.0 ** -120)
+    s = A.colsum_f64().float()
+    X = torch.as_tensor(X0, device="cuda")
+    ctx.mlem(A, torch.as_tensor(Y, device="cuda"), s, X, 1)
+    assert ctx.batched_config(A, F)["path"].startswith("bricks")
+    rp, col, val = decoded(A)
+    X64 = oracle.mlem_f64_frames(A.m, A.n, val, rp, col, Y, s.cpu().numpy(), X0.astype(np.float64), 1)
+    X = X.cpu().numpy()
+    for f in range(F):
+        assert np.linalg.norm(X[:, f] - X64[:, f]) <= 2e-6 * np.linalg.norm(X64[:, f]), f
