@@ -34,7 +34,8 @@
 // of it).  So k_brk_gather writes the vector times BRK_UP, and the sums are multiplied
 // by 1 / BRK_UP (a factor in the main loop instead took 1 to 4% of the product).  The
 // ratios that the forward product hands to the back projection are not scaled, as they
-// may be large.
+// may be large.  Matrices with stored values out of [BRK_VAL_MIN, BRK_VAL_MAX] stay
+// with the other kernels.
 // Measured against 64 bits (relative 2-norm of the images, 2 to 10 iterations of
 // the four series in perf/cases.py): 1.9e-7 to 3.6e-7, with k_blk 2.9e-7 to 3.9e-7.
 // The parts of the gathered vector are columns of the other operand: 8 frames x 3
@@ -46,7 +47,9 @@
 // Cells without an entry multiply the gathered vector by 0, which is not 0 for
 // an infinity or NaN: frames that hold one are recomputed from the same bricks and
 // the caller's vector entry by entry, and so are frames with numbers above BRK_BIG,
-// whose scaled sums could leave the range, and with ratios below BRK_SMALL.
+// whose scaled sums could leave the range, and with ratios below BRK_SMALL.  An
+// infinite stored value would meet the zero parts of the vector: it is out of the
+// range above.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -78,6 +81,7 @@ constexpr int BRK_MIN_ENTRIES = 80;
 
 // scaled sums stay below 2^96 times a row's sum of magnitudes
 constexpr float BRK_UP = 0x1p+24f, BRK_BIG = 0x1p+72f, BRK_SMALL = 0x1p-100f;
+constexpr float BRK_VAL_MIN = 0x1p-100f, BRK_VAL_MAX = 0x1p+16f;
 
 typedef __bf16 brk_bf8 __attribute__((ext_vector_type(8)));
 typedef float brk_f16v __attribute__((ext_vector_type(16)));
@@ -800,7 +804,8 @@ __global__ __launch_bounds__(BRK_BUILD) void k_brk_values(int nwords, int vt, in
                                                           const int64_t* __restrict__ gent,
                                                           const unsigned* __restrict__ rec,
                                                           uint16_t* __restrict__ val,
-                                                          long long vstride) {
+                                                          long long vstride,
+                                                          int* __restrict__ out_of_range) {
   extern __shared__ unsigned brk_lds[];
   __shared__ int s_wave[BRK_BUILD / WAVE];
   int* before = reinterpret_cast<int*>(brk_lds + nwords);
@@ -819,11 +824,13 @@ __global__ __launch_bounds__(BRK_BUILD) void k_brk_values(int nwords, int vt, in
       const unsigned* hd = rec + brk_head_at(s0 + (q >> 1), q & 1);
       const long long at = e0 + hd[1] + 2 * ((r < 32 ? hd[2] : hd[3] & 0xFFFFu) + ((m >> 8) & 0xFFu)) +
                            __popc(m & 0xFFu & ((1u << (pos & 7)) - 1u));
+      float v = vt == EPET_VAL_F32    ? (float)mval[k]
+                : vt == EPET_VAL_BF16 ? brk_bf((unsigned)mval[k])
+                                      : __half2float(__ushort_as_half((uint16_t)mval[k]));
+      if (v != 0.0f && !(fabsf(v) >= BRK_VAL_MIN && fabsf(v) <= BRK_VAL_MAX)) *out_of_range = 1;
       if (vt == EPET_VAL_BF16) {
         val[at] = (uint16_t)mval[k];
       } else {
-        float v = vt == EPET_VAL_F32 ? (float)mval[k]
-                                     : __half2float(__ushort_as_half((uint16_t)mval[k]));
         for (int i = 0; i < parts; i++) {
           val[i * vstride + at] = (uint16_t)(__float_as_uint(v) >> 16);
           v -= brk_hi(v);
@@ -876,7 +883,7 @@ static std::vector<int> brk_voxel_positions(const MatGeo& g) {
 // ------------------------------------------------------------------ build (host)
 // Bricks of M with row positions `rows` and column positions `cols` (-1: none).
 // EPET_OK with *out == nullptr when memory is short, or (*unfit) the sizes are
-// beyond the kernel's, or the bricks too empty to pay.
+// beyond the kernel's, the values beyond the split's or the bricks too empty to pay.
 static int brk_build(epet_ctx* ctx, const epet_matrix* M, const std::vector<int>& rows,
                      const std::vector<int>& cols, BrkCopy** out, bool* unfit) {
   *out = nullptr;
@@ -967,18 +974,24 @@ static int brk_build(epet_ctx* ctx, const epet_matrix* M, const std::vector<int>
   alloc(&B->val, sizeof(uint16_t) * B->parts * vstride);
   if (!ok) return EPET_OK;
   brk_zero(st, B->val, sizeof(uint16_t) * B->parts * vstride);
+  brk_zero(st, ns, sizeof(int));
   if (M->value_type == EPET_VAL_F32)
     k_brk_values<float><<<B->G, BRK_BUILD, lds, st>>>(nwords, M->value_type, B->parts, B->rowperm,
                                                       M->rowptr, M->col, (const float*)M->val,
                                                       cpos_d, B->gstep, B->gent, B->rec,
-                                                      B->val, vstride);
+                                                      B->val, vstride, ns);
   else
     k_brk_values<uint16_t><<<B->G, BRK_BUILD, lds, st>>>(nwords, M->value_type, B->parts,
                                                          B->rowperm, M->rowptr, M->col,
                                                          (const uint16_t*)M->val, cpos_d, B->gstep,
-                                                         B->gent, B->rec, B->val, vstride);
+                                                         B->gent, B->rec, B->val, vstride, ns);
   EPET_HIP(hipGetLastError());
-  EPET_HIP(hipStreamSynchronize(st));
+  int out_of_range = 0;
+  EPET_TRY(read_pinned(ctx, &out_of_range, ns, sizeof(int)));
+  if (out_of_range) {
+    *unfit = true;
+    return EPET_OK;
+  }
   own.b = nullptr;
   *out = B;
   return EPET_OK;

@@ -1,5 +1,6 @@
 """Bricks over the whole range of FP32: gathered vectors with numbers down to the
-smallest, infinities and NaN, and vectors of small and huge numbers at once.
+smallest, infinities and NaN, vectors of small and huge numbers at once, and stored
+values that a split into bfloat16 parts cannot hold.
 
 Tolerance against FP64: a row has a few hundred entries, so its FP32 sums keep a
 relative error of some 1e-7 of the sum of magnitudes; bar 2e-6, where a vector of
@@ -7,6 +8,8 @@ numbers near 2^-120 that lost the bits below 2^-133 misses 1e-4.  Results below 
 normal numbers are multiples of 2^-149: 2^-148 beside that for each of up to 64
 partial sums (2^-142).  MLEM
 divides by such sums once per iteration: same bar for one iteration."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -107,3 +110,48 @@ def test_mlem_of_a_small_image(bricks, oracle, F):
     X = X.cpu().numpy()
     for f in range(F):
         assert np.linalg.norm(X[:, f] - X64[:, f]) <= 2e-6 * np.linalg.norm(X64[:, f]), f
+
+
+def _rewrite(ctx, A, change):
+    """The stored values changed through the library's own array, before any copy."""
+    from epetreco_amd._lib import check, lib
+    v = A.to_torch()[2].clone()
+    change(v)
+    check(lib().epet_memcpy_d2d(ctx.handle, ctypes.c_void_p(A.arrays()[2]),
+                                ctypes.c_void_p(v.data_ptr()), 4 * A.nnz))
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("what", ["inf", "nan", "small", "one small"])
+def test_stored_values_out_of_range(gpu_ctx_factory, monkeypatch, what):
+    """Values that are no sum of ordinary bfloat16 parts: products and MLEM come out as
+    without bricks."""
+    from epetreco_amd.api import OP_N, OP_T
+    from epetreco_amd.geometry import MeasurementSetup, VoxelGrid
+    s = MeasurementSetup(-0.23, 0.23, 3, 13, 13, 13, 13, 120.0, 0.02, 0.004, 0.004)
+    g = VoxelGrid(-0.025, -0.025, -0.025, 0.001, 0.001, 0.001, 50, 50, 50)
+    ctx = gpu_ctx_factory(setup=s, grid=g, nrays=64, seed=6)
+    A = ctx.sm_build((s.nchannels // 3 + np.arange(5000)).astype(np.int32))
+
+    def change(v):
+        if what == "small":
+            v *= 2.0 ** -113
+        else:
+            v[A.nnz // 2] = {"inf": float("inf"), "nan": float("nan"), "one small": 2.0 ** -120}[what]
+
+    _rewrite(ctx, A, change)
+    A.attach_transpose()
+    rows_only = env_ctx(monkeypatch, EPET_BATCHED="gather")
+    Z = torch.zeros(A.m, 64, device="cuda")
+    for _ in range(40):
+        product(ctx, A, OP_T, Z)     # products enough for bricks
+    K = _sparse(A)
+    for op, n in ((OP_N, A.n), (OP_T, A.m)):
+        X = torch.rand(n, 16, device="cuda") + 0.5
+        got, want = product(ctx, A, op, X), product(rows_only, A, op, X)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        if what.endswith("small"):
+            _agree(got, K if op == OP_N else K.T, X, (what, op))
+    x = torch.full((A.n, 3), 1.0 / A.n, device="cuda")
+    ctx.mlem(A, torch.ones(A.m, 3, device="cuda"), torch.ones(A.n, device="cuda"), x, 1)
+    assert not ctx.batched_config(A, 3)["path"].startswith("bricks")
