@@ -58,6 +58,7 @@ SIGNATURES = {
     "epet_matrix_info": (ctypes.c_int, [P, c_int_p, c_int_p, c_ll_p, c_int_p]),
     "epet_matrix_arrays": (ctypes.c_int, [P, ctypes.POINTER(P), ctypes.POINTER(P),
                                           ctypes.POINTER(P), ctypes.POINTER(P)]),
+    "epet_matrix_read": (ctypes.c_int, [P, P, P, P, P, P]),
     "epet_matrix_destroy": (ctypes.c_int, [P]),
     "epet_matrix_create": (ctypes.c_int, [P, ctypes.c_int, ctypes.c_int, ctypes.c_longlong, P, P,
                                           P, ctypes.POINTER(P)]),

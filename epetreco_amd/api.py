@@ -368,7 +368,8 @@ class Matrix:
         return cls(ctx, h)
 
     def arrays(self):
-        """(rowptr, col, val, rowscale) device pointers as ints."""
+        """(rowptr, col, val, rowscale) device pointers as ints.  Values may be written
+        through them: multi-frame products then use no copies of the matrix."""
         rp, c, v, s = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
         check(lib().epet_matrix_arrays(self._h, ctypes.byref(rp), ctypes.byref(c),
                                        ctypes.byref(v), ctypes.byref(s)))
@@ -376,21 +377,15 @@ class Matrix:
 
     def to_torch(self):
         """Copies (rowptr int64, col int32, val float32|int16 bits, rowscale|None)."""
-        rp, c, v, s = self.arrays()
         dev = self.ctx.device
         trp = torch.empty(self.m + 1, dtype=torch.int64, device=dev)
         tc = torch.empty(max(self.nnz, 1), dtype=torch.int32, device=dev)
         vdt = torch.float32 if self.value_type == VAL_F32 else torch.int16
         tv = torch.empty(max(self.nnz, 1), dtype=vdt, device=dev)
-        L, h = lib(), self.ctx.handle
-        check(L.epet_memcpy_d2d(h, _p(trp), ctypes.c_void_p(rp), 8 * (self.m + 1)))
-        if self.nnz:
-            check(L.epet_memcpy_d2d(h, _p(tc), ctypes.c_void_p(c), 4 * self.nnz))
-            check(L.epet_memcpy_d2d(h, _p(tv), ctypes.c_void_p(v), tv.element_size() * self.nnz))
-        ts = None
-        if s:
-            ts = torch.empty(max(self.m, 1), dtype=torch.float32, device=dev)
-            check(L.epet_memcpy_d2d(h, _p(ts), ctypes.c_void_p(s), 4 * self.m))
+        ts = (None if self.value_type == VAL_F32
+              else torch.empty(max(self.m, 1), dtype=torch.float32, device=dev))
+        check(lib().epet_matrix_read(self.ctx.handle, self._h, _p(trp), _p(tc), _p(tv),
+                                     _p(ts) if ts is not None else None))
         self.ctx.synchronize()
         return trp, tc[:self.nnz], tv[:self.nnz], ts
 

@@ -1240,7 +1240,8 @@ int brk_spmm(epet_ctx* ctx, const epet_matrix* cA, int op, int F, float alpha, c
              float beta, float* Y, bool* done) {
   *done = false;
   epet_matrix* A = const_cast<epet_matrix*>(cA);
-  if (!brk_wanted(A, F) || A->brk_state.load() < 0) return EPET_OK;
+  // (bricks of a matrix whose arrays a caller holds may be out of date)
+  if (!brk_wanted(A, F) || A->brk_state.load() < 0 || A->exposed.load()) return EPET_OK;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
     (void)hipGetLastError();

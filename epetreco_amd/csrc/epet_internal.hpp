@@ -232,6 +232,8 @@ struct epet_matrix {
   // (brk_state on the matrix itself: 0 not asked for yet, 1 built, -1 not to be)
   epet::BrkCopy* brk = nullptr;
   std::atomic<int> brk_state{0};
+  // whether a caller holds the arrays, and may write values at any time
+  std::atomic<bool> exposed{false};
   std::atomic<long long> brk_work{0};   // entries x frames multiplied before the bricks
   // multi-frame kernel configuration picked by the autotuner for mf_F frames
   // (rows per wavefront R, frames per lane tile P) and the times it measured

@@ -1010,6 +1010,23 @@ int epet_matrix_arrays(const epet_matrix* A, int64_t** rowptr, int** col, void**
   if (col) *col = A->col;
   if (val) *val = A->val;
   if (rowscale) *rowscale = A->rowscale;
+  const_cast<epet_matrix*>(A)->exposed.store(true);
+  return EPET_OK;
+}
+
+int epet_matrix_read(epet_ctx* ctx, const epet_matrix* A, int64_t* rowptr, int* col, void* val,
+                     float* rowscale) {
+  EPET_CHECK(ctx && A, EPET_ERR_ARG, "null argument");
+  hipStream_t st = ctx->stream;
+  const size_t vb = A->value_type == EPET_VAL_F32 ? 4 : 2;
+  if (rowptr)
+    EPET_HIP(hipMemcpyAsync(rowptr, A->rowptr, sizeof(int64_t) * ((size_t)A->m + 1),
+                            hipMemcpyDeviceToDevice, st));
+  if (col && A->nnz)
+    EPET_HIP(hipMemcpyAsync(col, A->col, sizeof(int) * A->nnz, hipMemcpyDeviceToDevice, st));
+  if (val && A->nnz) EPET_HIP(hipMemcpyAsync(val, A->val, vb * A->nnz, hipMemcpyDeviceToDevice, st));
+  if (rowscale && A->rowscale && A->m)
+    EPET_HIP(hipMemcpyAsync(rowscale, A->rowscale, sizeof(float) * A->m, hipMemcpyDeviceToDevice, st));
   return EPET_OK;
 }
 

@@ -173,9 +173,17 @@ int epet_sm_build(epet_ctx* ctx, const int* list_dev, int m, epet_matrix** out);
 
 int epet_matrix_info(const epet_matrix* A, int* m, int* n, long long* nnz,
                      int* value_type);
-/* Device arrays of a matrix (rowscale NULL for FP32 storage). */
+/* Device arrays of a matrix (rowscale NULL for FP32 storage).  A caller may write
+ * values through them: epet_matrix_spmm reads the arrays at every call from then on
+ * (no bricks).  Copies that other calls have made (the transposed copy, tile-major
+ * copies of epet_matrix_spmv and epet_mlem, the copies of multi-frame MLEM) keep the
+ * values they were made of.  To read a matrix use epet_matrix_read. */
 int epet_matrix_arrays(const epet_matrix* A, int64_t** rowptr, int** col,
                        void** val, float** rowscale);
+/* The matrix's arrays copied to device memory of the caller's: rowptr m + 1, col and val
+ * nnz, rowscale m elements (left alone for FP32 storage).  NULL: not wanted. */
+int epet_matrix_read(epet_ctx* ctx, const epet_matrix* A, int64_t* rowptr_dev,
+                     int* col_dev, void* val_dev, float* rowscale_dev);
 int epet_matrix_destroy(epet_matrix* A);
 /* Library matrix from caller arrays (copied): rowptr int64[m+1], col, FP32 val. */
 int epet_matrix_create(epet_ctx* ctx, int m, int n, long long nnz,

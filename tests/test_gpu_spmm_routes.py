@@ -119,3 +119,22 @@ def test_streams_and_a_graph(gpu_ctx_factory, monkeypatch):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, rows)
+
+
+def test_values_written_in_place(gpu_ctx_factory):
+    """Products after values were written through the matrix's own arrays are products of
+    those values, bricks built or not."""
+    from epetreco_amd._lib import check, lib
+    from epetreco_amd.api import OP_N, OP_T
+    ctx, A = scan(gpu_ctx_factory, 52, 52, 52, 64, 6001)
+    with_bricks(ctx, A)
+    X = {OP_N: torch.rand(A.n, 8, device="cuda"), OP_T: torch.rand(A.m, 8, device="cuda")}
+    before = {op: product(ctx, A, op, x) for op, x in X.items()}
+    val = A.arrays()[2]
+    for factor in (2.0, 0.5):       # exact in FP32
+        v = A.to_torch()[2] * factor
+        check(lib().epet_memcpy_d2d(ctx.handle, ctypes.c_void_p(val), ctypes.c_void_p(v.data_ptr()),
+                                    4 * A.nnz))
+        for op, x in X.items():
+            got, want = product(ctx, A, op, x), before[op] * (2.0 if factor == 2.0 else 1.0)
+            assert (got - want).abs().max() <= 2e-5 * want.abs().max()
