@@ -62,6 +62,7 @@
 
 #include "epet_block.hpp"
 #include "epet_internal.hpp"
+#include "epet_plan.hpp"
 #include "epet_rows.hpp"
 
 namespace epet {
@@ -1162,8 +1163,8 @@ static int brk_gather_x(epet_ctx* ctx, const BrkCopy* f, const BrkCopy* b, int F
 // Builds the bricks of A and of its transposed copy once (allocates and
 // synchronises: call outside graph capture), where the matrix knows its
 // channels and grid (what makes neighbours of rows and columns).  Nothing is
-// built when the bricks would be too empty or memory is short.  Two threads may
-// ask at once.
+// built when the bricks would be too empty or memory is short; short of memory it is
+// tried again once clearly more is available.  Two threads may ask at once.
 static std::mutex g_brk_build;
 static bool brk_wanted(const epet_matrix* A, int F) {
   return A->tr && F >= 2 && F <= 64 && A->cols_strict && A->m > 0 && A->n > 0 && A->row_ids &&
@@ -1173,6 +1174,12 @@ static int brk_build_both(epet_ctx* ctx, epet_matrix* A) {
   std::lock_guard<std::mutex> lock(g_brk_build);
   epet_matrix* At = A->tr;
   if (A->brk_state.load() != 0) return EPET_OK;
+  const unsigned long long available = dev_available();
+  if (!memory_worth_trying(available, A->brk_short.load())) return EPET_OK;
+  if (available < bricks_at_least(A->nnz, brk_parts(A->value_type))) {
+    A->brk_short.store(std::max(1ull, available));
+    return EPET_OK;
+  }
   bool unfit = false;
   int rc = EPET_OK;
   try {
@@ -1190,7 +1197,8 @@ static int brk_build_both(epet_ctx* ctx, epet_matrix* A) {
     brk_release(A);
     brk_release(At);
   }
-  A->brk_state.store(ok ? 1 : unfit ? -1 : 0);   // short of memory: asked again next time
+  A->brk_state.store(ok ? 1 : unfit ? -1 : 0);
+  if (!ok && !unfit) A->brk_short.store(std::max(1ull, available));
   return rc;
 }
 
@@ -1251,11 +1259,9 @@ int brk_spmm(epet_ctx* ctx, const epet_matrix* cA, int op, int F, float alpha, c
   if (A->brk_state.load() == 0) {
     const long long work = A->nnz * F;
     if (A->brk_work.fetch_add(work) + work < BRK_WORK * ((long long)A->m + A->n)) return EPET_OK;
-    size_t free_b = 0, total_b = 0;
-    EPET_HIP(hipMemGetInfo(&free_b, &total_b));
     // values with a quarter of padding, records, and as much again while building
     const double need = (double)A->nnz * 2.0 * (2.5 * brk_parts(A->value_type) + 4.0);
-    if (need > 0.25 * (double)free_b) return EPET_OK;
+    if (need > 0.25 * (double)dev_available()) return EPET_OK;
     EPET_TRY(brk_build_both(ctx, A));
     if (A->brk_state.load() != 1) return EPET_OK;
   }

@@ -169,6 +169,19 @@ hipError_t dev_free(void* p) {
   return e;
 }
 
+unsigned long long dev_available() {
+  int dev = 0;
+  size_t free_b = 0, total_b = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (dev < 0 || dev >= DEV_MAX) return free_b;
+  DevBlocks& d = dev_blocks()[dev];
+  std::lock_guard<std::mutex> lock(d.mu);
+  return free_b + d.kept_bytes;
+}
+
 // A caller may have given a block from epet_malloc to hipFree and have another one at
 // its address: forgets the block that was there unless this one is as large.
 static void dev_check(void* p) {

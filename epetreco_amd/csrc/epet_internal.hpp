@@ -35,6 +35,8 @@ int fail(int code, const char* file, int line, const std::string& msg);
 // the next ones (core.hip)
 hipError_t dev_malloc(void** p, size_t bytes);
 hipError_t dev_free(void* p);
+// bytes that dev_malloc could still get: free ones and those kept (0: unknown)
+unsigned long long dev_available();
 // hipMallocAsync from the library's pool (freed with hipFreeAsync)
 hipError_t tmp_malloc(void** p, size_t bytes, hipStream_t st);
 
@@ -232,6 +234,7 @@ struct epet_matrix {
   // (brk_state on the matrix itself: 0 not asked for yet, 1 built, -1 not to be)
   epet::BrkCopy* brk = nullptr;
   std::atomic<int> brk_state{0};
+  std::atomic<unsigned long long> brk_short{0};   // bytes available when bricks did not fit
   // whether a caller holds the arrays, and may write values at any time
   std::atomic<bool> exposed{false};
   std::atomic<long long> brk_work{0};   // entries x frames multiplied before the bricks
