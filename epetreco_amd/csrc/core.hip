@@ -62,8 +62,9 @@ int ctx_scratch(epet_ctx* ctx, size_t bytes, void** out) {
 // once the device has finished all work (which hipFree waits for as well), so
 // any thread or stream may take it.
 constexpr size_t DEV_KEEP = (size_t)16 << 30;
-// Stream-ordered temporaries: the pairs of a transposed copy take up to 1 GB beside
-// others (reconstructions of 88M entries in turn: 14.5 ms with 1 GB, 12.6 with 2).
+// Stream-ordered temporaries: cooSort takes 20 bytes a pair and some (60M pairs out of
+// order, 1.3 GB: 6.75 ms with 1 GB kept, 6.05 with 2; up to 40M pairs, and
+// reconstructions of 88M entries, whose largest temporary is 144 MB, the same).
 constexpr size_t TMP_KEEP = (size_t)2 << 30;
 constexpr int DEV_MAX = 64;
 
