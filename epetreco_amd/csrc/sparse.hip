@@ -660,7 +660,7 @@ __device__ __forceinline__ long long tr_bucket_start(long long n, long long blk,
   return p;
 }
 
-template <typename V, typename P>
+template <typename V>
 __global__ __launch_bounds__(TRP_BLOCK) void k_tr_bucket(int m, int n, int T, int tile,
                                                          int rows_per_block,
                                                          const int64_t* __restrict__ rowptr,
@@ -669,8 +669,7 @@ __global__ __launch_bounds__(TRP_BLOCK) void k_tr_bucket(int m, int n, int T, in
                                                          const uint32_t* __restrict__ cnt,
                                                          const int64_t* __restrict__ tptr,
                                                          TrPair<V>* __restrict__ out) {
-  extern __shared__ unsigned char tr_raw[];
-  P* cur = reinterpret_cast<P*>(tr_raw);       // next position of the tile's buckets
+  extern __shared__ unsigned tr_cur[];          // next position of the tile's buckets
   __shared__ int64_t s_lo[TRP_BLOCK];
   __shared__ int s_n[TRP_BLOCK];
   const int t = blockIdx.x % T;
@@ -678,7 +677,7 @@ __global__ __launch_bounds__(TRP_BLOCK) void k_tr_bucket(int m, int n, int T, in
   const int c0 = t * tile, c1 = min(n, c0 + tile);   // tile: whole buckets
   const int b0 = c0 / TR_BUCKET, nb = (c1 - c0 + TR_BUCKET - 1) / TR_BUCKET;
   for (int i = threadIdx.x; i < nb; i += TRP_BLOCK)
-    cur[i] = (P)tr_bucket_start(n, blk, b0 + i, cnt, tptr);
+    tr_cur[i] = (unsigned)tr_bucket_start(n, blk, b0 + i, cnt, tptr);
   const int lane = lane_id();
   const long long r0 = blk * rows_per_block, r1 = min((long long)m, r0 + rows_per_block);
   // one entry per thread: runs of one bucket take their places together
@@ -692,10 +691,10 @@ __global__ __launch_bounds__(TRP_BLOCK) void k_tr_bucket(int m, int n, int T, in
     const unsigned long long below = heads & (~0ull >> (63 - lane));
     const int h = 63 - __clzll((long long)(below | 1ull));
     const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1);
-    P base = 0;
+    unsigned base = 0;
     if (head) {
       const int next = above ? lane + __ffsll((long long)above) : __popcll(live);
-      base = (P)atomicAdd(&cur[b], (P)(next - lane));
+      base = atomicAdd(&tr_cur[b], (unsigned)(next - lane));
     }
     base = __shfl(base, h, WAVE);
     if (in) out[(long long)base + (lane - h)] = TrPair<V>{(unsigned)r * TR_BUCKET + (c & (TR_BUCKET - 1)), v};
@@ -817,13 +816,13 @@ __global__ __launch_bounds__(TR_WAVES * WAVE) void k_tr_place(int n, int B,
 // Places the entries by buckets; *done = false where that does not apply: rows too
 // short to occupy a workgroup (57 entries: no gain), keys beyond 32 bits, counters
 // beyond LDS, pairs of more than TR_PAIR_BYTES, or no memory for them.
-template <typename V, typename P>
+template <typename V>
 static int tr_by_buckets(epet_ctx* ctx, const epet_matrix* A, int rpb, int B, const uint32_t* cnt,
                          const int64_t* tptr, int* orow, void* oval, bool* done) {
   *done = false;
   const int nbuckets = (int)(((long long)A->n + TR_BUCKET - 1) / TR_BUCKET);
   if (A->nnz < 128ll * A->m || A->m >= (1 << (32 - TR_BITS))) return EPET_OK;
-  const int per_wg = 48 * 1024 / (int)sizeof(P);
+  const int per_wg = 48 * 1024 / (int)sizeof(unsigned);
   // two workgroups per CU (one to eight made no difference)
   const int fit = (nbuckets + per_wg - 1) / per_wg;
   int T = std::max(fit, std::min(16, std::max(1, 512 / B)));
@@ -831,8 +830,8 @@ static int tr_by_buckets(epet_ctx* ctx, const epet_matrix* A, int rpb, int B, co
   const int tile = (nbuckets + T - 1) / T * TR_BUCKET;
   T = (A->n + tile - 1) / tile;
   hipStream_t st = ctx->stream;
-  // A block that is kept for the next matrix once freed: 0.7 GB from the pool of
-  // temporaries, which keeps less, took 35 ms longer a reconstruction.
+  // A block that is kept for the next matrix once freed (0.7 GB from the pool of
+  // temporaries, beyond what that kept, took 35 ms longer a reconstruction).
   const size_t bytes = sizeof(TrPair<V>) * (size_t)A->nnz;
   if (bytes > TR_PAIR_BYTES) return EPET_OK;
   struct Block {
@@ -844,7 +843,7 @@ static int tr_by_buckets(epet_ctx* ctx, const epet_matrix* A, int rpb, int B, co
     return EPET_OK;
   }
   TrPair<V>* pairs = (TrPair<V>*)block.p;
-  k_tr_bucket<V, P><<<(unsigned)(B * T), TRP_BLOCK, sizeof(P) * (size_t)(tile / TR_BUCKET), st>>>(
+  k_tr_bucket<V><<<(unsigned)(B * T), TRP_BLOCK, sizeof(unsigned) * (size_t)(tile / TR_BUCKET), st>>>(
       A->m, A->n, T, tile, rpb, A->rowptr, A->col, (const V*)A->val, cnt, tptr, pairs);
   k_tr_place<V><<<(unsigned)nbuckets, TR_WAVES * WAVE, 0, st>>>(A->n, B, cnt, tptr, pairs, orow,
                                                                 (V*)oval);
@@ -1229,18 +1228,11 @@ int epet_matrix_transpose(epet_ctx* ctx, epet_matrix* A) {
   if (any) {
     const int g = B * nt;
     bool done = false;
-    if (A->value_type == EPET_VAL_F32 && wide)
-      EPET_TRY((tr_by_buckets<float, unsigned long long>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
-                                                   &done)));
-    else if (A->value_type == EPET_VAL_F32)
-      EPET_TRY((tr_by_buckets<float, unsigned>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
-                                         &done)));
-    else if (wide)
-      EPET_TRY((tr_by_buckets<uint16_t, unsigned long long>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
-                                                      &done)));
+    // (pairs of at most TR_PAIR_BYTES: positions of 32 bits)
+    if (A->value_type == EPET_VAL_F32)
+      EPET_TRY((tr_by_buckets<float>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val, &done)));
     else
-      EPET_TRY((tr_by_buckets<uint16_t, unsigned>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val,
-                                            &done)));
+      EPET_TRY((tr_by_buckets<uint16_t>(ctx, A, rpb, B, cnt, T->rowptr, T->col, T->val, &done)));
     if (!done && A->value_type == EPET_VAL_F32) {
       if (wide)
         launch_tr_fill<float, uint64_t>(st, g, A->m, A->n, nt, tile, rpb, A->rowptr, A->col, A->val,
