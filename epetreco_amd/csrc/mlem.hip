@@ -132,16 +132,6 @@ __global__ void k_zero_f64(double* p, int n) {
 }
 
 // ------------------------------------------------------------------ fused MLEM
-struct MlemState {
-  int it;          // iterations completed
-  int F;
-  double* sum;     // [2][F]
-  double* loglik;  // [niter][F]
-  int* active;     // [F]
-  int niter;
-};
-
-
 // Single frame, short rows: L lanes per row, grid-stride over rows; one FP64
 // log-likelihood atomic per workgroup.  fold = 1 multiplies the ratio by the row
 // scale, for a back projection through the transposed copy (which stores the
@@ -623,7 +613,7 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
   // 2766 against 2381; 150,000 rows, 52^3, 13 frames, 3: 1955 against 1859).
   (void)use_graph;
   hipStream_t st = ctx->stream;
-  // one block: e (m F), c (n F), s (n), doubles [ssum, sum[2F], loglik[niter F]],
+  // one block: e (m F), c (n F), s (n), doubles [sum of s, sum[2F], loglik[niter F]],
   // ints [it, it of the update, active[F]]
   const size_t nd = 1 + 2 * (size_t)F + (size_t)std::max(1, niter) * F;
   const size_t e_b = align256(sizeof(float) * (size_t)A->m * F);
@@ -651,7 +641,6 @@ int epet_mlem(epet_ctx* ctx, const epet_matrix* A, int F, const float* y, const 
   double* dbuf = (double*)(block + e_b + c_b + s_b);
   int* itp = (int*)(block + e_b + c_b + s_b + d_b);
   int* active = itp + 2;
-  double* ssum = dbuf;
   double* sum = dbuf + 1;
   double* ll = dbuf + 1 + 2 * F;
   EPET_MLEM_HIP(mlem_start(ctx, A->n, F, s_in, dbuf, (long long)nd, itp, c, s));
@@ -749,7 +738,6 @@ int epet_mlem_noalloc(epet_ctx* ctx, const epet_matrix* A, const float* y, const
   EPET_TRY(scratch_address(ctx->device, &base));
   hipStream_t st = ctx->stream;
   double* dbuf = (double*)(base + L.d);
-  double* ssum = dbuf;
   double* sum = dbuf + 1;
   double* ll = dbuf + 3;
   int* itp = (int*)(base + L.it);
