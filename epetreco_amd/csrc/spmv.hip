@@ -179,13 +179,24 @@ __global__ __launch_bounds__(256) void k_spmv_n_vec(int m, const int64_t* __rest
 }
 
 // ------------------------------------------------------------------ tiled back projection
-// The image is cut into tiles of BP_TILE consecutive voxel ids (128 KB of LDS).
-// Workgroup (row block, tile) accumulates a_ij e_i of its rows' entries inside
-// the tile with LDS double atomics and writes the tile into its row block's
-// partial image; a reduction sums the partial images.  Entry ranges of every
+// The image is cut into tiles of BP_TILE consecutive voxel ids (64 KB of LDS, two
+// workgroups a CU).  Workgroup (row block, tile) accumulates a_ij e_i of its rows'
+// entries inside the tile with LDS double atomics and writes the tile into its row
+// block's partial image; a reduction sums the partial images.  Entry ranges of every
 // (row, tile) come from a per-matrix plan of tile-boundary offsets.
-constexpr int BP_TILE = 16384;
+//
+// The sums are FP64, as a block's come in any order and have to round to the same
+// floats.  SUB lanes take a row's entries in a tile, U a lane at once: 32 and 4, or 16
+// and 2 where rows have fewer than BP_SHORT entries in a tile.  Product with its
+// reduction (rows, entries a row, voxels), floats in tiles of 16,384 by 32 lanes as
+// first written / doubles in the same tiles / these: 1,000 of 900, 52^3 69 / 18 / 16
+// us; 20,000 of 927, 52^3 159 / 120 / 97; 11,250 of 388, 52^3 86 / 71 / 53; 3,000 of
+// 2,947, 104^3 123 / 135 / 98; 11,250 of 999, 104^3 184 / 250 / 151.  Of the last three
+// (7 to 22 entries in a tile) 32 lanes take 63, 112 and 244; of the first two (50) 16
+// lanes 18 and 102.
+constexpr int BP_TILE = 8192;
 constexpr int BP_BLOCK = 1024;
+constexpr int BP_SHORT = 32;
 
 __global__ __launch_bounds__(256) void k_bp_plan(int m, int T, int TS,
                                                  const int64_t* __restrict__ rowptr,
@@ -207,8 +218,8 @@ __global__ __launch_bounds__(256) void k_bp_plan(int m, int T, int TS,
   toff[idx] = (uint32_t)(lo - b);
 }
 
-template <typename VT>
-__global__ __launch_bounds__(BP_BLOCK) void k_bp_tiled(int m, int n, int T, int rows_per_block,
+template <typename VT, int SUB, int U>
+__global__ __launch_bounds__(BP_BLOCK) void k_bp_tiled(int m, int n, int T, int nblk, int rows_per_block,
                                                        const int64_t* __restrict__ rowptr,
                                                        const int* __restrict__ col,
                                                        const typename VT::T* __restrict__ val,
@@ -216,20 +227,17 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_tiled(int m, int n, int T, int 
                                                        const uint32_t* __restrict__ toff,
                                                        const float* __restrict__ e, float alpha,
                                                        float* __restrict__ partial) {
-  // FP64: a block's sums come in any order, and have to round to the same floats
-  // (11,250 rows of 405 entries, 52^3: 58 us, with floats 51)
   __shared__ double acc[BP_TILE];
-  const int t = blockIdx.y;
-  const long long r0 = (long long)blockIdx.x * rows_per_block;
+  const int t = blockIdx.x / nblk, blk = blockIdx.x % nblk;
+  const long long r0 = (long long)blk * rows_per_block;
   const long long r1 = min((long long)m, r0 + rows_per_block);
   const int tile0 = t * BP_TILE;
   const int tn = min(BP_TILE, n - tile0);
   for (int j = threadIdx.x; j < BP_TILE; j += BP_BLOCK) acc[j] = 0.0;
   __syncthreads();
-  const int sub = threadIdx.x & 31;          // 32 lanes per row segment
-  const int seg = threadIdx.x >> 5;          // 32 segments per workgroup
-  // a row's weight and ends are requested while the row before it is worked, and four
-  // entries a lane at once (11,250 rows of 405 entries, 52^3: 57 -> 51 us)
+  const int sub = threadIdx.x % SUB;
+  const int seg = threadIdx.x / SUB;
+  // a row's weight and ends are requested while the row before it is worked
   auto row = [&](long long r, float& ev, long long& lo, long long& hi) {
     ev = 0.0f;
     if (r >= r1) return;
@@ -241,31 +249,31 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_tiled(int m, int n, int T, int 
   float en = 0.0f;
   long long ln = 0, hn = 0;
   row(r0 + seg, en, ln, hn);
-  for (long long r = r0 + seg; r < r1; r += BP_BLOCK / 32) {
+  for (long long r = r0 + seg; r < r1; r += BP_BLOCK / SUB) {
     float ev = en;
     const long long lo = ln, hi = hn;
     const float sc = rowscale ? rowscale[r] : 1.0f;
-    row(r + BP_BLOCK / 32, en, ln, hn);
+    row(r + BP_BLOCK / SUB, en, ln, hn);
     if (ev == 0.0f) continue;
     ev *= alpha * sc;
-    for (long long k = lo + sub; k < hi; k += 128) {
-      unsigned j[4];
-      float v[4];
+    for (long long k = lo + sub; k < hi; k += U * SUB) {
+      unsigned j[U];
+      float v[U];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const long long ki = k + 32 * i < hi ? k + 32 * i : k;
+      for (int i = 0; i < U; i++) {
+        const long long ki = k + SUB * i < hi ? k + SUB * i : k;
         j[i] = (unsigned)(ldcol(col, ki) - tile0);
         v[i] = VT::get(val, ki);
       }
       // the plan puts every column of [lo, hi) inside the tile; the unsigned
       // compare keeps LDS indices in range even for an inconsistent plan
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-        if (k + 32 * i < hi && j[i] < BP_TILE) unsafeAtomicAdd(&acc[j[i]], (double)(v[i] * ev));
+      for (int i = 0; i < U; i++)
+        if (k + SUB * i < hi && j[i] < BP_TILE) unsafeAtomicAdd(&acc[j[i]], (double)(v[i] * ev));
     }
   }
   __syncthreads();
-  float* out = partial + (size_t)blockIdx.x * n + tile0;
+  float* out = partial + (size_t)blk * n + tile0;
   for (int j = threadIdx.x; j < tn; j += BP_BLOCK) out[j] = (float)acc[j];
 }
 
@@ -338,10 +346,11 @@ static int launch_bp_tiled(hipStream_t st, const epet_matrix* A, const float* x,
                            float beta, float* y) {
   using T = typename VT::T;
   const int rows_per_block = (A->m + A->bp_nblk - 1) / A->bp_nblk;
-  dim3 grid(A->bp_nblk, A->bp_T);
-  k_bp_tiled<VT><<<grid, BP_BLOCK, 0, st>>>(A->m, A->n, A->bp_T, rows_per_block, A->rowptr, A->col,
-                                            (const T*)A->val, A->rowscale, A->bp_toff, x, alpha,
-                                            A->bp_partial);
+  const auto kern = A->nnz < (long long)BP_SHORT * A->m * A->bp_T ? k_bp_tiled<VT, 16, 2>
+                                                                   : k_bp_tiled<VT, 32, 4>;
+  kern<<<(unsigned)(A->bp_nblk * A->bp_T), BP_BLOCK, 0, st>>>(
+      A->m, A->n, A->bp_T, A->bp_nblk, rows_per_block, A->rowptr, A->col, (const T*)A->val,
+      A->rowscale, A->bp_toff, x, alpha, A->bp_partial);
   k_bp_reduce<<<grid_for(A->n, WAVE, 1ll << 31), BPR_WAVES * WAVE, 0, st>>>(
       A->n, A->bp_nblk, A->bp_partial, beta, y);
   EPET_HIP(hipGetLastError());
