@@ -606,8 +606,14 @@ __global__ __launch_bounds__(256) void k_blk_gather(float* __restrict__ Gp,
 // W = 1: a thread adds an element's partial sums in split order.  A few rows over
 // many column tiles have hundreds of splits and few elements, which that left to
 // wait for one load after the other (120 rows over 641,424 voxels, 14 frames, 627
-// splits: 153 us); W wavefronts then share 64 elements (8 us).
+// splits: 153 us); W wavefronts then share 64 elements (8 us).  Where elements fill the
+// SIMDs (BLK_WIDE_ITEMS: a wavefront each) a thread an element is the faster one.  MLEM
+// iterations W = 16 / W = 1 in us: 500 rows of 4 frames, 311 splits 148 / 168; 1,000 of
+// 14, 138 splits 103 / 109; 4,000 of 14, 512 splits 380 / 408; 3,000 of 14, 138 splits
+// 126 / 126; 12,000 of 14, 138 splits 294 / 275; 20,000 of 14, 103 splits 794 / 762;
+// and with few splits 40,000 of 4, 26 splits 500 / 465.
 constexpr int BLK_WIDE = 16, BLK_WIDE_SPLITS = 32;
+constexpr long long BLK_WIDE_ITEMS = 65536;
 template <int W>
 __global__ __launch_bounds__(W == 1 ? 256 : W * WAVE) void k_blk_reduce(BlkArgs a) {
   constexpr int ITEMS = W == 1 ? 256 : WAVE;
@@ -1122,7 +1128,7 @@ static int blk_launch(epet_ctx* ctx, const BlkCopy* B, int P, int rb, int splits
   if (splits > 1) {
     a.mode = mode;
     const long long items = (long long)B->m_pad * F;
-    if (splits > BLK_WIDE_SPLITS)
+    if (splits > BLK_WIDE_SPLITS && items <= BLK_WIDE_ITEMS)
       k_blk_reduce<BLK_WIDE><<<grid_for(items, WAVE, 16ll * ctx->num_cus), BLK_WIDE * WAVE, 0,
                                ctx->stream>>>(a);
     else
