@@ -76,8 +76,12 @@ constexpr int BRK_TAIL = 1024;     // readable entries past the last one (a step
 constexpr int BRK_LL = 64;         // copies of the log-likelihood sums
 // A step costs about the same however few entries it holds: 170 to 250 cycles of
 // a CU measured (8 frames of FP16 values; 16 and 32), where k_blk took 2.3 to 2.9
-// an entry.  At 92 to 110 entries a step bricks still won (16^3, 8 rays, 5 frames:
-// 17 and 23 us against 27 and 32); below 80 k_blk is kept.
+// an entry.  MLEM iterations on bricks / k_blk / gather kernels in us, by the entries a
+// step of both directions, FP32 values: 106 and 100, 4 frames 167 / 303 / 383; 85 and
+// 130, 66 / 136 / 90; 67 and 84, 78 / 147 / 104; 50 and 65, 629 / 842 / 1434; 42 and 65,
+// 69 / 104 / 81; 30 and 89, 401 / 346 / 714 (16 frames 408 / 510 / 607); 15 and 61,
+// 1751 / 1499 / 2393 (32 frames 2500 / 5513 / 2349); BF16 values have won at all of
+// them.  The line could lie at 40 to 50; it is where it was first drawn.
 constexpr int BRK_MIN_ENTRIES = 80;
 
 // scaled sums stay below 2^96 times a row's sum of magnitudes
@@ -1219,7 +1223,8 @@ int brk_prepare(epet_ctx* ctx, epet_matrix* A, int F) {
 // else an entry and frame take 2 to 3 ps, 0.7 to 0.8 where the gathered vector stays
 // near.  Rows / bricks in us, FP32: 9,001 rows, 0.49M entries, 16^3 voxels, 8 frames
 // 6 / 34; 0.90M, 64 frames 46 / 39; 700 rows, 0.60M, 52^3, 4 frames 17 / 33, 16 frames
-// 83 / 33; 4.4M, 2 frames 32 / 51, 4 frames 55 / 51; 48.8M, 2 frames 197 / 156.
+// 83 / 33; 4.4M, 2 frames 32 / 51, 4 frames 55 / 51; 18.5M, 2 frames 87 / 97, 3 frames
+// 156 / 94; 48.8M, 2 frames 197 / 156.
 // The back projection by the rows adds with float atomics, several times further from
 // the exact sums (4e-7 against 1.1e-7, 50,000 rows of 899 entries), and stays on bricks.
 static bool brk_rows_faster(const epet_matrix* A, int F) {
@@ -1227,7 +1232,7 @@ static bool brk_rows_faster(const epet_matrix* A, int F) {
   int P = 2;
   while (P < F) P *= 2;
   const double serial = 0.4 / WAVE * P * (double)A->nnz / A->m;
-  const double rows = 5.0 + std::max(serial, e * F * (A->n < 32768 ? 0.8 : 3.0));
+  const double rows = 5.0 + std::max(serial, e * F * (A->n < 32768 ? 0.8 : 2.5));
   return rows < 35.0 + e * (1.5 + 0.7 * brk_parts(A->value_type));
 }
 
