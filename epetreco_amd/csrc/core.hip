@@ -203,8 +203,9 @@ static void dev_check(void* p) {
 // between calls (the device's default pool gives them back at every
 // synchronisation)
 hipError_t tmp_malloc(void** p, size_t bytes, hipStream_t st) {
-  int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < DEV_MAX) {
+  // of the stream's device, as hipMallocAsync takes them, whichever device is current
+  hipDevice_t dev = 0;
+  if (hipStreamGetDevice(st, &dev) == hipSuccess && dev >= 0 && dev < DEV_MAX) {
     DevBlocks& d = dev_blocks()[dev];
     hipMemPool_t pool;
     {
