@@ -1336,14 +1336,17 @@ int brk_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& m) {
 
 // Splits of a group's steps, per direction: enough wavefronts to fill the chip
 // against partial sums to add, by time.  Tried are splits of two batches of steps
-// and more, up to BRK_TRY_WAVES wavefronts, 16 rounds of 16 per CU: the fastest had
-// 2,256 (9,001 rows, 16^3 voxels) to 35,152 (99,000 rows back, 104^3), and each takes
-// as many partial sums: 64 frames of 3.3M rows in 64 parts, the limit by steps alone,
-// would take 55 GB to find that one part is best.
-constexpr long long BRK_TRY_WAVES = 65536;
-static int brk_most_splits(const BrkCopy* B) {
+// and more whose partial sums take up to BRK_TRY_BYTES: 64 frames of 3.3M rows in 64
+// parts, the limit by steps alone, would take 55 GB to find that one part is best.
+// (A limit at 65,536 wavefronts instead left the back projection of 3.3M rows 16 parts
+// for 32 to 64, and so longer FP32 sums: 2.4e-6 from 64 bits after 20 iterations of 32
+// frames against 1.0e-6 to 1.5e-6.)
+constexpr long long BRK_TRY_BYTES = 4ll << 30;
+static int brk_most_splits(const BrkCopy* B, int Fp) {
   int most = 1;
-  while (most < 64 && B->nsteps >= 8ll * B->G * most && 2ll * B->G * most <= BRK_TRY_WAVES) most *= 2;
+  while (most < 64 && B->nsteps >= 8ll * B->G * most &&
+         (long long)sizeof(float) * brk_partials(B, 2 * most, Fp) <= BRK_TRY_BYTES)
+    most *= 2;
   return most;
 }
 int brk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& m, int reps) {
@@ -1358,7 +1361,7 @@ int brk_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& m, int reps) {
   for (int d = 0; d < 2 && rc == EPET_OK; d++) {
     BrkCopy* B = dirs[d];
     float best = 1e30f;
-    int most = brk_most_splits(B);
+    int most = brk_most_splits(B, Fp);
     while (most > 1 && !brk_partial_ensure(B, brk_partials(B, most, Fp))) most /= 2;
     for (int splits = 1; splits <= most && rc == EPET_OK; splits *= 2) {
       auto run = [&]() {
