@@ -1164,7 +1164,7 @@ static BlkCopy* blk_find(const epet_matrix* M, int Fp) {
 
 // Builds the blocked copies of A (forward) and of its transposed copy (back
 // projection) for F frames, once per padded frame count (allocates and
-// synchronises: call outside graph capture).  Without memory nothing is built
+// synchronises).  Without memory nothing is built
 // and the gather kernels run instead.
 int blk_prepare(epet_ctx* ctx, epet_matrix* A, int F) {
   epet_matrix* At = A->tr;
@@ -1213,7 +1213,7 @@ bool blk_ready(const epet_matrix* A, int F) {
 }
 
 // Forward + back projection of one multi-frame MLEM iteration with the tuned
-// shapes (capturable once prepared and tuned).
+// shapes (allocates nothing once prepared and tuned).
 int blk_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& a) {
   const int Fp = padded_frames(a.F);
   const BlkCopy* f = blk_find(A, Fp);

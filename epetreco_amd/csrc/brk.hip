@@ -1165,7 +1165,7 @@ static int brk_gather_x(epet_ctx* ctx, const BrkCopy* f, const BrkCopy* b, int F
 }
 
 // Builds the bricks of A and of its transposed copy once (allocates and
-// synchronises: call outside graph capture), where the matrix knows its
+// synchronises), where the matrix knows its
 // channels and grid (what makes neighbours of rows and columns).  Nothing is
 // built when the bricks would be too empty or memory is short; short of memory it is
 // tried again once clearly more is available.  Two threads may ask at once.
@@ -1324,7 +1324,7 @@ bool brk_ready(const epet_matrix* A, int F) {
   return true;
 }
 
-// One multi-frame iteration's products (capturable once prepared and tuned).
+// One multi-frame iteration's products (allocates nothing once prepared and tuned).
 int brk_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& m) {
   const int Fp = brk_pad(m.F), s = brk_slot(Fp);
   const BrkCopy *f = A->brk, *b = A->tr->brk;

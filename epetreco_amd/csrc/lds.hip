@@ -638,7 +638,7 @@ static ColMap voxel_map(const epet_ctx* ctx, const epet_matrix* A) {
 }
 
 // Builds the tile-major copy and the partial buffer once (allocates and
-// synchronises: call outside graph capture).  voxel_columns: the columns are
+// synchronises).  voxel_columns: the columns are
 // image voxels (a forward projector), so they may be renumbered.  Leaves the
 // matrix without them when an allocation fails; the other products then run.
 int lds_prepare_map(epet_ctx* ctx, epet_matrix* A, bool voxel_columns) {
@@ -697,7 +697,7 @@ int lds_spmv(epet_ctx* ctx, const epet_matrix* A, const float* x, float alpha, f
   return EPET_OK;
 }
 
-// MLEM forward step (capturable once prepared)
+// MLEM forward step (allocates nothing once prepared)
 int lds_fwd_ratio(epet_ctx* ctx, const epet_matrix* A, const float* x, const float* y, float* e,
                   int fold, const int* itp, double* loglik) {
   rows_lds<0>(ctx, A, x, A->lds_partial, LdsStore{});

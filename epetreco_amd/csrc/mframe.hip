@@ -294,7 +294,7 @@ int mf_tune(epet_ctx* ctx, epet_matrix* A, const MfArgs& a, int reps) {
   return EPET_OK;
 }
 
-// Forward + back projection of one multi-frame MLEM iteration (capturable).
+// Forward + back projection of one multi-frame MLEM iteration (allocates nothing).
 int mf_iteration(epet_ctx* ctx, const epet_matrix* A, const MfArgs& a) {
   int Rf = A->mf_fwd_R, Pf = A->mf_fwd_P, Rb = A->mf_bwd_R, Pb = A->mf_bwd_P;
   if (A->mf_F != a.F) { mf_default(a.F, Rf, Pf); Rb = Rf; Pb = Pf; }

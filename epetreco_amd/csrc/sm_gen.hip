@@ -376,9 +376,9 @@ __global__ __launch_bounds__(GEN_BLOCK) void k_sm_rows(Geo g, const int* __restr
 // Bound by VALU work (68% busy) and, at 10 workgroups per CU by their LDS, the chain
 // of LDS reads of one ray after the other.  Channels of 916 entries (52^3, 64 rays):
 // 40,000 took 7.86 ms in k_sm_rows, 100,000 18.6; walked with divisions and every
-// voxel of the rectangles tried 2.11 and 5.1 ms; now 1.49 and 4.0 ms (divisions 0.3,
-// steps 0.15, windows from sums 0.15 of the 0.62 ms).  11,250 of 57 entries (16^3, 8
-// rays): 275, 59, 48 us.
+// voxel of the rectangles tried 2.11 and 5.1 ms; now 1.20 and 3.5 ms (of 40,000: divisions
+// 0.3, steps 0.15, windows from sums 0.15, the candidate stage 0.1 ms and more).  11,250
+// of 57 entries (16^3, 8 rays): 275, 59, 44 us.
 //
 // A ray parallel to an axis meets every voxel of that axis (the reference
 // ignores the axis then), so its windows span it.  Rows it does not take are
@@ -409,7 +409,7 @@ __device__ __forceinline__ bool walk_plain(float v, bool zero_too) {
 
 // Integer divisions of v and roots and quotients per voxel were most of the candidate
 // stage (2,001 rows with all 40M candidates: 481 us, with walk_div and CandidateTest
-// 307; 40,000 rows of 916 entries: 1,280 and 1,186).
+// 307; 40,000 rows of 916 entries: 1,280 and 1,190).
 // n / d for 0 <= n < 2^24, d >= 1 and quotients below 2^20, r about 1 / d: the
 // rounded quotient is off by one at most
 __device__ __forceinline__ int walk_div(int n, int d, float r) {
